@@ -137,7 +137,7 @@ namespace lbx
         // density fitting (ri.hip): the fitted 3-index tensor W (nbf^2 naux doubles, P-major),
         // built on the first lbx_ri_jk call and kept, and the exchange work buffer (same size,
         // made on the first call with K); both in allocations
-        double *ri_w = nullptr, *ri_t = nullptr;
+        double *ri_w = nullptr, *ri_t = nullptr, *ri_h = nullptr;   // ri_h: naux doubles
         bool ri_ready = false;
         std::mutex ri_mu;
 

@@ -6,13 +6,16 @@
 //   K = sum_P W_P D W_P
 // W depends on the geometry only: the first call builds it (eri3, a transpose to P-major, eri2,
 // the Cholesky factorisation, one triangular solve) and the context keeps it, so every later
-// call (an SCF iteration) costs two matrix-vector products for J and, for K, one batched GEMM
-// W_P D and one GEMM over k = nbf * naux.  Factorisation by rocSOLVER, products by rocBLAS.
+// call (an SCF iteration) costs one or two passes over W for J and, for K, the products
+// T_P = W_P D and K = sum_P T_P W_P^T (k = nbf * naux), on FP64 MFMA kernels of this file.
+// Factorisation by rocSOLVER, the triangular solve by rocBLAS.
 #include <rocblas/rocblas.h>
 #include <rocsolver/rocsolver.h>
 
+#include "device_common.hpp"
 #include "lbx_internal.hpp"
 
+#include <algorithm>
 #include <memory>
 #include <string>
 
@@ -45,6 +48,191 @@ namespace lbx
                 }
                 __syncthreads();
             }
+        }
+
+        // sum over the workgroup's 256 threads, valid in thread 0
+        __device__ __forceinline__ double blockSum256(double x)
+        {
+            __shared__ double part[4];
+            x = waveSum(x);
+            if ((threadIdx.x & 63) == 0)
+                part[threadIdx.x >> 6] = x;
+            __syncthreads();
+            return part[0] + part[1] + part[2] + part[3];
+        }
+
+        // h_P = sum_mn W_P(mn) D_mn, one workgroup per P
+        __global__ __launch_bounds__(256) void fitDotKernel(const double *__restrict__ W, const double *__restrict__ D,
+                                                            double *__restrict__ h, long long n2)
+        {
+            const double *w = W + blockIdx.x * n2;
+            double s = 0.0;
+            for (long long i = threadIdx.x; i < n2; i += 256)
+                s = fma(w[i], D[i], s);
+            s = blockSum256(s);
+            if (threadIdx.x == 0)
+                h[blockIdx.x] = s;
+        }
+
+        // h_P = tr(T_P) where T_P = W_P D is there already
+        __global__ __launch_bounds__(256) void fitTraceKernel(const double *__restrict__ T, double *__restrict__ h,
+                                                              long long n)
+        {
+            const double *t = T + blockIdx.x * n * n;
+            double s = 0.0;
+            for (long long i = threadIdx.x; i < n; i += 256)
+                s += t[i * (n + 1)];
+            s = blockSum256(s);
+            if (threadIdx.x == 0)
+                h[blockIdx.x] = s;
+        }
+
+        // J += sum over the P of group blockIdx.y of W_P h_P
+        __global__ __launch_bounds__(256) void fitCoulombKernel(const double *__restrict__ W, const double *__restrict__ h,
+                                                                double *__restrict__ J, long long n2, int naux, int group)
+        {
+            const long long i = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
+            if (i >= n2)
+                return;
+            const int p0 = blockIdx.y * group, p1 = min(naux, p0 + group);
+            double s = 0.0;
+#pragma unroll 8
+            for (int p = p0; p < p1; p++)
+                s = fma(W[p * n2 + i], h[p], s);
+            unsafeAtomicAdd(&J[i], s);
+        }
+
+        __global__ void zeroKernel(double *p, long long n)
+        {
+            for (long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
+                 i += static_cast<long long>(gridDim.x) * blockDim.x)
+                p[i] = 0.0;
+        }
+
+        // upper triangle from the lower one
+        __global__ void mirrorKernel(double *K, int n)
+        {
+            const long long tot = static_cast<long long>(n) * n;
+            for (long long e = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; e < tot;
+                 e += static_cast<long long>(gridDim.x) * blockDim.x)
+            {
+                const int i = static_cast<int>(e / n), j = static_cast<int>(e % n);
+                if (j > i)
+                    K[e] = K[static_cast<long long>(j) * n + i];
+            }
+        }
+
+        // C[m n + c] (+)= sum_k A[m + n k] B[c + n k]: both operands have the row index contiguous, so
+        // the A and B fragments of v_mfma_f64_16x16x4f64 load straight from memory in 128-byte
+        // segments.  A workgroup of 2 x 2 waves makes a 64 x 64 tile, a wave 32 x 32 of it (four
+        // MFMAs per four loads, the next 16 k fetched while 16 are multiplied); the waves' shared
+        // fragments meet in L1.
+        //   SPLIT = false: T_P = W_P D column by column, A = D, B = W_P (k < n, C stored;
+        //     blockIdx.y = P)
+        //   SPLIT = true:  K = sum_P T_P W_P^T with k = (P, l) running over n naux: for a small n
+        //     the n x n tiles alone leave the chip idle (nine tiles at n = 192), so k is split over
+        //     gridDim.y workgroups per tile that add into C by atomics, and only the tiles with
+        //     row >= column are made (K is symmetric).
+        // At n = 192, naux = 904 (k = 1.7e5): see the figures at riJK.
+        template <bool SPLIT>
+        __global__ __launch_bounds__(256) void panelGemm(const double *__restrict__ A, const double *__restrict__ B,
+                                                         double *__restrict__ C, int n, long long kTotal, long long kChunk)
+        {
+            const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+            const int g = lane >> 4, j = lane & 15;
+            const int nt = (n + 63) / 64;
+            int tr, tc;
+            long long k0, k1;
+            if constexpr (SPLIT)
+            {
+                // blockIdx.y = lower-triangle tile, blockIdx.x = split: the tiles of one split are
+                // gridDim.x apart (a multiple of 8), so one XCD's L2 serves them
+                tr = 0;
+                int t = blockIdx.y;
+                while (t > tr)
+                    t -= ++tr;
+                tc = t;
+                k0 = blockIdx.x * kChunk;
+                k1 = min(kTotal, k0 + kChunk);
+            }
+            else
+            {
+                tr = blockIdx.x / nt;
+                tc = blockIdx.x % nt;
+                k0 = 0;
+                k1 = kTotal;
+                B += blockIdx.y * static_cast<long long>(n) * n;
+                C += blockIdx.y * static_cast<long long>(n) * n;
+            }
+            const int r0 = tr * 64 + (wave >> 1) * 32, c0 = tc * 64 + (wave & 1) * 32;
+            v4d acc[2][2];
+#pragma unroll
+            for (int x = 0; x < 2; x++)
+#pragma unroll
+                for (int y = 0; y < 2; y++)
+                    acc[x][y] = v4d{0, 0, 0, 0};
+            // rows past n read row n - 1; their results are not stored
+            const int ra[2] = {min(r0 + j, n - 1), min(r0 + 16 + j, n - 1)};
+            const int cb[2] = {min(c0 + j, n - 1), min(c0 + 16 + j, n - 1)};
+            auto load = [&](long long k, double (&a)[4][2], double (&b)[4][2]) {
+#pragma unroll
+                for (int s = 0; s < 4; s++)
+                {
+                    const long long kk = k + 4 * s + g;
+                    const bool in = kk < k1;
+                    const long long off = (in ? kk : k1 - 1) * n;
+#pragma unroll
+                    for (int x = 0; x < 2; x++)
+                    {
+                        const double v = A[off + ra[x]];
+                        a[s][x] = in ? v : 0.0;
+                        b[s][x] = B[off + cb[x]];
+                    }
+                }
+            };
+            double a[4][2], b[4][2], an[4][2], bn[4][2];
+            if (k0 < k1)
+            {
+                load(k0, a, b);
+                for (long long k = k0; k < k1; k += 16)
+                {
+                    if (k + 16 < k1)
+                        load(k + 16, an, bn);
+#pragma unroll
+                    for (int s = 0; s < 4; s++)
+#pragma unroll
+                        for (int x = 0; x < 2; x++)
+#pragma unroll
+                            for (int y = 0; y < 2; y++)
+                                acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s][x], b[s][y], acc[x][y], 0, 0, 0);
+#pragma unroll
+                    for (int s = 0; s < 4; s++)
+#pragma unroll
+                        for (int x = 0; x < 2; x++)
+                        {
+                            a[s][x] = an[s][x];
+                            b[s][x] = bn[s][x];
+                        }
+                }
+            }
+            // accumulator element r of lane (g, j): row 4 r + g, column j
+#pragma unroll
+            for (int x = 0; x < 2; x++)
+#pragma unroll
+                for (int y = 0; y < 2; y++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                    {
+                        const int row = r0 + 16 * x + 4 * r + g, col = c0 + 16 * y + j;
+                        if (row < n && col < n)
+                        {
+                            double *dst = &C[static_cast<long long>(row) * n + col];
+                            if constexpr (SPLIT)
+                                unsafeAtomicAdd(dst, acc[x][y][r]);
+                            else
+                                *dst = acc[x][y][r];
+                        }
+                    }
         }
 
         void rb(rocblas_status s, const char *what)
@@ -87,11 +275,13 @@ namespace lbx
     {
         std::lock_guard<std::mutex> lk(c.ri_mu);
         const long long n2 = n * n;
-        Handle h(stream);
         if (K && !c.ri_t)
             c.ri_t = c.alloc<double>(static_cast<size_t>(n2 * naux));
         if (!c.ri_ready)
         {
+            Handle h(stream);
+            if (!c.ri_h)
+                c.ri_h = c.alloc<double>(static_cast<size_t>(naux));
             if (!c.ri_w)
                 c.ri_w = c.alloc<double>(static_cast<size_t>(n2 * naux));
             // dense (mn|P), mn-major as the eri3 entry writes it, then P-major into W's buffer
@@ -140,23 +330,42 @@ namespace lbx
             LBX_HIP(hipStreamSynchronize(stream));
             c.ri_ready = true;
         }
-        const double one = 1.0, zero = 0.0;
-        Buf g(sizeof(double) * naux);
-        rb(rocblas_dgemv_64(h.h, rocblas_operation_transpose, n2, naux, &one, c.ri_w, n2, D, 1, &zero, g.d(), 1),
-           "rocblas_dgemv (h = W^T d)");
-        rb(rocblas_dgemv_64(h.h, rocblas_operation_none, n2, naux, &one, c.ri_w, n2, g.d(), 1, &zero, J, 1),
-           "rocblas_dgemv (J = W h)");
+        const int ni = static_cast<int>(n);
+        auto blocks1d = [](long long m) { return dim3(static_cast<int>(std::min<long long>((m + 255) / 256, 65536))); };
         if (K)
         {
-            // T_P = W_P D (W_P and D symmetric, so row- and column-major readings agree)
-            rb(rocblas_dgemm_strided_batched_64(h.h, rocblas_operation_none, rocblas_operation_none, n, n, n, &one,
-                                                c.ri_w, n, n2, D, n, 0, &zero, c.ri_t, n, n2, naux),
-               "rocblas_dgemm_strided_batched (T_P = W_P D)");
-            // K = sum_P T_P W_P^T = [T_1 .. T_naux] [W_1 .. W_naux]^T, k = nbf * naux
-            rb(rocblas_dgemm_64(h.h, rocblas_operation_none, rocblas_operation_transpose, n, n, n * naux, &one,
-                                c.ri_t, n, c.ri_w, n, &zero, K, n),
-               "rocblas_dgemm (K)");
+            // T_P = W_P D (W_P and D symmetric, so row- and column-major readings agree); blockIdx.y
+            // holds at most 65535 auxiliary functions
+            const int nt = (ni + 63) / 64;
+            for (long long p0 = 0; p0 < naux; p0 += 65535)
+            {
+                const int np = static_cast<int>(std::min<long long>(65535, naux - p0));
+                hipLaunchKernelGGL((panelGemm<false>), dim3(nt * nt, np), dim3(256), 0, stream, D, c.ri_w + p0 * n2,
+                                   c.ri_t + p0 * n2, ni, n, n);
+            }
+            // K = sum_P T_P W_P^T
+            hipLaunchKernelGGL(zeroKernel, blocks1d(n2), dim3(256), 0, stream, K, n2);
+            const long long tiles = static_cast<long long>(nt) * (nt + 1) / 2, kTotal = n * naux;
+            long long splits = std::max<long long>(1, 1024 / tiles);
+            splits = std::min(splits, (kTotal + 255) / 256);   // at least 256 k per workgroup
+            splits = (splits + 7) / 8 * 8;
+            const long long chunk = ((kTotal + splits - 1) / splits + 15) / 16 * 16;
+            hipLaunchKernelGGL((panelGemm<true>), dim3(static_cast<int>(splits), static_cast<int>(tiles)), dim3(256), 0,
+                               stream, c.ri_t, c.ri_w, K, ni, kTotal, chunk);
+            hipLaunchKernelGGL(mirrorKernel, blocks1d(n2), dim3(256), 0, stream, K, ni);
+            hipLaunchKernelGGL(fitTraceKernel, dim3(static_cast<int>(naux)), dim3(256), 0, stream, c.ri_t, c.ri_h, n);
         }
+        else
+            hipLaunchKernelGGL(fitDotKernel, dim3(static_cast<int>(naux)), dim3(256), 0, stream, c.ri_w, D, c.ri_h, n2);
+        {
+            // J: groups of P so that about 2048 workgroups share the pass over W
+            const long long bx = (n2 + 255) / 256;
+            const int group = static_cast<int>(std::max<long long>(8, naux * bx / 2048));
+            hipLaunchKernelGGL(zeroKernel, blocks1d(n2), dim3(256), 0, stream, J, n2);
+            hipLaunchKernelGGL(fitCoulombKernel, dim3(static_cast<int>(bx), static_cast<int>((naux + group - 1) / group)),
+                               dim3(256), 0, stream, c.ri_w, c.ri_h, J, n2, static_cast<int>(naux), group);
+        }
+        LBX_HIP(hipGetLastError());
         LBX_HIP(hipStreamSynchronize(stream));
     }
 }
