@@ -24,12 +24,17 @@ SELFTEST_SRC = os.path.join(ROOT, "tests", "cpp", "ints_selftest.cpp")
 SELFTEST = os.path.join(HERE, "bin", "ints_selftest")
 
 N_UNITS = 24   # csrc/instances.hip: 0..11 FP64 forms and dense outputs, 12..23 FP32 forms
+N_PARTS = 5    # parts of the units whose bra class is above (pp|; the others are one part
+N_WAVE_UNITS = 27   # csrc/wave_instances.hip: 0..11 FP64 one-wave MFMA forms, 12..21 FP32 forms, 22..26 g pairs
 N_GRAD_UNITS = 10   # csrc/grad_instances.hip: one per lane-side main pair class
 N_BLOCK_UNITS = 20  # csrc/block_instances.hip: 0..9 FP64 block J/K forms per bra class, 10..19 FP32
 
 FLAGS = [
     "-O3", "-std=c++17", "-fPIC", "--offload-arch=gfx950", "-mcode-object-version=5",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # The kernels fill the register file; machine LICM hoists the constants of the Boys function and
+    # unrolled addresses out of the task loops into 30-60 more registers, which then spill.
+    "-mllvm", "-disable-machine-licm",
     "-munsafe-fp-atomics", "-ffp-contract=fast", f"-I{INCLUDE}",
     "-Wall", "-Wno-unused-function", "-Wno-unused-variable",
 ]
@@ -77,7 +82,7 @@ def _big_stack():
 
 def _compile(src: str, obj: str, defines: list[str]) -> tuple[str, float]:
     t = time.time()
-    cmd = [hipcc(), "-x", "hip", "-c", src, "-o", obj] + FLAGS + defines
+    cmd = [hipcc(), "-x", "hip", "-c", src, "-o", obj, "-MMD", "-MF", obj + ".d"] + FLAGS + defines
     r = subprocess.run(cmd, capture_output=True, text=True, preexec_fn=_big_stack)
     if r.returncode != 0:
         raise RuntimeError(f"compile failed: {' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
@@ -85,14 +90,13 @@ def _compile(src: str, obj: str, defines: list[str]) -> tuple[str, float]:
 
 
 def _stale(src: str, obj: str) -> bool:
-    """True unless obj is newer than src, every header and this script."""
-    if not os.path.exists(obj):
+    """True unless obj is newer than src and every project header its last compilation read."""
+    if not os.path.exists(obj) or not os.path.exists(obj + ".d"):
         return True
-    deps = [src, os.path.abspath(__file__)]
-    for d in (CSRC, INCLUDE):
-        for base, _, files in os.walk(d):
-            deps += [os.path.join(base, f) for f in files if f.endswith((".h", ".hpp"))]
-    return os.path.getmtime(obj) < max(os.path.getmtime(p) for p in deps)
+    with open(obj + ".d") as f:
+        words = f.read().replace("\\\n", " ").split()
+    deps = [src] + [w for w in words if not w.endswith(":") and (w.startswith(ROOT) or w.startswith(CSRC))]
+    return any(not os.path.exists(p) or os.path.getmtime(obj) < os.path.getmtime(p) for p in deps)
 
 
 def build(jobs: int | None = None, verbose: bool = True, incremental: bool = False) -> str:
@@ -110,7 +114,12 @@ def build(jobs: int | None = None, verbose: bool = True, incremental: bool = Fal
         (os.path.join(CSRC, "generic.hip"), os.path.join(BUILD, "generic.o"), []),
     ]
     for u in range(N_UNITS):
-        work.append((os.path.join(CSRC, "instances.hip"), os.path.join(BUILD, f"inst_{u}.o"),
+        parts = N_PARTS if u % 12 > 2 else 1
+        for k in range(parts):
+            work.append((os.path.join(CSRC, "instances.hip"), os.path.join(BUILD, f"inst_{u}_{k}.o"),
+                         [f"-DLBX_UNIT={u}", f"-DLBX_NPARTS={parts}", f"-DLBX_PART={k}"]))
+    for u in range(N_WAVE_UNITS):
+        work.append((os.path.join(CSRC, "wave_instances.hip"), os.path.join(BUILD, f"wave_{u}.o"),
                      [f"-DLBX_UNIT={u}"]))
     for u in range(N_BLOCK_UNITS):
         work.append((os.path.join(CSRC, "block_instances.hip"), os.path.join(BUILD, f"block_{u}.o"),

@@ -1,6 +1,7 @@
 // The C-ABI of lbx (include/lbx.h): context set-up, Schwarz screening, task tables and the
 // drivers that launch the quartet kernels class pair by class pair.
 #include "grad.hpp"
+#include "lbx_internal.hpp"
 #include "quartet.hpp"
 #include "registry.hpp"
 #include "tasks.hpp"
@@ -442,6 +443,8 @@ namespace lbx
             return valuCost(lane, unif, nc, true) > 2.0 * valuCost(lane, unif, nc);
         }
 
+        bool lane(const KernelSlot &s) { return s.fn && s.kind == KIND_LANE; }
+
         // Default variant before tuning: the cheaper one-lane-per-quartet form by the work
         // estimate (with the lane side's longest-lane contraction); MFMA when no such form fits the
         // registers; for J/K the block form when the cheaper one-lane form diverges.
@@ -449,9 +452,9 @@ namespace lbx
         {
             const KernelSlot &vb = kernelSlot(mode, bra.la, bra.lb, ket.la, ket.lb, VAR_VALU_BRA);
             const KernelSlot &vk = kernelSlot(mode, bra.la, bra.lb, ket.la, ket.lb, VAR_VALU_KET);
-            double cb = vb.fn ? valuCost(bra, ket, vb.nc, true) : 1e300;
-            double ck = vk.fn ? valuCost(ket, bra, vk.nc, true) : 1e300;
-            if (!vb.fn && !vk.fn)
+            double cb = lane(vb) ? valuCost(bra, ket, vb.nc, true) : 1e300;
+            double ck = lane(vk) ? valuCost(ket, bra, vk.nc, true) : 1e300;
+            if (!lane(vb) && !lane(vk))
                 return VAR_MFMA;
             const bool bra_lanes = cb <= ck;
             if (mode == MODE_JK && kernelSlot(mode, bra.la, bra.lb, ket.la, ket.lb, VAR_BLOCK).fn &&
@@ -467,10 +470,10 @@ namespace lbx
         {
             const KernelSlot &vb = kernelSlot(MODE_JK, bra.la, bra.lb, ket.la, ket.lb, VAR_VALU_BRA32);
             const KernelSlot &vk = kernelSlot(MODE_JK, bra.la, bra.lb, ket.la, ket.lb, VAR_VALU_KET32);
-            if (!vb.fn && !vk.fn)
+            if (!lane(vb) && !lane(vk))
                 return kernelSlot(MODE_JK, bra.la, bra.lb, ket.la, ket.lb, VAR_MFMA32).fn ? VAR_MFMA32 : -1;
-            double cb = vb.fn ? valuCost(bra, ket, vb.nc, true) : 1e300;
-            double ck = vk.fn ? valuCost(ket, bra, vk.nc, true) : 1e300;
+            double cb = lane(vb) ? valuCost(bra, ket, vb.nc, true) : 1e300;
+            double ck = lane(vk) ? valuCost(ket, bra, vk.nc, true) : 1e300;
             const bool bra_lanes = cb <= ck;
             if (kernelSlot(MODE_JK, bra.la, bra.lb, ket.la, ket.lb, VAR_BLOCK32).fn &&
                 (bra_lanes ? laneDivergent(bra, ket, vb.nc) : laneDivergent(ket, bra, vk.nc)))
@@ -685,6 +688,9 @@ struct lbx_context : Context
     double window_lo = 0.0, window_hi = kNoUpper;
     // lbx_eri*_batch: (shell a, shell b) -> pair index per main pair class
     std::vector<std::unordered_map<long long, int>> pair_maps;
+    // their task list on the device (1 MiB, made on first use; every call waits for its kernel)
+    static constexpr size_t kBlockTaskInts = 1 << 18;
+    int *block_tasks = nullptr;
     // this device's scratch array (lbx_eri4_batch_static)
     int *d_scratch = nullptr;
 
@@ -1643,7 +1649,6 @@ extern "C"
             long long bsize = 1;
             for (int k = 0; k < per; k++)
                 bsize *= nSph(l[k]);
-            fill(out, nq * ncomp * bsize, 0.0, c.stream);
             // library pair classes of the two sides
             PairClass *bra, *ket;
             int ibra = -1, iket = -1;
@@ -1677,6 +1682,17 @@ extern "C"
                 auto it = std::lower_bound(pc.sh_a.begin(), pc.sh_a.end(), s);
                 return it != pc.sh_a.end() && *it == s ? static_cast<int>(it - pc.sh_a.begin()) : -1;
             };
+            // The integrals themselves: the compiled one-wave kernel of the class pair, whose bra is
+            // the side with the higher class (or higher l of two auxiliary shells); the run-time-L
+            // kernel for derivatives and for main-basis g shells, which it does not cover.
+            const bool flip = kind == 2 ? bra->la < ket->la
+                                        : kernelSlot(MODE_BLOCK, bra->la, bra->lb, ket->la, ket->lb, VAR_MFMA).fn == nullptr;
+            const KernelSlot *wave = nullptr;
+            if (op == D1_OP_PLAIN)
+                wave = flip ? &kernelSlot(MODE_BLOCK, ket->la, ket->lb, bra->la, bra->lb, VAR_MFMA)
+                            : &kernelSlot(MODE_BLOCK, bra->la, bra->lb, ket->la, ket->lb, VAR_MFMA);
+            if (wave && !wave->fn)
+                wave = nullptr;
             std::vector<int> tasks;
             tasks.reserve(4 * nq);
             for (long long t = 0; t < nq; t++)
@@ -1696,8 +1712,14 @@ extern "C"
                 }
                 if (p < 0 || q < 0)
                     continue;
-                tasks.insert(tasks.end(), {p, q, (sab ? 1 : 0) | (scd ? 2 : 0), static_cast<int>(t)});
+                if (wave && flip)
+                    tasks.insert(tasks.end(), {q, p, (scd ? 1 : 0) | (sab ? 2 : 0) | 4, static_cast<int>(t)});
+                else
+                    tasks.insert(tasks.end(), {p, q, (sab ? 1 : 0) | (scd ? 2 : 0), static_cast<int>(t)});
             }
+            // entries without a task stay zero; the one-wave kernel writes every element of the others
+            if (!wave || static_cast<long long>(tasks.size()) < 4 * nq)
+                fill(out, nq * ncomp * bsize, 0.0, c.stream);
             if (tasks.empty())
                 return;
             if (op == D1_OP_DERIV || op == D1_OP_SOC)
@@ -1707,44 +1729,67 @@ extern "C"
                 if (kind == 4 && op == D1_OP_DERIV)
                     computeEcoeffsD1(c, *ket);
             }
-            // the task list: in a buffer of this call, or in the device's scratch array
-            // (staging != nullptr: the allocation-free entry, at most kStaticEntries entries)
+            // the task list: in the device's scratch array (staging != nullptr: the allocation-free
+            // entry, at most kStaticEntries entries), in the context's buffer (lists of up to
+            // kBlockTaskInts ints), or in a buffer of this call
+            const bool kept = !staging && tasks.size() <= lbx_context::kBlockTaskInts;
             void *d = staging;
-            if (!staging)
+            if (kept)
+            {
+                if (!c.block_tasks)
+                    c.block_tasks = c.alloc<int>(lbx_context::kBlockTaskInts);
+                d = c.block_tasks;
+            }
+            else if (!staging)
                 LBX_HIP(hipMalloc(&d, tasks.size() * sizeof(int)));
             try
             {
                 LBX_HIP(hipMemcpyAsync(d, tasks.data(), tasks.size() * sizeof(int), hipMemcpyHostToDevice,
                                        c.stream));
-                D1Args a{};
-                a.bra = bra->view();
-                a.ket = ket->view();
-                a.la = bra->la;
-                a.lb = bra->lb;
-                a.lc = ket->la;
-                a.ld = ket->lb;
-                a.bra_single = bra->single ? 1 : 0;
-                a.ket_single = ket->single ? 1 : 0;
-                a.tasks = static_cast<const int *>(d);
-                a.ntasks = static_cast<long long>(tasks.size() / 4);
-                a.boys = c.d_boys;
-                a.out = out;
-                a.kind = kind;
-                a.nbf = static_cast<long long>(c.nbf);
-                a.naux = static_cast<long long>(c.nbf_aux);
-                a.blocks = 1;
-                a.op = op;
-                launchD1(a, c.stream);
+                if (wave)
+                {
+                    KArgs a{};
+                    a.bra = (flip ? ket : bra)->view();
+                    a.ket = (flip ? bra : ket)->view();
+                    a.plo = static_cast<const int *>(d);
+                    a.ntasks = static_cast<long long>(tasks.size() / 4);
+                    a.boys = c.d_boys;
+                    a.out = out;
+                    wave->fn(a, c.stream);
+                    LBX_HIP(hipGetLastError());
+                }
+                else
+                {
+                    D1Args a{};
+                    a.bra = bra->view();
+                    a.ket = ket->view();
+                    a.la = bra->la;
+                    a.lb = bra->lb;
+                    a.lc = ket->la;
+                    a.ld = ket->lb;
+                    a.bra_single = bra->single ? 1 : 0;
+                    a.ket_single = ket->single ? 1 : 0;
+                    a.tasks = static_cast<const int *>(d);
+                    a.ntasks = static_cast<long long>(tasks.size() / 4);
+                    a.boys = c.d_boys;
+                    a.out = out;
+                    a.kind = kind;
+                    a.nbf = static_cast<long long>(c.nbf);
+                    a.naux = static_cast<long long>(c.nbf_aux);
+                    a.blocks = 1;
+                    a.op = op;
+                    launchD1(a, c.stream);
+                }
                 LBX_HIP(hipStreamSynchronize(c.stream));
             }
             catch (...)
             {
                 (void)hipStreamSynchronize(c.stream);
-                if (!staging)
+                if (!staging && !kept)
                     (void)hipFree(d);
                 throw;
             }
-            if (!staging)
+            if (!staging && !kept)
                 (void)hipFree(d);
         }
 

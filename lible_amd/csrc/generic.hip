@@ -21,7 +21,8 @@
 //     U_x = sum_{ab,cd} W[ab][cd] sum_h Eb'_i,x[h][ab] X[h][cd]
 //     dA += (a/p) T + U,  dB += (b/p) T - U,  dC += V - (c/q) T,  dD = -(dA + dB + dC).
 #include "grad.hpp"
-#include "quartet.hpp"
+#include "lbx_internal.hpp"
+#include "quartet_wave.hpp"
 #include "runtime_l.hpp"
 
 #include <utility>
@@ -662,7 +663,9 @@ namespace lbx
         void regQuartetSlot()
         {
             constexpr int lb = N / 36, lc = (N / 6) % 6, ld = N % 6;
-            if constexpr (wantedSlot(MODE, 4, lb, lc, ld))
+            // J/K: only the class pairs the compiled one-wave form does not cover
+            constexpr bool compiled = MODE == MODE_JK && lc <= 4 && WavePlan<4, lb, lc, ld, double>::kFitsG;
+            if constexpr (wantedSlot(MODE, 4, lb, lc, ld) && !compiled)
             {
                 KernelSlot &s = kernelSlot(MODE, 4, lb, lc, ld, VAR_MFMA);
                 s.fn = &launchGenericQuartet<MODE, 4, lb, lc, ld>;

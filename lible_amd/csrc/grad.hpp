@@ -25,7 +25,7 @@
 #pragma once
 
 #include "device_common.hpp"
-#include "lbx_internal.hpp"
+#include "dpairs.hpp"
 
 namespace lbx
 {

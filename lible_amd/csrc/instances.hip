@@ -4,11 +4,17 @@
 //          (ab|c) against every auxiliary shell l = 0..5 not already covered;
 //   10, 11 bra = single auxiliary shell l = 4, 5: eri2 (a|b) for b <= l and the (a|a) diagonal;
 //   12..23 the FP32 forms of units 0..11: J/K and the batched RI sums.
-// Splitting the instantiations lets the build compile the units in parallel.
+// The one-lane forms (quartet.hpp); the one-wave MFMA forms are in wave_instances.hip.
+// Splitting the instantiations lets the build compile the units in parallel: each unit once per
+// LBX_PART in 0..LBX_NPARTS-1, which takes the ket classes with index % LBX_NPARTS == LBX_PART.
 #include "quartet.hpp"
 
 #ifndef LBX_UNIT
 #error "LBX_UNIT must be defined"
+#endif
+#ifndef LBX_NPARTS
+#define LBX_NPARTS 1
+#define LBX_PART 0
 #endif
 
 namespace lbx
@@ -33,10 +39,12 @@ namespace lbx
         constexpr int PA = unitLa(), PB = unitLb();
         constexpr int CI = pairClassIdx(PA, PB);
 
+        constexpr bool mine(int i) { return i % LBX_NPARTS == LBX_PART; }
+
         template <int LC, int LD>
         void regEri4()
         {
-            if constexpr (kPairUnit < 10 && pairClassIdx(LC, LD) <= CI)
+            if constexpr (mine(pairClassIdx(LC, LD)) && kPairUnit < 10 && pairClassIdx(LC, LD) <= CI)
             {
                 if constexpr (kF32Unit)
                     registerQuartet<PA, PB, LC, LD, MODE_JK, 2>();
@@ -51,22 +59,22 @@ namespace lbx
         template <int LC>
         void regEri3()
         {
-            if constexpr (!kF32Unit && kPairUnit < 10 && !(LC <= 3 && pairClassIdx(LC, 0) <= CI))
+            if constexpr (mine(LC) && !kF32Unit && kPairUnit < 10 && !(LC <= 3 && pairClassIdx(LC, 0) <= CI))
                 registerQuartet<PA, PB, LC, 0, MODE_DENSE, 1>();
             // batched RI sums: eri3 (PA PB | LC), and eri2 (PA | LC) when PB = 0
-            if constexpr (kPairUnit < 10)
+            if constexpr (mine(LC) && kPairUnit < 10)
                 registerQuartet<PA, PB, LC, 0, MODE_SUM, kF32Unit ? 2 : 1>();
         }
 
         template <int LC>
         void regEri2()
         {
-            if constexpr (!kF32Unit && kPairUnit >= 10 && LC <= PA)
+            if constexpr (mine(LC) && !kF32Unit && kPairUnit >= 10 && LC <= PA)
             {
                 registerQuartet<PA, 0, LC, 0, MODE_DENSE, 1>();
                 registerQuartet<PA, 0, LC, 0, MODE_SUM, 1>();
             }
-            if constexpr (kF32Unit && kPairUnit >= 10 && LC <= PA)
+            if constexpr (mine(LC) && kF32Unit && kPairUnit >= 10 && LC <= PA)
                 registerQuartet<PA, 0, LC, 0, MODE_SUM, 2>();
         }
 
@@ -96,7 +104,7 @@ namespace lbx
                 regEri2<3>();
                 regEri2<4>();
                 regEri2<5>();
-                if constexpr (!kF32Unit)
+                if constexpr (mine(0) && !kF32Unit)
                     registerQuartet<PA, PB, PA, PB, MODE_DIAG, 1>();
             }
         } registrar;

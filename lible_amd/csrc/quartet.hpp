@@ -26,8 +26,11 @@
 // Epilogues: J/K contraction with atomics, dense tensor scatter, or the (ab|ab) diagonal.
 #pragma once
 
+#include <algorithm>
+#include <type_traits>
+
 #include "device_common.hpp"
-#include "lbx_internal.hpp"
+#include "dpairs.hpp"
 #include "registry.hpp"
 
 namespace lbx
@@ -38,7 +41,11 @@ namespace lbx
         MODE_DENSE = 1,
         MODE_DIAG = 2,
         MODE_SUM = 3,   // per-molecule sums of |value| and value of the dense eri3 / eri2 tensors
-        N_MODES = 4
+        MODE_BLOCK = 4, // blocks of listed pair combinations (one-wave form only): plo = ntasks x
+                        // (bra pair, ket pair, flags, slot), block at out + slot * its size; flags
+                        // bit 0 / 1: the caller's bra / ket shells are the pair's in reverse,
+                        // bit 2: the caller's first side is the ket
+        N_MODES = 5
     };
 
     struct KArgs
@@ -116,19 +123,22 @@ namespace lbx
         }
         static constexpr int NC0f = ncFor32(SP, HP, SQ);
         static constexpr int NC1f = ncFor32(SQ, HQ, SP);
+        // Whether the one-lane form is built: at most three column passes (each its own instance) or
+        // up to seven of at least three columns, and at most 5500 FMAs in the unrolled transforms.
+        // Past that its waves run 2-28 times slower than the one-wave form (spilled registers,
+        // code beyond the instruction cache: (ff|ps) FP32 28x, (fd|ps) FP32 27x, (dp|dp) FP64 1.2 ms
+        // for one wave), which then serves the class pair under this variant too.
+        static constexpr bool laneBuilt(int nc, int sl, int hl, int su, int hu)
+        {
+            if (nc < 1)
+                return false;
+            const int passes = ceilDiv(su, nc);
+            return (passes <= 3 || (passes <= 7 && nc >= 3)) && nc * (hl * hu + sl * hl) <= 5500;
+        }
+        static constexpr bool kLane0 = laneBuilt(NC0, SP, HP, SQ, HQ), kLane1 = laneBuilt(NC1, SQ, HQ, SP, HP);
+        static constexpr bool kLane0f = laneBuilt(NC0f, SP, HP, SQ, HQ), kLane1f = laneBuilt(NC1f, SQ, HQ, SP, HP);
         template <typename T, bool SWAP>
         static constexpr int nc() { return sizeof(T) == 4 ? (SWAP ? NC1f : NC0f) : (SWAP ? NC1 : NC0); }
-
-        // ---- MFMA tiling
-        static constexpr int NQ = ceilDiv(SQ, 16), NP = ceilDiv(SP, 16), KQ = ceilDiv(HQ, 4);
-        // row tiles per chunk: accumulators (acc1 + acc2) within ~96 doubles per lane, rows for
-        // about four primitive pairs, at least one tile
-        static constexpr int mtBudget = (96 - 4 * NQ * NP) / (4 * NQ);
-        static constexpr int mtRows = ceilDiv(4 * HP, 16);
-        static constexpr int MT0 = mtBudget < mtRows ? mtBudget : mtRows;
-        static constexpr int MT = MT0 < 1 ? 1 : MT0;
-        static constexpr int RC = 16 * MT;                          // rows per chunk
-        static constexpr int CHP = (RC - 1) / HP + 2;               // primitives a chunk touches
     };
 
     // ------------------------------------------------------------------------------- dense out
@@ -221,6 +231,20 @@ namespace lbx
             unsafeAtomicAdd(addr, v);
     }
 
+    // MODE_SUM: a wave's sums (per lane) to its molecule's.  Once per run of tasks of a molecule:
+    // additions to one line run at about 60 M/s, which a flush per task would exhaust.
+    __device__ __forceinline__ void flushSums(const KArgs &A, int mol, int lane, double sabs, double ssum)
+    {
+        sabs = waveSum(sabs);
+        ssum = waveSum(ssum);
+        if (lane == 0)
+        {
+            double *o = A.out + 4 * static_cast<long long>(mol) + (A.kind == 3 ? 0 : 2);
+            unsafeAtomicAdd(o, sabs);
+            unsafeAtomicAdd(o + 1, ssum);
+        }
+    }
+
     // ------------------------------------------------------------------------------- quartetV
     // One quartet per lane: lane-side pair l (64 consecutive sorted positions) against the
     // wave-uniform pair u.  SWAP = false: lanes = bra, u = ket; SWAP = true: lanes = ket, u = bra.
@@ -230,6 +254,8 @@ namespace lbx
     // scaled by 2f.  CARRY = false: zeroed here and added to J at the end of the task; CARRY =
     // true: accumulated into the caller's array, which adds it to J once for a run of tasks that
     // share the lane-side pairs.
+    // MODE_SUM: the lane's weighted sums of |value| and value are added to jl[0] and jl[1], which
+    // the caller adds to the molecule's sums once for a run of tasks of one molecule.
     template <int LA, int LB, int LC, int LD, int MODE, bool SWAP, typename T, bool CARRY = false>
     __device__ __forceinline__ void quartetVTask(const KArgs &A, int q, int local, int lane, double *jl)
     {
@@ -599,14 +625,8 @@ namespace lbx
             // images in the dense tensor: (ab|P) and (ba|P) for distinct shells; (P|Q), (Q|P)
             const bool one = A.kind == 3 ? LP.sh_a[l] == LP.sh_b[l] : (A.same_class && p == q);
             const double w = active ? (one ? 1.0 : 2.0) : 0.0;
-            sabs = waveSum(w * sabs);
-            ssum = waveSum(w * ssum);
-            if (lane == 0)
-            {
-                double *o = A.out + 4 * static_cast<long long>(uniform(UP.mol[u])) + (A.kind == 3 ? 0 : 2);
-                unsafeAtomicAdd(o, sabs);
-                unsafeAtomicAdd(o + 1, ssum);
-            }
+            jl[0] = fma(w, sabs, jl[0]);
+            jl[1] = fma(w, ssum, jl[1]);
         }
     }
 
@@ -627,7 +647,7 @@ namespace lbx
         const long long w = static_cast<long long>(blockIdx.x) * 4 + wave;
         constexpr int SLb = nSph(SWAP ? LD : LB);
         constexpr int SL = nSph(SWAP ? LC : LA) * SLb;
-        double jl[SL];
+        double jl[MODE == MODE_SUM ? 2 : SL];
         if constexpr (MODE == MODE_JK)
         {
             if (A.block_major)
@@ -681,6 +701,7 @@ namespace lbx
             return;
         int q = uniform(findKet(A.prefix, A.nket, t0));
         long long base = A.prefix[q], next = A.prefix[q + 1];
+        int mol = -1;   // MODE_SUM: the molecule of the sums in jl
         for (long long t = t0; t < t1; t++)
         {
             while (t >= next)
@@ -688,370 +709,23 @@ namespace lbx
                 q++;
                 base = next;
                 next = A.prefix[q + 1];
+            }
+            if constexpr (MODE == MODE_SUM)
+            {
+                const int m = uniform(A.ket.mol[A.ket.order[q]]);
+                if (m != mol)
+                {
+                    if (mol >= 0)
+                        flushSums(A, mol, lane, jl[0], jl[1]);
+                    mol = m;
+                    jl[0] = jl[1] = 0.0;
+                }
             }
             quartetVTask<LA, LB, LC, LD, MODE, SWAP, T>(A, q, uniform(A.plo[q]) + 64 * static_cast<int>(t - base),
                                                         lane, jl);
         }
-    }
-
-    // ------------------------------------------------------------------------------- quartetM
-    typedef float v4f __attribute__((ext_vector_type(4)));
-
-    // 16x16x4 MFMA in FP64 or FP32.  Both take A[j][g] and B[g][j] from lane (g, j) = (lane / 16,
-    // lane % 16); accumulator element r of that lane holds D[4 r + g][j] for FP64 and
-    // D[4 g + r][j] for FP32.
-    __device__ __forceinline__ v4d mfma16(double a, double b, v4d c)
-    {
-        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-    }
-    __device__ __forceinline__ v4f mfma16(float a, float b, v4f c)
-    {
-        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-    }
-
-    // T = double, or float (the small-bound quartets of mixed-precision J/K: R, the E matrices
-    // and both transforms in FP32 on the FP32 MFMA; Boys values and the epilogue in FP64).
-    template <int LA, int LB, int LC, int LD, int MODE, typename T = double>
-    __global__ __launch_bounds__(64) void quartetM(const KArgs A)
-    {
-        using C = Cls<LA, LB, LC, LD>;
-        constexpr int L = C::L, HP = C::HP, HQ = C::HQ, SP = C::SP, SQ = C::SQ, HL = C::HL;
-        constexpr int NQ = C::NQ, NP = C::NP, KQ = C::KQ, MT = C::MT, RC = C::RC, CHP = C::CHP;
-        constexpr int SA = C::SA, SB = C::SB, SC = C::SC, SD = C::SD;
-        constexpr bool F32 = sizeof(T) == 4;
-        using Acc = std::conditional_t<F32, v4f, v4d>;
-        static_assert(!F32 || MODE == MODE_JK, "FP32 MFMA form: J/K only");
-        static_assert(CHP <= 64, "one lane per primitive pair of a chunk");
-        __shared__ T sR[2][CHP][HL];
-        __shared__ double sInit[CHP][L + 1];
-        __shared__ T sPQ[CHP][3];
-        __shared__ unsigned short sTab[HP][4 * KQ];
-        __shared__ double sI[SP * SQ];
-        __shared__ double sD[6][49];
-
-        const int lane = threadIdx.x;
-        const int g = lane >> 4, j = lane & 15;
-
-        // Hermite-sum table: row tuv, column t'u'v' -> index of the summed Hermite function
-        for (int e = lane; e < HP * 4 * KQ; e += 64)
-        {
-            const int h = e / (4 * KQ), k = e % (4 * KQ);
-            int v = 0;
-            if (k < HQ)
-            {
-                const int a = hermTuv(h), b = hermTuv(k);
-                v = hermIdx((a & 255) + (b & 255), ((a >> 8) & 255) + ((b >> 8) & 255),
-                            (a >> 16) + (b >> 16));
-            }
-            sTab[h][k] = static_cast<unsigned short>(v);
-        }
-        for (int e = lane; e < 2 * CHP * HL; e += 64)
-            (&sR[0][0][0])[e] = T(0);
-        __syncthreads();
-
-        // contiguous task range per workgroup
-        const long long t0 = A.ntasks * blockIdx.x / gridDim.x;
-        const long long t1 = A.ntasks * (blockIdx.x + 1) / gridDim.x;
-        if (t0 >= t1)
-            return;
-        int q = uniform(findKet(A.prefix, A.nket, t0));
-        long long base = A.prefix[q], next = A.prefix[q + 1];
-        for (long long t = t0; t < t1; t++)
-        {
-            while (t >= next)
-            {
-                q++;
-                base = next;
-                next = A.prefix[q + 1];
-            }
-            const int p = uniform(A.plo[q] + static_cast<int>(t - base));
-            // task tables run over the ket pairs of one bra pair when bra_major is set (the
-            // larger E matrix is then shared by consecutive tasks and stays in cache)
-            const int cd = uniform(A.ket.order[A.bra_major ? p : q]);
-            const int ab = uniform(A.bra.order[A.bra_major ? q : p]);
-            const int kpoff = uniform(A.ket.poff[cd]), kcnt = uniform(A.ket.pcnt[cd]);
-            const int bpoff = uniform(A.bra.poff[ab]), bcnt = uniform(A.bra.pcnt[ab]);
-            const int nrows = bcnt * HP;
-
-            Acc acc2[NQ][NP];
-#pragma unroll
-            for (int a = 0; a < NQ; a++)
-#pragma unroll
-                for (int b = 0; b < NP; b++)
-                    acc2[a][b] = Acc{0, 0, 0, 0};
-
-            for (int rowbase = 0; rowbase < nrows; rowbase += RC)
-            {
-                const int prim0 = rowbase / HP;
-                const int primEnd = min(bcnt, (rowbase + RC - 1) / HP + 1);
-                const int nprim = primEnd - prim0;
-
-                Acc acc1[MT][NQ];
-#pragma unroll
-                for (int a = 0; a < MT; a++)
-#pragma unroll
-                    for (int b = 0; b < NQ; b++)
-                        acc1[a][b] = Acc{0, 0, 0, 0};
-
-                for (int k = 0; k < kcnt; k++)
-                {
-                    const double4 Q = A.ket.pp[kpoff + k];
-                    // Boys + scaled R^{(n)}_000 for the chunk's primitive quartets
-                    if (lane < nprim)
-                    {
-                        const double4 P = A.bra.pp[bpoff + prim0 + lane];
-                        const double pq = P.x * Q.x, ps = P.x + Q.x;
-                        const double alpha = pq / ps;
-                        const double X_ = P.y - Q.y, Y_ = P.z - Q.z, Z_ = P.w - Q.w;
-                        const double Tb = alpha * (X_ * X_ + Y_ * Y_ + Z_ * Z_);
-                        double F[L + 1];
-                        boysF<L>(Tb, A.boys, F);
-                        double sc = kTwoPi52 / (pq * sqrt(ps));
-#pragma unroll
-                        for (int m = 0; m <= L; m++)
-                        {
-                            sInit[lane][m] = F[m] * sc;
-                            sc *= -2.0 * alpha;
-                        }
-                        sPQ[lane][0] = T(X_);
-                        sPQ[lane][1] = T(Y_);
-                        sPQ[lane][2] = T(Z_);
-                        sR[L & 1][lane][0] = T(sInit[lane][L]);
-                    }
-                    __syncthreads();
-                    // levels n = L-1 .. 0, ping-pong buffers
-#pragma unroll
-                    for (int n = L - 1; n >= 0; n--)
-                    {
-                        const int nh = nHerm(L - n) - 1;
-                        const T(*in)[HL] = sR[(n + 1) & 1];
-                        T(*out)[HL] = sR[n & 1];
-                        const int items = nprim * nh;
-                        for (int it = lane; it < items; it += 64)
-                        {
-                            const int pr = it / nh;
-                            const int h = it - pr * nh + 1;
-                            const unsigned r = kRecTab.v[h];
-                            const int s1 = r & 2047, s2 = (r >> 11) & 2047, ax = (r >> 22) & 3,
-                                      c = (r >> 24);
-                            out[pr][h] = fma(sPQ[pr][ax], in[pr][s1], T(c) * in[pr][s2]);
-                        }
-                        if (lane < nprim)
-                            out[lane][0] = T(sInit[lane][n]);
-                        __syncthreads();
-                    }
-                    // ket transform on MFMA: acc1[mt][nt] += Rg[rows, k] Ek[k, cols]
-                    const T *ek;
-                    if constexpr (F32)
-                        ek = A.ket.ek32 + static_cast<size_t>(kpoff + k) * HQ * SQ;
-                    else
-                        ek = A.ket.ek + static_cast<size_t>(kpoff + k) * HQ * SQ;
-#pragma unroll
-                    for (int kt = 0; kt < KQ; kt++)
-                    {
-                        const int kk = 4 * kt + g;
-                        T b1[NQ];
-#pragma unroll
-                        for (int nt = 0; nt < NQ; nt++)
-                        {
-                            const int col = 16 * nt + j;
-                            b1[nt] = (kk < HQ && col < SQ) ? ek[kk * SQ + col] : T(0);
-                        }
-#pragma unroll
-                        for (int mt = 0; mt < MT; mt++)
-                        {
-                            if (rowbase + 16 * mt >= nrows)
-                                continue;
-                            const int gr = rowbase + 16 * mt + j;
-                            const int pr = gr / HP;
-                            const int h = gr - pr * HP;
-                            const T a = (pr < bcnt) ? sR[0][pr - prim0][sTab[h][kk]] : T(0);
-#pragma unroll
-                            for (int nt = 0; nt < NQ; nt++)
-                                acc1[mt][nt] = mfma16(a, b1[nt], acc1[mt][nt]);
-                        }
-                    }
-                    __syncthreads();
-                }
-                // bra transform: I^T[kl, mn] += X^T[kl, rows] Eb[rows, mn]
-#pragma unroll
-                for (int mt = 0; mt < MT; mt++)
-                {
-                    if (rowbase + 16 * mt >= nrows)
-                        continue;
-#pragma unroll
-                    for (int c = 0; c < 4; c++)
-                    {
-                        // K-chunk c of X^T = accumulator element c of every lane: rows
-                        // 16 mt + 4 c + (0..3) in FP64 (element c holds row 4 c + g), rows
-                        // 16 mt + c + 4 (0..3) in FP32 (element c holds row 4 g + c)
-                        const int gr = rowbase + 16 * mt + (F32 ? 4 * g + c : 4 * c + g);
-                        const int pr = gr / HP;
-                        const int h = gr - pr * HP;
-                        const bool rv = pr < bcnt;
-                        const T *eb;
-                        if constexpr (F32)
-                            eb = A.bra.eb32 + (static_cast<size_t>(bpoff + pr) * HP + h) * SP;
-                        else
-                            eb = A.bra.eb + (static_cast<size_t>(bpoff + pr) * HP + h) * SP;
-#pragma unroll
-                        for (int np = 0; np < NP; np++)
-                        {
-                            const int col = 16 * np + j;
-                            const T b2 = (rv && col < SP) ? eb[col] : T(0);
-#pragma unroll
-                            for (int nq = 0; nq < NQ; nq++)
-                                acc2[nq][np] = mfma16(acc1[mt][nq][c], b2, acc2[nq][np]);
-                        }
-                    }
-                }
-            }
-            // accumulator element r of lane (g, j) holds D[4 r + g][j] (FP64) or D[4 g + r][j]
-            // (FP32); here D = I^T[16 nq + row][16 np + j]
-#pragma unroll
-            for (int nq = 0; nq < NQ; nq++)
-#pragma unroll
-                for (int np = 0; np < NP; np++)
-#pragma unroll
-                    for (int r = 0; r < 4; r++)
-                    {
-                        const int kl = 16 * nq + (F32 ? 4 * g + r : 4 * r + g), mn = 16 * np + j;
-                        if (kl < SQ && mn < SP)
-                            sI[mn * SQ + kl] = double(acc2[nq][np][r]);
-                    }
-            __syncthreads();
-
-            const int a0 = A.bra.ao_a[ab], b0 = A.bra.ao_b[ab];
-            const int c0 = A.ket.ao_a[cd], d0 = A.ket.ao_b[cd];
-            if constexpr (MODE == MODE_JK)
-            {
-                double f = 1.0;
-                if (A.bra.sh_a[ab] == A.bra.sh_b[ab])
-                    f *= 0.5;
-                if (A.ket.sh_a[cd] == A.ket.sh_b[cd])
-                    f *= 0.5;
-                if (A.same_class && p == q)
-                    f *= 0.5;
-                const long long n = A.nbf;
-                const double *D = A.D;
-                // D blocks: 0 ab, 1 cd, 2 bd, 3 ad, 4 bc, 5 ac
-                for (int e = lane; e < SA * SB; e += 64)
-                    sD[0][e] = D[(a0 + e / SB) * n + b0 + e % SB];
-                for (int e = lane; e < SC * SD; e += 64)
-                    sD[1][e] = D[(c0 + e / SD) * n + d0 + e % SD];
-                for (int e = lane; e < SB * SD; e += 64)
-                    sD[2][e] = D[(b0 + e / SD) * n + d0 + e % SD];
-                for (int e = lane; e < SA * SD; e += 64)
-                    sD[3][e] = D[(a0 + e / SD) * n + d0 + e % SD];
-                for (int e = lane; e < SB * SC; e += 64)
-                    sD[4][e] = D[(b0 + e / SC) * n + c0 + e % SC];
-                for (int e = lane; e < SA * SC; e += 64)
-                    sD[5][e] = D[(a0 + e / SC) * n + c0 + e % SC];
-                __syncthreads();
-                for (int mn = lane; mn < SP; mn += 64)
-                {
-                    double s = 0.0;
-                    for (int kl = 0; kl < SQ; kl++)
-                        s = fma(sI[mn * SQ + kl], sD[1][kl], s);
-                    unsafeAtomicAdd(&A.J[(a0 + mn / SB) * n + b0 + mn % SB], 2.0 * f * s);
-                }
-                for (int kl = lane; kl < SQ; kl += 64)
-                {
-                    double s = 0.0;
-                    for (int mn = 0; mn < SP; mn++)
-                        s = fma(sI[mn * SQ + kl], sD[0][mn], s);
-                    unsafeAtomicAdd(&A.J[(c0 + kl / SD) * n + d0 + kl % SD], 2.0 * f * s);
-                }
-                // K_ac[mu,ka] += f sum_{nu,la} I D_bd[nu,la]
-                for (int e = lane; e < SA * SC; e += 64)
-                {
-                    const int mu = e / SC, ka = e % SC;
-                    double s = 0.0;
-                    for (int nu = 0; nu < SB; nu++)
-                        for (int la = 0; la < SD; la++)
-                            s = fma(sI[(mu * SB + nu) * SQ + ka * SD + la], sD[2][nu * SD + la], s);
-                    unsafeAtomicAdd(&A.K[(c0 + ka) * n + a0 + mu], f * s);
-                }
-                // K_bc[nu,ka] += f sum_{mu,la} I D_ad[mu,la]
-                for (int e = lane; e < SB * SC; e += 64)
-                {
-                    const int nu = e / SC, ka = e % SC;
-                    double s = 0.0;
-                    for (int mu = 0; mu < SA; mu++)
-                        for (int la = 0; la < SD; la++)
-                            s = fma(sI[(mu * SB + nu) * SQ + ka * SD + la], sD[3][mu * SD + la], s);
-                    unsafeAtomicAdd(&A.K[(c0 + ka) * n + b0 + nu], f * s);
-                }
-                // K_ad[mu,la] += f sum_{nu,ka} I D_bc[nu,ka]
-                for (int e = lane; e < SA * SD; e += 64)
-                {
-                    const int mu = e / SD, la = e % SD;
-                    double s = 0.0;
-                    for (int nu = 0; nu < SB; nu++)
-                        for (int ka = 0; ka < SC; ka++)
-                            s = fma(sI[(mu * SB + nu) * SQ + ka * SD + la], sD[4][nu * SC + ka], s);
-                    unsafeAtomicAdd(&A.K[(d0 + la) * n + a0 + mu], f * s);
-                }
-                // K_bd[nu,la] += f sum_{mu,ka} I D_ac[mu,ka]
-                for (int e = lane; e < SB * SD; e += 64)
-                {
-                    const int nu = e / SD, la = e % SD;
-                    double s = 0.0;
-                    for (int mu = 0; mu < SA; mu++)
-                        for (int ka = 0; ka < SC; ka++)
-                            s = fma(sI[(mu * SB + nu) * SQ + ka * SD + la], sD[5][mu * SC + ka], s);
-                    unsafeAtomicAdd(&A.K[(d0 + la) * n + b0 + nu], f * s);
-                }
-            }
-            else if constexpr (MODE == MODE_DENSE)
-            {
-                for (int e = lane; e < SP * SQ; e += 64)
-                    denseStore<C>(A, sI[e], e / SQ, e % SQ, a0, b0, c0, d0);
-            }
-            else if constexpr (MODE == MODE_SUM)
-            {
-                double sa = 0.0, ss = 0.0;
-                for (int e = lane; e < SP * SQ; e += 64)
-                {
-                    sa += fabs(sI[e]);
-                    ss += sI[e];
-                }
-                const bool one = A.kind == 3 ? A.bra.sh_a[ab] == A.bra.sh_b[ab] : (A.same_class && p == q);
-                const double w = one ? 1.0 : 2.0;
-                sa = waveSum(w * sa);
-                ss = waveSum(w * ss);
-                if (lane == 0)
-                {
-                    double *o = A.out + 4 * static_cast<long long>(A.ket.mol[cd]) + (A.kind == 3 ? 0 : 2);
-                    unsafeAtomicAdd(o, sa);
-                    unsafeAtomicAdd(o + 1, ss);
-                }
-            }
-            else
-            {
-                if (lane == 0)
-                {
-                    double m = 0.0;
-                    for (int mn = 0; mn < SP; mn++)
-                        m = fmax(m, fabs(sI[mn * SQ + mn]));
-                    A.qout[ab] = sqrt(m);
-                }
-                if (A.dout)
-                    for (int mn = lane; mn < SP; mn += 64)
-                    {
-                        const int mu = mn / SB, nu = mn % SB;
-                        const double v = sI[mn * SQ + mn];
-                        if (A.kind == 2)
-                            A.dout[a0 + mu] = v;
-                        else
-                        {
-                            A.dout[(a0 + mu) * A.nbf + b0 + nu] = v;
-                            A.dout[(b0 + nu) * A.nbf + a0 + mu] = v;
-                        }
-                    }
-            }
-            __syncthreads();
-        }
+        if constexpr (MODE == MODE_SUM)
+            flushSums(A, mol, lane, jl[0], jl[1]);
     }
 
     template <int LA, int LB, int LC, int LD, int MODE, bool SWAP, typename T>
@@ -1072,38 +746,20 @@ namespace lbx
                 return 8192;
             return std::max(1, per_cu) * std::max(1, ncu);
         }();
-        const long long cap = A.block_major ? std::min(resident, 8192) : 8192;
+        // per-molecule sums: four rounds of them, each wave ending in one addition per molecule
+        const long long cap = A.block_major ? std::min(resident, 8192) : MODE == MODE_SUM ? std::min(4 * resident, 8192) : 8192;
         long long wg = (A.ntasks + 3) / 4;
         int grid = static_cast<int>(wg < cap ? wg : cap);
         hipLaunchKernelGGL((quartetV<LA, LB, LC, LD, MODE, SWAP, T>), dim3(grid), dim3(256), 0, s, A);
     }
 
-    template <int LA, int LB, int LC, int LD, int MODE>
-    void launchMfma(const KArgs &A, hipStream_t s)
-    {
-        if (A.ntasks <= 0)
-            return;
-        int grid = static_cast<int>(A.ntasks < 16384 ? A.ntasks : 16384);
-        hipLaunchKernelGGL((quartetM<LA, LB, LC, LD, MODE>), dim3(grid), dim3(64), 0, s, A);
-    }
-
-    template <int LA, int LB, int LC, int LD>
-    void launchMfma32(const KArgs &A, hipStream_t s)
-    {
-        if (A.ntasks <= 0)
-            return;
-        int grid = static_cast<int>(A.ntasks < 16384 ? A.ntasks : 16384);
-        hipLaunchKernelGGL((quartetM<LA, LB, LC, LD, MODE_JK, float>), dim3(grid), dim3(64), 0, s, A);
-    }
-
-    // The FP32 forms: one lane per quartet (J/K and RI sums), one wave per quartet on the FP32
-    // MFMA (J/K).
+    // The FP32 forms (J/K and RI sums).
     template <int LA, int LB, int LC, int LD, int MODE>
     void registerQuartet32()
     {
         using C = Cls<LA, LB, LC, LD>;
         constexpr bool same = LA == LC && LB == LD;
-        if constexpr ((MODE == MODE_JK || MODE == MODE_SUM) && C::NC0f > 0)
+        if constexpr ((MODE == MODE_JK || MODE == MODE_SUM) && C::kLane0f)
         {
             KernelSlot &s = kernelSlot(MODE, LA, LB, LC, LD, VAR_VALU_BRA32);
             s.fn = &launchValu<LA, LB, LC, LD, MODE, false, float>;
@@ -1111,7 +767,7 @@ namespace lbx
             s.swap = false;
             s.nc = C::NC0f;
         }
-        if constexpr (MODE == MODE_JK && C::NC1f > 0 && !same)
+        if constexpr (MODE == MODE_JK && C::kLane1f && !same)
         {
             KernelSlot &s = kernelSlot(MODE, LA, LB, LC, LD, VAR_VALU_KET32);
             s.fn = &launchValu<LA, LB, LC, LD, MODE, true, float>;
@@ -1119,19 +775,11 @@ namespace lbx
             s.swap = true;
             s.nc = C::NC1f;
         }
-        if constexpr (MODE == MODE_JK)
-        {
-            KernelSlot &s = kernelSlot(MODE, LA, LB, LC, LD, VAR_MFMA32);
-            s.fn = &launchMfma32<LA, LB, LC, LD>;
-            s.width = 1;
-            s.swap = false;
-            s.kind = KIND_WAVE;
-        }
     }
 
-    // Registers every variant the class supports in this mode.  The ket-on-lanes VALU form
+    // Registers the one-lane variants the class supports in this mode.  The ket-on-lanes form
     // only serves J/K between different classes (dense and diagonal outputs keep the bra on
-    // the lanes; for one class both forms coincide).  The MFMA form is always available.
+    // the lanes; for one class both forms coincide).
     // FORMS: 1 the FP64 forms, 2 the FP32 forms, 3 both (lets the build compile them apart).
     template <int LA, int LB, int LC, int LD, int MODE, int FORMS = 3>
     void registerQuartet()
@@ -1141,7 +789,7 @@ namespace lbx
             registerQuartet32<LA, LB, LC, LD, MODE>();
         if constexpr (!(FORMS & 1))
             return;
-        if constexpr (C::NC0 > 0)
+        if constexpr (C::kLane0)
         {
             KernelSlot &s = kernelSlot(MODE, LA, LB, LC, LD, VAR_VALU_BRA);
             s.fn = &launchValu<LA, LB, LC, LD, MODE, false, double>;
@@ -1150,7 +798,7 @@ namespace lbx
             s.nc = C::NC0;
         }
         constexpr bool same = LA == LC && LB == LD;
-        if constexpr (MODE == MODE_JK && C::NC1 > 0 && !same)
+        if constexpr (MODE == MODE_JK && C::kLane1 && !same)
         {
             KernelSlot &s = kernelSlot(MODE, LA, LB, LC, LD, VAR_VALU_KET);
             s.fn = &launchValu<LA, LB, LC, LD, MODE, true, double>;
@@ -1158,10 +806,5 @@ namespace lbx
             s.swap = true;
             s.nc = C::NC1;
         }
-        KernelSlot &s = kernelSlot(MODE, LA, LB, LC, LD, VAR_MFMA);
-        s.fn = &launchMfma<LA, LB, LC, LD, MODE>;
-        s.width = 1;
-        s.swap = false;
-        s.kind = KIND_WAVE;
     }
 }

@@ -13,9 +13,8 @@
 //
 // Phases of a task, per bra primitive i:
 //   R + X  wave w takes ket pairs w, w + 4, ...; per chunk of up to PB ket primitives: Boys
-//          function and R^(n)_000 (one lane per primitive quartet), the Hermite recursion level
-//          by level in the wave's LDS buffers (lanes over (primitive, tuv)), then the ket
-//          transform with one lane per row tuv of X, the ket's E matrix through scalar loads
+//          function, R^(n)_000 and the Hermite recursion in the wave's LDS (hermite_lds.hpp), then
+//          the ket transform with one lane per row tuv of X, the ket's E matrix through scalar loads
 //          (wave-uniform), X held in registers and written to the shared LDS buffer.
 //   I      the four waves split the 16x16 tiles of I; A operand Eb_i from global memory (L2),
 //          B operand X from LDS; accumulators stay in registers across i.
@@ -25,7 +24,7 @@
 // the workgroup synchronises only around the MFMA phase and the epilogue.
 #pragma once
 
-#include "quartet.hpp"
+#include "quartet_wave.hpp"
 
 namespace lbx
 {
@@ -34,7 +33,6 @@ namespace lbx
     {
         static constexpr int L = LA + LB + LC + LD;
         static constexpr int HA = nHerm(LA + LB), HB = nHerm(LC + LD), HL = nHerm(L);
-        static constexpr int H1 = L >= 1 ? nHerm(L - 1) : 1;   // entries of recursion level 1
         static constexpr int SAa = nSph(LA), SAb = nSph(LB), SBc = nSph(LC), SBd = nSph(LD);
         static constexpr int SA = SAa * SAb, SB = SBc * SBd;
         static constexpr int NB = SB >= 48 ? 1 : 48 / SB;      // ket pairs per task
@@ -44,8 +42,8 @@ namespace lbx
         static constexpr int XS = 16 * NT + 1;                 // row stride of X (padded)
         static constexpr int XR = 4 * KT;                      // rows of X (zero from HA on)
         static constexpr int RP = ceilDiv(HA, 64);             // rows of X per lane
-        // ket primitives per recursion chunk: about 8 KiB of level buffers per wave
-        static constexpr int PB0 = 8192 / ((HL + H1) * static_cast<int>(sizeof(T)));
+        // ket primitives per recursion chunk: about 8 KiB of R per wave
+        static constexpr int PB0 = 8192 / (HL * static_cast<int>(sizeof(T)));
         static constexpr int PB = PB0 < 1 ? 1 : (PB0 > 16 ? 16 : PB0);
         static constexpr int CW = SB < 16 ? SB : 16;           // X columns per register pass
         static constexpr bool kRegIdx = HB <= 20;              // gather indices in registers
@@ -61,20 +59,11 @@ namespace lbx
         return hermIdx(t, u, v);
     }
 
-    // LDS ordering inside one wave: a wave's LDS operations execute in issue order, so only the
-    // compiler has to be kept from moving loads and stores across this point.
-    __device__ __forceinline__ void waveFence()
-    {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
-
     template <int LA, int LB, int LC, int LD, typename T>
     __global__ __launch_bounds__(256) void quartetB(const KArgs A)
     {
         using P = BlockPlan<LA, LB, LC, LD, T>;
-        constexpr int L = P::L, HA = P::HA, HB = P::HB, HL = P::HL, H1 = P::H1;
+        constexpr int L = P::L, HA = P::HA, HB = P::HB, HL = P::HL;
         constexpr int SA = P::SA, SB = P::SB, SAa = P::SAa, SAb = P::SAb, SBc = P::SBc, SBd = P::SBd;
         constexpr int NB = P::NB, NCOL = P::NCOL, NT = P::NT, KT = P::KT, NTILE = P::NTILE;
         constexpr int TPW = P::TPW, XS = P::XS, XR = P::XR, RP = P::RP, PB = P::PB, CW = P::CW;
@@ -82,10 +71,9 @@ namespace lbx
         using Acc = std::conditional_t<F32, v4f, v4d>;
 
         __shared__ T sX[XR * XS];               // X (rows tuv, columns (j, kl)); I in the epilogue
-        __shared__ T sRe[4][PB * HL];           // recursion buffers per wave: even levels
-        __shared__ T sRo[4][PB * H1];           // odd levels
-        __shared__ double sInit[4][PB][L + 1];  // R^(n)_000 of the chunk's primitive quartets
-        __shared__ T sPQ[4][PB][3];
+        __shared__ T sR[4][PB * HL];            // R of the chunk's primitive quartets, per wave
+        __shared__ T sInit[4][PB * (L + 1)];    // their R^(n)_000
+        __shared__ T sPQ[4][4 * PB];
         __shared__ unsigned short sTab[P::kRegIdx ? 1 : HB * HA];   // gather index [t'u'v'][tuv]
         __shared__ int sKet[NB][5];             // ket pair: pair index, first prim, prims, AO c, AO d
         __shared__ double sF[NB];               // permutational weight of each quartet
@@ -96,6 +84,8 @@ namespace lbx
         const long long n = A.nbf;
         const double *__restrict__ D = A.D;
 
+        RecLane<L> rec;
+        rec.load(lane);
         for (int e = tid; e < XR * XS; e += 256)
             sX[e] = T(0);
         if constexpr (!P::kRegIdx)
@@ -159,7 +149,6 @@ namespace lbx
 
             for (int i = 0; i < bcnt; i++)
             {
-                const double4 Pa = A.bra.pp[bpoff + i];
                 // ---- Hermite integrals and ket transforms: wave w takes ket pairs w, w + 4, ...
                 for (int jj = w; jj < NB; jj += 4)
                 {
@@ -176,57 +165,12 @@ namespace lbx
                         ekb = A.ket.ek32;
                     else
                         ekb = A.ket.ek;
-                    T *const bufE = sRe[w];
-                    T *const bufO = sRo[w];
                     for (int k0 = 0; k0 < kcnt; k0 += PB)
                     {
                         const int np = min(PB, kcnt - k0);
-                        if (lane < np)
-                        {
-                            const double4 Q = A.ket.pp[kpoff + k0 + lane];
-                            const double pq = Pa.x * Q.x, ps = Pa.x + Q.x;
-                            const double alpha = pq / ps;
-                            const double X_ = Pa.y - Q.y, Y_ = Pa.z - Q.z, Z_ = Pa.w - Q.w;
-                            double F[L + 1];
-                            boysF<L>(alpha * (X_ * X_ + Y_ * Y_ + Z_ * Z_), A.boys, F);
-                            double sc = kTwoPi52 / (pq * sqrt(ps));
-#pragma unroll
-                            for (int m = 0; m <= L; m++)
-                            {
-                                sInit[w][lane][m] = F[m] * sc;
-                                sc *= -2.0 * alpha;
-                            }
-                            sPQ[w][lane][0] = T(X_);
-                            sPQ[w][lane][1] = T(Y_);
-                            sPQ[w][lane][2] = T(Z_);
-                            if constexpr (L & 1)
-                                bufO[lane * H1] = T(sInit[w][lane][L]);
-                            else
-                                bufE[lane * HL] = T(sInit[w][lane][L]);
-                        }
                         waveFence();
-                        // levels L-1 .. 0: level n holds R^(n)_tuv for |tuv| <= L - n
-#pragma unroll
-                        for (int lev = L - 1; lev >= 0; lev--)
-                        {
-                            const T *in = ((lev + 1) & 1) ? bufO : bufE;
-                            T *out = (lev & 1) ? bufO : bufE;
-                            const int si = ((lev + 1) & 1) ? H1 : HL, so = (lev & 1) ? H1 : HL;
-                            const int nh = nHerm(L - lev) - 1;
-                            const int items = np * nh;
-                            for (int it = lane; it < items; it += 64)
-                            {
-                                const int p = it / nh;
-                                const int h = it - p * nh + 1;
-                                const unsigned r = kRecTab.v[h];
-                                const int s1 = r & 2047, s2 = (r >> 11) & 2047, ax = (r >> 22) & 3,
-                                          c = static_cast<int>(r >> 24);
-                                out[p * so + h] = fma(sPQ[w][p][ax], in[p * si + s1], T(c) * in[p * si + s2]);
-                            }
-                            if (lane < np)
-                                out[lane * so] = T(sInit[w][lane][lev]);
-                            waveFence();
-                        }
+                        hermiteBatch<L, T>(sR[w], sInit[w], sPQ[w], rec, np, lane, A.bra.pp + bpoff + i,
+                                           A.ket.pp + kpoff + k0 + lane, A.boys);
                         // ket transform: X[h][(jj, kl)] += sum_p sum_g R_p[h + g] Ek_p[g][kl]
 #pragma unroll
                         for (int r = 0; r < RP; r++)
@@ -245,7 +189,7 @@ namespace lbx
                                     {
                                         const cptr<T> e =
                                                 constView(ekb + static_cast<size_t>(kpoff + k0 + p) * HB * SB);
-                                        const T *rr = bufE + p * HL;
+                                        const T *rr = sR[w] + p * HL;
 #pragma unroll
                                         for (int g = 0; g < HB; g++)
                                         {
