@@ -43,6 +43,40 @@ namespace lbx
             DevBuf &operator=(const DevBuf &) = delete;
         };
 
+        // The extra streams of a context (default priority) and the events that tie them to its
+        // stream; made on first use.
+        struct SideStreams
+        {
+            static constexpr int kCount = 3;
+            hipStream_t s[kCount] = {};
+            hipEvent_t fork = nullptr, joined[kCount] = {};
+
+            void ensure()
+            {
+                for (int i = 0; i < kCount; i++)
+                {
+                    if (!s[i])
+                        LBX_HIP(hipStreamCreateWithFlags(&s[i], hipStreamNonBlocking));
+                    if (!joined[i])
+                        LBX_HIP(hipEventCreateWithFlags(&joined[i], hipEventDisableTiming));
+                }
+                if (!fork)
+                    LBX_HIP(hipEventCreateWithFlags(&fork, hipEventDisableTiming));
+            }
+            ~SideStreams()
+            {
+                for (int i = 0; i < kCount; i++)
+                {
+                    if (s[i])
+                        (void)hipStreamDestroy(s[i]);
+                    if (joined[i])
+                        (void)hipEventDestroy(joined[i]);
+                }
+                if (fork)
+                    (void)hipEventDestroy(fork);
+            }
+        };
+
         template <class F>
         int guarded(F &&f)
         {
@@ -262,9 +296,9 @@ namespace lbx
             }
             t.prefix[t.nket] = acc;
             t.ntasks = acc;
-            t.d_prefix = c.upload(t.prefix);
-            t.d_plo = c.upload(t.plo);
-            t.d_phi = c.upload(t.phi);
+            t.d_prefix = c.stage(t.prefix);
+            t.d_plo = c.stage(t.plo);
+            t.d_phi = c.stage(t.phi);
             return t;
         }
 
@@ -297,8 +331,8 @@ namespace lbx
             t.bprefix = std::move(b.bprefix);
             t.bq0 = std::move(b.bq0);
             t.btasks = b.ntasks;
-            t.d_bprefix = c.upload(t.bprefix);
-            t.d_bq0 = c.upload(t.bq0);
+            t.d_bprefix = c.stage(t.bprefix);
+            t.d_bq0 = c.stage(t.bq0);
             return b.quartets;
         }
 
@@ -307,7 +341,8 @@ namespace lbx
         // positions p >= q, and with bounds (both sides sorted by Q within each molecule) only
         // those with lo <= Q_p Q_q < hi.  No screening below: every triplet of the tensors.
         TaskTable buildTasksMol(Context &c, const PairClass &lane, const PairClass &unif, bool same,
-                                int width, double lo_bound = 0.0, double hi_bound = kNoUpper)
+                                int width, double lo_bound = 0.0, double hi_bound = kNoUpper,
+                                bool staged = true)
         {
             const bool bounded = lo_bound > 0.0 || hi_bound < kNoUpper;
             auto qOf = [](const PairClass &pc, int pos) { return pc.Q.empty() ? 1.0 : pc.Q[pc.order[pos]]; };
@@ -376,9 +411,10 @@ namespace lbx
             }
             t.prefix[t.nket] = acc;
             t.ntasks = acc;
-            t.d_prefix = c.upload(t.prefix);
-            t.d_plo = c.upload(t.plo);
-            t.d_phi = c.upload(t.phi);
+            // staged arrays stay with the context, uploaded ones can be freed one by one
+            t.d_prefix = staged ? c.stage(t.prefix) : c.upload(t.prefix);
+            t.d_plo = staged ? c.stage(t.plo) : c.upload(t.plo);
+            t.d_phi = staged ? c.stage(t.phi) : c.upload(t.phi);
             return t;
         }
 
@@ -551,35 +587,101 @@ namespace lbx
             return s;
         }
 
-        void run(Context &c, int mode, const PairClass &bra, const PairClass &ket, Pairing pairing,
-                 bool same, double thresh, KArgs extra)
+        // One launch of an unscreened driver: every (bra, ket) pair combination of a class pair
+        struct PlainJob
         {
-            if (bra.n_pairs == 0 || ket.n_pairs == 0)
-                return;
-            const KernelSlot &s = slotFor(mode, bra, ket, defaultVariant(mode, bra, ket));
-            TaskTable t = buildTasks(c, bra, ket, pairing, same, thresh, s.width);
-            KArgs a = baseArgs(c, bra, ket, t, same);
-            a.D = extra.D;
-            a.J = extra.J;
-            a.K = extra.K;
-            a.out = extra.out;
-            a.kind = extra.kind;
-            a.qout = extra.qout;
-            a.dout = extra.dout;
-            s.fn(a, c.stream);
-            LBX_HIP(hipGetLastError());
-            LBX_HIP(hipStreamSynchronize(c.stream));
-            // the task table's device arrays were allocated from the context; free them now
-            for (void *p : {static_cast<void *>(t.d_prefix), static_cast<void *>(t.d_plo),
-                            static_cast<void *>(t.d_phi)})
+            int mode;
+            const PairClass *bra, *ket;
+            Pairing pairing;
+            bool same;
+            KArgs extra;
+        };
+
+        // One kernel of a call whose kernels are independent
+        struct QueuedLaunch
+        {
+            Launcher fn;
+            KArgs a;
+            double cost;   // relative estimate of its time
+        };
+
+        // streams beside the context's that share the launches of one call (a process has four
+        // hardware queues)
+        constexpr int kSideStreams = SideStreams::kCount;
+
+        // The independent launches of one call, spread over the context's stream and its side
+        // streams: the side streams start after what the context's stream holds at construction
+        // (fork event) and join() makes the context's stream wait for them.  Off (on = false):
+        // everything on the context's stream.
+        class Fan
+        {
+        public:
+            Fan(SideStreams &side, hipStream_t main, bool on) : side_(side), main_(main), on_(on)
             {
-                auto it = std::find(c.allocations.begin(), c.allocations.end(), p);
-                if (it != c.allocations.end())
-                {
-                    (void)hipFree(p);
-                    c.allocations.erase(it);
-                }
+                if (!on_)
+                    return;
+                side_.ensure();
+                LBX_HIP(hipEventRecord(side_.fork, main_));
             }
+            ~Fan()
+            {
+                // after an exception: still bring the side streams back to the context's stream
+                for (int i = 0; i < kSideStreams; i++)
+                    if (used_[i] && hipEventRecord(side_.joined[i], side_.s[i]) == hipSuccess)
+                        (void)hipStreamWaitEvent(main_, side_.joined[i], 0);
+            }
+            Fan(const Fan &) = delete;
+            Fan &operator=(const Fan &) = delete;
+
+            // the least loaded stream
+            hipStream_t pick(double cost)
+            {
+                int b = 0;
+                if (on_)
+                    for (int i = 1; i <= kSideStreams; i++)
+                        if (load_[i] < load_[b])
+                            b = i;
+                load_[b] += cost;
+                if (b == 0)
+                    return main_;
+                if (!used_[b - 1])
+                {
+                    LBX_HIP(hipStreamWaitEvent(side_.s[b - 1], side_.fork, 0));
+                    used_[b - 1] = true;
+                }
+                return side_.s[b - 1];
+            }
+
+            void join()
+            {
+                for (int i = 0; i < kSideStreams; i++)
+                    if (used_[i])
+                    {
+                        LBX_HIP(hipEventRecord(side_.joined[i], side_.s[i]));
+                        LBX_HIP(hipStreamWaitEvent(main_, side_.joined[i], 0));
+                        used_[i] = false;
+                    }
+            }
+
+        private:
+            SideStreams &side_;
+            hipStream_t main_;
+            bool on_;
+            double load_[kSideStreams + 1] = {};
+            bool used_[kSideStreams] = {};
+        };
+
+        // Launches the queue, most expensive first, over the fan's streams.
+        void launchAll(std::vector<QueuedLaunch> &queue, Fan &fan)
+        {
+            std::stable_sort(queue.begin(), queue.end(),
+                             [](const QueuedLaunch &x, const QueuedLaunch &y) { return x.cost > y.cost; });
+            for (auto &l : queue)
+            {
+                l.fn(l.a, fan.pick(l.cost));
+                LBX_HIP(hipGetLastError());
+            }
+            fan.join();
         }
     }
 
@@ -611,19 +713,14 @@ namespace lbx
                t.sum_kbra * 9 * 2 * Sab * Hab * Scd + t.quartets * 72 * Sab * Scd;
     }
 
-    // Schwarz factors Q_ab = sqrt(max |(ab|ab)|) per pair of every main class; pairs sorted by
-    // descending Q so that each ket's surviving bra pairs form a prefix.
-    // Schwarz factors Q = sqrt(max |(ab|ab)|) of one class (kind 4: pairs, kind 2: single
-    // auxiliary shells) and the sorted order: by molecule, then Q descending (one molecule in an
-    // ordinary context), so each molecule's pairs keep their contiguous range of positions.
-    void sortByBound(Context &c, PairClass &pc, int kind)
+    // Schwarz factors Q = sqrt(max |(ab|ab)|) of a class (computed on the device into d_q, pair
+    // order) and the sorted order: by molecule, then Q descending (one molecule in an ordinary
+    // context), so that each ket's surviving bra pairs form a prefix and each molecule's pairs
+    // keep their contiguous range of positions.
+    void sortByBound(PairClass &pc)
     {
         if (pc.n_pairs == 0)
             return;
-        KArgs extra{};
-        extra.qout = pc.d_q;
-        extra.kind = kind;
-        run(c, MODE_DIAG, pc, pc, Pairing::Diagonal, true, 0.0, extra);
         pc.Q.resize(pc.n_pairs);
         LBX_HIP(hipMemcpy(pc.Q.data(), pc.d_q, pc.n_pairs * sizeof(double), hipMemcpyDeviceToHost));
         std::vector<int> order(pc.n_pairs);
@@ -647,25 +744,6 @@ namespace lbx
         LBX_HIP(hipMemcpy(pc.d_order, order.data(), order.size() * sizeof(int), hipMemcpyHostToDevice));
         LBX_HIP(hipMemcpy(pc.d_q, qs.data(), qs.size() * sizeof(double), hipMemcpyHostToDevice));
     }
-
-    void ensureSchwarz(Context &c)
-    {
-        if (c.have_schwarz)
-            return;
-        for (auto &pc : c.cls)
-            sortByBound(c, pc, 4);
-        c.have_schwarz = true;
-    }
-
-    // the same for the auxiliary shells (bounds of the RI sums' precision split)
-    void ensureSchwarzAux(Context &c)
-    {
-        if (c.have_schwarz_aux)
-            return;
-        for (auto &pc : c.aux)
-            sortByBound(c, pc, 2);
-        c.have_schwarz_aux = true;
-    }
 }
 
 using namespace lbx;
@@ -686,6 +764,71 @@ struct lbx_context : Context
     bool graphs = false;
     // lbx_set_bound_window: lbx_jk evaluates only quartets with window_lo <= Q_ab Q_cd < window_hi
     double window_lo = 0.0, window_hi = kNoUpper;
+    SideStreams side;
+    // task tables of the unscreened drivers per (lane class, uniform class, pairing, same, width)
+    std::map<std::tuple<const PairClass *, const PairClass *, int, bool, int>, TaskTable> plain_tasks;
+
+    // Runs the jobs (independent of each other) over the context's streams and waits for them.
+    void runPlain(const std::vector<PlainJob> &jobs)
+    {
+        std::vector<QueuedLaunch> queue;
+        for (const PlainJob &job : jobs)
+        {
+            const PairClass &bra = *job.bra, &ket = *job.ket;
+            if (bra.n_pairs == 0 || ket.n_pairs == 0)
+                continue;
+            const KernelSlot &s = slotFor(job.mode, bra, ket, defaultVariant(job.mode, bra, ket));
+            const auto key = std::make_tuple(&bra, &ket, static_cast<int>(job.pairing), job.same, s.width);
+            auto it = plain_tasks.find(key);
+            if (it == plain_tasks.end())
+                it = plain_tasks.emplace(key, buildTasks(*this, bra, ket, job.pairing, job.same, 0.0, s.width)).first;
+            KArgs a = baseArgs(*this, bra, ket, it->second, job.same);
+            a.out = job.extra.out;
+            a.kind = job.extra.kind;
+            a.qout = job.extra.qout;
+            a.dout = job.extra.dout;
+            queue.push_back({s.fn, a, it->second.flops});
+        }
+        flushStaged();
+        Fan fan(side, stream, queue.size() > 1);
+        launchAll(queue, fan);
+        LBX_HIP(hipStreamSynchronize(stream));
+    }
+
+    // Schwarz factors and sorted order of every main class (kind 4: pairs) or auxiliary class
+    // (kind 2: single shells)
+    void sortAll(std::vector<PairClass> &classes, int kind)
+    {
+        std::vector<PlainJob> jobs;
+        for (auto &pc : classes)
+        {
+            KArgs extra{};
+            extra.qout = pc.d_q;
+            extra.kind = kind;
+            jobs.push_back({MODE_DIAG, &pc, &pc, Pairing::Diagonal, true, extra});
+        }
+        runPlain(jobs);
+        for (auto &pc : classes)
+            sortByBound(pc);
+    }
+
+    void ensureSchwarz()
+    {
+        if (have_schwarz)
+            return;
+        sortAll(cls, 4);
+        have_schwarz = true;
+    }
+
+    // the same for the auxiliary shells (bounds of the RI sums' precision split)
+    void ensureSchwarzAux()
+    {
+        if (have_schwarz_aux)
+            return;
+        sortAll(aux, 2);
+        have_schwarz_aux = true;
+    }
+
     // lbx_eri*_batch: (shell a, shell b) -> pair index per main pair class
     std::vector<std::unordered_map<long long, int>> pair_maps;
     // their task list on the device (1 MiB, made on first use; every call waits for its kernel)
@@ -742,17 +885,24 @@ struct lbx_context : Context
         std::vector<int> perm = std::move(lo.perm);
         lp.bqlo = std::move(lo.bqlo);
         lp.bqhi = std::move(lo.bqhi);
-        lp.d_perm = upload(perm);
-        lp.d_bqlo = upload(lp.bqlo);
-        lp.d_bqhi = upload(lp.bqhi);
+        lp.d_perm = stage(perm);
+        lp.d_bqlo = stage(lp.bqlo);
+        lp.d_bqhi = stage(lp.bqhi);
         lp.perm = std::move(perm);
         return lane_perm.emplace(idx, std::move(lp)).first->second;
     }
 
-    // Queues the J/K kernel of class pair (i >= j) with the given variant on the context stream,
-    // over the quartets with lo <= Q_ab Q_cd < hi.
-    const TaskTable &launchJK(int i, int j, int var, const double *D, double *J, double *K,
-                              double thresh, double thresh_hi = kNoUpper)
+    // The J/K kernel of class pair (i >= j) with the given variant, its arguments over the
+    // quartets with lo <= Q_ab Q_cd < hi (staged tables: flushStaged() before the launch) and its
+    // task table.
+    struct JKLaunch
+    {
+        Launcher fn;
+        KArgs a;
+        const TaskTable *t;
+    };
+    JKLaunch prepareJK(int i, int j, int var, const double *D, double *J, double *K,
+                       double thresh, double thresh_hi = kNoUpper)
     {
         const PairClass &bra = cls[i], &ket = cls[j];
         const KernelSlot &s = slotFor(MODE_JK, bra, ket, var);
@@ -855,9 +1005,9 @@ struct lbx_context : Context
                 }
                 ts.prefix[t.nket] = acc;
                 ts.ntasks = acc;
-                ts.d_prefix = upload(ts.prefix);
-                ts.d_plo = upload(ts.plo);
-                ts.d_phi = upload(ts.phi);
+                ts.d_prefix = stage(ts.prefix);
+                ts.d_plo = stage(ts.plo);
+                ts.d_phi = stage(ts.phi);
                 st = tune_tasks.emplace(key, std::move(ts)).first;
             }
             const TaskTable &ts = st->second;
@@ -867,9 +1017,16 @@ struct lbx_context : Context
             a.ntasks = ts.ntasks;
             sampled = ts.quartets;
         }
-        s.fn(a, stream);
+        return {s.fn, a, &t};
+    }
+
+    // Queues it on the context stream.
+    void launchJK(int i, int j, int var, const double *D, double *J, double *K, double thresh)
+    {
+        const JKLaunch l = prepareJK(i, j, var, D, J, K, thresh);
+        flushStaged();
+        l.fn(l.a, stream);
         LBX_HIP(hipGetLastError());
-        return t;
     }
 
     // when > 0, launchJK runs only a sample of ~sample_quartets quartets (autotuner timing) and
@@ -903,8 +1060,8 @@ struct lbx_context : Context
     // (aux l | aux l' <= l) class pair, with task tables built once per precision split (device
     // memory cannot be allocated while a stream is being captured).  split > 0: the triplets and
     // doublets with bound Q_ab Q_P below it in the FP32 form where the class has one.
-    std::vector<std::pair<Launcher, KArgs>> ri_launches;
-    std::map<double, std::vector<std::pair<Launcher, KArgs>>> ri_prepared;
+    std::vector<QueuedLaunch> ri_launches;
+    std::map<double, std::vector<QueuedLaunch>> ri_prepared;
     std::map<double, std::array<double, 5>> ri_counts;   // triplets, doublets, flops, FP32 ones
     // FP64 variant of each RI class pair chosen by lbx_tune on a batched context, keyed by
     // (kind, lane class, uniform class): kind 3 (main pair class | aux l), 2 (aux l | aux l')
@@ -937,7 +1094,7 @@ struct lbx_context : Context
                 const KernelSlot &k = kernelSlot(MODE_SUM, lane.la, lane.lb, unif.la, unif.lb, v);
                 if (!k.fn)
                     continue;
-                TaskTable t = buildTasksMol(*this, lane, unif, same, k.width);
+                TaskTable t = buildTasksMol(*this, lane, unif, same, k.width, 0.0, kNoUpper, false);
                 KArgs a = baseArgs(*this, lane, unif, t, same);
                 a.kind = kind;
                 a.out = scratch.p;
@@ -997,7 +1154,7 @@ struct lbx_context : Context
         auto it = ri_prepared.find(split);
         if (it == ri_prepared.end())
         {
-            std::vector<std::pair<Launcher, KArgs>> launches;
+            std::vector<QueuedLaunch> launches;
             std::array<double, 5> n{0, 0, 0, 0, 0};
             auto add = [&](const PairClass &lane, const PairClass &unif, bool same, int kind, int il, int iu)
             {
@@ -1012,7 +1169,7 @@ struct lbx_context : Context
                     TaskTable t = buildTasksMol(*this, lane, unif, same, k.width, lo, hi);
                     KArgs a = baseArgs(*this, lane, unif, t, same);
                     a.kind = kind;
-                    launches.emplace_back(k.fn, a);
+                    launches.push_back({k.fn, a, t.flops});
                     n[kind == 3 ? 0 : 1] += t.quartets;
                     n[2] += t.flops;
                     if (fp32)
@@ -1032,6 +1189,7 @@ struct lbx_context : Context
             for (int la = 0; la < static_cast<int>(aux.size()); la++)
                 for (int lc = 0; lc <= la; lc++)
                     add(aux[la], aux[lc], la == lc, 2, la, lc);
+            flushStaged();
             it = ri_prepared.emplace(split, std::move(launches)).first;
             ri_counts[split] = n;
         }
@@ -1048,13 +1206,11 @@ struct lbx_context : Context
     void queueRiSums(double *out, hipStream_t s)
     {
         fill(out, 4LL * nmol, 0.0, s);
-        for (auto &l : ri_launches)
-        {
-            KArgs a = l.second;
-            a.out = out;
-            l.first(a, s);
-            LBX_HIP(hipGetLastError());
-        }
+        std::vector<QueuedLaunch> queue = ri_launches;
+        for (auto &l : queue)
+            l.a.out = out;
+        Fan fan(side, s, queue.size() > 1);
+        launchAll(queue, fan);
     }
 
     // Queues the gradient kernel of class pair (i >= j) over the quartets with
@@ -1089,6 +1245,7 @@ struct lbx_context : Context
         a.D = D;
         a.nbf = static_cast<long long>(nbf);
         a.grad = grad;
+        flushStaged();
         (fp32 ? s.fn32 : s.fn)(a, stream);
         LBX_HIP(hipGetLastError());
         return t;
@@ -1412,9 +1569,11 @@ extern "C"
                            KArgs extra{};
                            extra.out = out;
                            extra.kind = 4;
+                           std::vector<PlainJob> jobs;
                            for (size_t i = 0; i < c.cls.size(); i++)
                                for (size_t j = 0; j <= i; j++)
-                                   run(c, MODE_DENSE, c.cls[i], c.cls[j], Pairing::Unique, i == j, 0.0, extra);
+                                   jobs.push_back({MODE_DENSE, &c.cls[i], &c.cls[j], Pairing::Unique, i == j, extra});
+                           ctx->runPlain(jobs);
                        });
     }
 
@@ -1429,17 +1588,22 @@ extern "C"
                            requireSingle(c, "lbx_eri4_diag");
                            const long long n = static_cast<long long>(c.nbf);
                            fill(out, n * n, 0.0, c.stream);
+                           size_t pairs = 0;
+                           for (auto &pc : c.cls)
+                               pairs += pc.n_pairs;
+                           DevBuf q(pairs);
+                           std::vector<PlainJob> jobs;
+                           pairs = 0;
                            for (auto &pc : c.cls)
                            {
-                               if (pc.n_pairs == 0)
-                                   continue;
-                               DevBuf q(pc.n_pairs);
                                KArgs extra{};
-                               extra.qout = q.p;
+                               extra.qout = q.p + pairs;
                                extra.dout = out;
                                extra.kind = 4;
-                               run(c, MODE_DIAG, pc, pc, Pairing::Diagonal, true, 0.0, extra);
+                               jobs.push_back({MODE_DIAG, &pc, &pc, Pairing::Diagonal, true, extra});
+                               pairs += pc.n_pairs;
                            }
+                           ctx->runPlain(jobs);
                        });
     }
 
@@ -1459,9 +1623,11 @@ extern "C"
                            KArgs extra{};
                            extra.out = out;
                            extra.kind = 3;
+                           std::vector<PlainJob> jobs;
                            for (auto &bra : c.cls)
                                for (auto &ket : c.aux)
-                                   run(c, MODE_DENSE, bra, ket, Pairing::All, false, 0.0, extra);
+                                   jobs.push_back({MODE_DENSE, &bra, &ket, Pairing::All, false, extra});
+                           ctx->runPlain(jobs);
                        });
     }
 
@@ -1481,9 +1647,11 @@ extern "C"
                            KArgs extra{};
                            extra.out = out;
                            extra.kind = 2;
+                           std::vector<PlainJob> jobs;
                            for (size_t i = 0; i < c.aux.size(); i++)
                                for (size_t j = 0; j <= i; j++)
-                                   run(c, MODE_DENSE, c.aux[i], c.aux[j], Pairing::Unique, i == j, 0.0, extra);
+                                   jobs.push_back({MODE_DENSE, &c.aux[i], &c.aux[j], Pairing::Unique, i == j, extra});
+                           ctx->runPlain(jobs);
                        });
     }
 
@@ -1499,17 +1667,22 @@ extern "C"
                            if (c.shells_aux.empty())
                                throw Error(LBX_ERR_STATE, "eri2Diagonal(): RI approximation is not enabled");
                            fill(out, static_cast<long long>(c.nbf_aux), 0.0, c.stream);
+                           size_t pairs = 0;
+                           for (auto &pc : c.aux)
+                               pairs += pc.n_pairs;
+                           DevBuf q(pairs);
+                           std::vector<PlainJob> jobs;
+                           pairs = 0;
                            for (auto &pc : c.aux)
                            {
-                               if (pc.n_pairs == 0)
-                                   continue;
-                               DevBuf q(pc.n_pairs);
                                KArgs extra{};
-                               extra.qout = q.p;
+                               extra.qout = q.p + pairs;
                                extra.dout = out;
                                extra.kind = 2;
-                               run(c, MODE_DIAG, pc, pc, Pairing::Diagonal, true, 0.0, extra);
+                               jobs.push_back({MODE_DIAG, &pc, &pc, Pairing::Diagonal, true, extra});
+                               pairs += pc.n_pairs;
                            }
+                           ctx->runPlain(jobs);
                        });
     }
 
@@ -1912,38 +2085,42 @@ extern "C"
         fill(J, n * n, 0.0, c.stream);
         fill(K, n * n, 0.0, c.stream);
         lbx_jk_stats st{};
+        std::vector<QueuedLaunch> queue;
         auto launch = [&](int i, int j, int tier, int var, double lo, double hi)
         {
             const PairClass &bra = c.cls[i], &ket = c.cls[j];
-            Prof *pr = nullptr;
-            if (prof_on)
-            {
-                pr = &prof[{i, j, tier}];
-                if (!pr->start)
-                {
-                    LBX_HIP(hipEventCreate(&pr->start));
-                    LBX_HIP(hipEventCreate(&pr->stop));
-                    pr->rec.la = bra.la;
-                    pr->rec.lb = bra.lb;
-                    pr->rec.lc = ket.la;
-                    pr->rec.ld = ket.lb;
-                }
-                pr->rec.kernel = var;
-                LBX_HIP(hipEventRecord(pr->start, c.stream));
-            }
-            const TaskTable &t = launchJK(i, j, var, D, J, K, lo, hi);
+            const JKLaunch l = prepareJK(i, j, var, D, J, K, lo, hi);
+            const TaskTable &t = *l.t;
             st.quartets += t.quartets;
             st.flops += t.flops;
             if (isF32Variant(var))
                 st.quartets_fp32 += t.quartets;
-            if (pr)
+            if (!prof_on)
             {
-                LBX_HIP(hipEventRecord(pr->stop, c.stream));
-                pr->pending = true;
-                pr->rec.calls += 1;
-                pr->rec.quartets += t.quartets;
-                pr->rec.flops += t.flops;
+                queue.push_back({l.fn, l.a, t.flops});
+                return;
             }
+            // one class pair at a time on the context stream, an event pair around each
+            Prof &pr = prof[{i, j, tier}];
+            if (!pr.start)
+            {
+                LBX_HIP(hipEventCreate(&pr.start));
+                LBX_HIP(hipEventCreate(&pr.stop));
+                pr.rec.la = bra.la;
+                pr.rec.lb = bra.lb;
+                pr.rec.lc = ket.la;
+                pr.rec.ld = ket.lb;
+            }
+            pr.rec.kernel = var;
+            flushStaged();
+            LBX_HIP(hipEventRecord(pr.start, c.stream));
+            l.fn(l.a, c.stream);
+            LBX_HIP(hipGetLastError());
+            LBX_HIP(hipEventRecord(pr.stop, c.stream));
+            pr.pending = true;
+            pr.rec.calls += 1;
+            pr.rec.quartets += t.quartets;
+            pr.rec.flops += t.flops;
         };
         for (int i = 0; i < static_cast<int>(c.cls.size()); i++)
             for (int j = 0; j <= i; j++)
@@ -1960,6 +2137,9 @@ extern "C"
                 if (mixed && lo1 < hi1)
                     launch(i, j, 1, variant32For(i, j), lo1, hi1);
             }
+        flushStaged();
+        Fan fan(side, c.stream, queue.size() > 1);
+        launchAll(queue, fan);
         const int gridn = static_cast<int>(std::min<long long>((n * n + 255) / 256, 65536));
         hipLaunchKernelGGL(symmetrizeKernel, dim3(gridn), dim3(256), 0, c.stream, J, static_cast<int>(n));
         hipLaunchKernelGGL(symmetrizeKernel, dim3(gridn), dim3(256), 0, c.stream, K, static_cast<int>(n));
@@ -1983,7 +2163,7 @@ extern "C"
                            std::lock_guard<std::mutex> lk(ctx->mu);
                            Context &c = *ctx;
                            requireSingle(c, "lbx_jk");
-                           ensureSchwarz(c);
+                           ctx->ensureSchwarz();
                            // quartets with schwarz <= Q_ab Q_cd < split run in FP32
                            const bool mixed = precision == LBX_MIXED && mixed_thresh > schwarz_thresh;
                            const double split = mixed ? mixed_thresh : schwarz_thresh;
@@ -2050,8 +2230,8 @@ extern "C"
                                // eager launches on the context stream
                                if (split > 0.0)
                                {
-                                   ensureSchwarz(c);
-                                   ensureSchwarzAux(c);
+                                   ctx->ensureSchwarz();
+                                   ctx->ensureSchwarzAux();
                                    ensureF32(c);
                                    ensureF32Aux(c);
                                }
@@ -2066,8 +2246,8 @@ extern "C"
                                ctx->dropRiGraph();
                                if (split > 0.0)
                                {
-                                   ensureSchwarz(c);
-                                   ensureSchwarzAux(c);
+                                   ctx->ensureSchwarz();
+                                   ctx->ensureSchwarzAux();
                                    ensureF32(c);
                                    ensureF32Aux(c);
                                }
@@ -2142,7 +2322,7 @@ extern "C"
                            std::lock_guard<std::mutex> lk(ctx->mu);
                            Context &c = *ctx;
                            requireSingle(c, "lbx_jk_grad");
-                           ensureSchwarz(c);
+                           ctx->ensureSchwarz();
                            for (auto &pc : c.cls)
                                computeEcoeffsD1(c, pc);
                            const bool mixed = precision == LBX_MIXED && mixed_thresh > schwarz_thresh;
@@ -2203,7 +2383,7 @@ extern "C"
                                throw Error(LBX_ERR_INVALID, "lbx_tune: negative Schwarz threshold");
                            std::lock_guard<std::mutex> lk(ctx->mu);
                            Context &c = *ctx;
-                           ensureSchwarz(c);
+                           ctx->ensureSchwarz();
                            const long long n = static_cast<long long>(c.nbf);
                            DevBuf J(n * n), K(n * n);
                            hipEvent_t e0, e1;

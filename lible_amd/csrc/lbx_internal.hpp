@@ -4,7 +4,9 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <array>
+#include <cstring>
 #include <mutex>
 #include <stdexcept>
 #include <string>
@@ -141,6 +143,47 @@ namespace lbx
             return d;
         }
 
+        // Device copies of small host arrays (task tables), packed into chunks that live as long
+        // as the context and sent by flushStaged() with one copy: a first call on a molecule
+        // makes a few hundred of them.
+        struct Staging
+        {
+            char *d = nullptr;
+            size_t cap = 0, used = 0;
+            std::vector<char> host;   // bytes [used - host.size(), used) not sent yet
+        } staging;
+
+        template <class T>
+        T *stage(const std::vector<T> &v)
+        {
+            const size_t bytes = (std::max<size_t>(v.size(), 1) * sizeof(T) + 15) / 16 * 16;
+            if (staging.used + bytes > staging.cap)
+            {
+                flushStaged();
+                const size_t cap = std::max<size_t>(bytes, size_t(1) << 20);
+                staging.d = alloc<char>(cap);
+                staging.cap = cap;
+                staging.used = 0;
+            }
+            T *d = reinterpret_cast<T *>(staging.d + staging.used);
+            const size_t at = staging.host.size();
+            staging.host.resize(at + bytes);
+            if (!v.empty())
+                std::memcpy(staging.host.data() + at, v.data(), v.size() * sizeof(T));
+            staging.used += bytes;
+            return d;
+        }
+
+        // before the first launch that reads a staged array
+        void flushStaged()
+        {
+            const size_t n = staging.host.size();
+            if (n == 0)
+                return;
+            LBX_HIP(hipMemcpy(staging.d + staging.used - n, staging.host.data(), n, hipMemcpyHostToDevice));
+            staging.host.clear();
+        }
+
         void release();
     };
 
@@ -171,9 +214,6 @@ namespace lbx
     // null); both added into
     void computeOneElectronGrad(Context &c, const double *D, const double *W, const double4 *charges, int ncharges,
                                 double *grad, double *charge_grad);
-
-    // schwarz / task tables (capi.cpp)
-    void ensureSchwarz(Context &c);
 
     // d1.hip: dense first-derivative tensors of one class pair
     struct D1Args
