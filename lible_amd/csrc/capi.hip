@@ -120,6 +120,18 @@ namespace lbx
             }
         }
 
+        // out[i] = sum over the copies of in[copy * n + i]
+        __global__ void sumCopiesKernel(const double *in, double *out, long long n, int copies)
+        {
+            const long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
+            if (i >= n)
+                return;
+            double s = 0.0;
+            for (int k = 0; k < copies; k++)
+                s += in[k * n + i];
+            out[i] = s;
+        }
+
         void fill(double *p, long long n, double v, hipStream_t s)
         {
             if (n <= 0)
@@ -1213,10 +1225,20 @@ struct lbx_context : Context
         launchAll(queue, fan);
     }
 
-    // Queues the gradient kernel of class pair (i >= j) over the quartets with
-    // thresh <= Q_ab Q_cd < thresh_hi, in FP32 arithmetic when fp32; returns its task table.
-    const TaskTable &launchGrad(int i, int j, const double *D, double *grad, double thresh,
-                                double thresh_hi = kNoUpper, bool fp32 = false)
+    // The gradient kernel of class pair (i >= j) over the quartets with
+    // thresh <= Q_ab Q_cd < thresh_hi, in FP32 arithmetic when fp32.
+    struct GradLaunch
+    {
+        GradLauncher fn;
+        GArgs a;
+        const TaskTable *t;
+    };
+    // gradients the kernels' workgroups add to (GArgs::grad), summed at the end
+    static constexpr int kGradCopies = 64;
+    double *grad_copies = nullptr;
+
+    GradLaunch prepareGrad(int i, int j, const double *D, double thresh,
+                           double thresh_hi = kNoUpper, bool fp32 = false)
     {
         const PairClass &ci = cls[i], &cj = cls[j];
         const bool lane_i = gradLaneFirst(ci.la, ci.lb, cj.la, cj.lb);
@@ -1244,11 +1266,10 @@ struct lbx_context : Context
         a.boys = d_boys;
         a.D = D;
         a.nbf = static_cast<long long>(nbf);
-        a.grad = grad;
-        flushStaged();
-        (fp32 ? s.fn32 : s.fn)(a, stream);
-        LBX_HIP(hipGetLastError());
-        return t;
+        a.grad = grad_copies;
+        a.ncopy = kGradCopies;
+        a.stride = 3LL * natoms;
+        return {fp32 ? s.fn32 : s.fn, a, &t};
     }
 
     // Queues one J/K build on the context stream: J and K cleared, every class pair's kernel
@@ -2331,27 +2352,44 @@ extern "C"
                                ensureF32(c);
                                ensureF32D1(c);
                            }
-                           fill(grad, 3LL * c.natoms, 0.0, c.stream);
+                           const long long ng = 3LL * c.natoms;
+                           if (!ctx->grad_copies)
+                               ctx->grad_copies = c.alloc<double>(lbx_context::kGradCopies * ng);
+                           fill(ctx->grad_copies, lbx_context::kGradCopies * ng, 0.0, c.stream);
                            double nq = 0, fl = 0, nq32 = 0;
+                           std::vector<std::pair<double, lbx_context::GradLaunch>> queue;
+                           auto add = [&](int i, int j, double lo, double hi, bool fp32)
+                           {
+                               const PairClass &bra = c.cls[i], &ket = c.cls[j];
+                               const auto l = ctx->prepareGrad(i, j, D, lo, hi, fp32);
+                               const double f = gradFlops(*l.t, bra.la, bra.lb, ket.la, ket.lb);
+                               nq += l.t->quartets;
+                               nq32 += fp32 ? l.t->quartets : 0.0;
+                               fl += f;
+                               queue.emplace_back(f, l);
+                           };
                            for (int i = 0; i < static_cast<int>(c.cls.size()); i++)
                                for (int j = 0; j <= i; j++)
                                {
-                                   const PairClass &bra = c.cls[i], &ket = c.cls[j];
-                                   if (bra.n_pairs == 0 || ket.n_pairs == 0)
+                                   if (c.cls[i].n_pairs == 0 || c.cls[j].n_pairs == 0)
                                        continue;
-                                   const TaskTable &t = ctx->launchGrad(i, j, D, grad,
-                                                                        mixed ? mixed_thresh : schwarz_thresh);
-                                   nq += t.quartets;
-                                   fl += gradFlops(t, bra.la, bra.lb, ket.la, ket.lb);
+                                   add(i, j, mixed ? mixed_thresh : schwarz_thresh, kNoUpper, false);
                                    if (mixed)
-                                   {
-                                       const TaskTable &t32 = ctx->launchGrad(i, j, D, grad, schwarz_thresh,
-                                                                              mixed_thresh, true);
-                                       nq += t32.quartets;
-                                       nq32 += t32.quartets;
-                                       fl += gradFlops(t32, bra.la, bra.lb, ket.la, ket.lb);
-                                   }
+                                       add(i, j, schwarz_thresh, mixed_thresh, true);
                                }
+                           c.flushStaged();
+                           std::stable_sort(queue.begin(), queue.end(),
+                                            [](const auto &x, const auto &y) { return x.first > y.first; });
+                           Fan fan(ctx->side, c.stream, queue.size() > 1);
+                           for (auto &l : queue)
+                           {
+                               l.second.fn(l.second.a, fan.pick(l.first));
+                               LBX_HIP(hipGetLastError());
+                           }
+                           fan.join();
+                           hipLaunchKernelGGL(sumCopiesKernel, dim3(static_cast<int>((ng + 63) / 64)), dim3(64), 0,
+                                              c.stream, ctx->grad_copies, grad, ng, lbx_context::kGradCopies);
+                           LBX_HIP(hipGetLastError());
                            LBX_HIP(hipStreamSynchronize(c.stream));
                            if (stats)
                            {

@@ -413,6 +413,7 @@ namespace lbx
         template <int NT>
         __global__ __launch_bounds__(NT) void genericGrad(const GArgs A, const GenPlan G)
         {
+            double *const grad = A.grad + static_cast<long long>(blockIdx.x % A.ncopy) * A.stride;
             extern __shared__ double smem[];
             double *const sR0 = smem + G.oR0, *const sR1 = smem + G.oR1, *const sF = smem + G.oF;
             int *const sTuv = reinterpret_cast<int *>(smem + G.oTuv);
@@ -584,10 +585,10 @@ namespace lbx
 #pragma unroll
                     for (int x = 0; x < 3; x++)
                     {
-                        unsafeAtomicAdd(&A.grad[3 * at[0] + x], gA[x]);
-                        unsafeAtomicAdd(&A.grad[3 * at[1] + x], gB[x]);
-                        unsafeAtomicAdd(&A.grad[3 * at[2] + x], gC[x]);
-                        unsafeAtomicAdd(&A.grad[3 * at[3] + x], -(gA[x] + gB[x] + gC[x]));
+                        unsafeAtomicAdd(&grad[3 * at[0] + x], gA[x]);
+                        unsafeAtomicAdd(&grad[3 * at[1] + x], gB[x]);
+                        unsafeAtomicAdd(&grad[3 * at[2] + x], gC[x]);
+                        unsafeAtomicAdd(&grad[3 * at[3] + x], -(gA[x] + gB[x] + gC[x]));
                     }
                 }
                 __syncthreads();   // density blocks of the next task

@@ -14,17 +14,20 @@
 // This is the quantity of the reference's ERI4D1 kernel (eri_kernel_funs.cpp:582-748) contracted
 // with the density weights.
 //
-// Evaluation, per primitive pair i of the lane-side pair and column pass of cd:
+// Two kernels: the slot form here for class pairs of low total angular momentum, the one-wave MFMA
+// form (grad_wave.hpp) for the others.
+//
+// Slot form: one wave per task, a task is G lane-side pairs against one uniform-side pair; each
+// pair (slot) has LPS = 64/G lanes that split its Hermite index h.  R of LPS primitive quartets per
+// slot is made at a time, one lane per primitive quartet with the recursion in registers, and goes
+// to LDS; then per primitive pair i of the lane side and column pass of cd
 //   Y[h][cd] = sum_ab Eb_i[ab][h] W[ab][cd]
 //   per ket primitive j:  T += sum_{h,g} (sum_cd Y Ek_j) R_{h+g+e_x},  V += sum_{h,g} R_{h+g}
 //                         (sum_cd Y Ek'_j,x),   X[h][cd] += sum_g R_{h+g} Ek_j[cd][g]
-//   then U = sum_{ab,cd} W[ab][cd] sum_h Eb'_i,x[ab][h] X[h][cd].
-// Work layout: one wave per task; a task is G lane-side pairs against one uniform-side pair;
-// each pair (slot) gets 64/G lanes that split its Hermite index h; R is built cooperatively in
-// LDS per slot, W sits in LDS per slot.
+//   U = sum_{ab,cd} W[ab][cd] sum_h Eb'_i,x[ab][h] X[h][cd].
 #pragma once
 
-#include "device_common.hpp"
+#include "hermite_lds.hpp"
 #include "dpairs.hpp"
 
 namespace lbx
@@ -40,7 +43,12 @@ namespace lbx
         const double *boys;
         const double *D;
         long long nbf;
-        double *grad;                // 3 natoms
+        // ncopy gradients of 3 natoms values, `stride` apart, which the caller adds up: a workgroup
+        // adds to copy blockIdx % ncopy (the few lines of a small molecule's gradient would
+        // serialise the atomics: about 60 M additions per second and line)
+        double *grad;
+        int ncopy;
+        long long stride;
     };
 
     using GradLauncher = void (*)(const GArgs &, hipStream_t);
@@ -61,12 +69,34 @@ namespace lbx
         return p;
     }
 
-    // lane side chosen for an unordered class pair: the larger Hermite dimension (more lanes in
-    // use), ties to the larger class index
+    // Class pairs whose R of order L + 1 stays in a lane's registers and 64 of them in 32 KiB of
+    // LDS take the slot form.
+    constexpr int kGradSlotL1 = 5;
+    constexpr LBX_HD bool gradUsesSlots(int la, int lb, int lc, int ld) { return la + lb + lc + ld + 1 <= kGradSlotL1; }
+
+    // MFMAs of a quartet of the one-wave form with two primitive pairs a side when (la lb) takes
+    // the rows
+    constexpr LBX_HD int gradWaveCost(int la, int lb, int lc, int ld)
+    {
+        const int hp = nHerm(la + lb), hp1 = nHerm(la + lb + 1), hq = nHerm(lc + ld);
+        const int sp = nSph(la) * nSph(lb), sq = nSph(lc) * nSph(ld);
+        const int nq = ceilDiv(sq, 16);
+        return nq * (4 * (ceilDiv(hp1, 16) * ceilDiv(hq, 4) + ceilDiv(hq, 16) * ceilDiv(hp, 4)) +
+                     2 * (ceilDiv(hp, 16) * ceilDiv(sp, 4) + 3 * ceilDiv(sp, 16) * ceilDiv(hp, 4)));
+    }
+
+    // lane side ("bra") chosen for an unordered class pair: in the one-wave form (main shells to f)
+    // the assignment with fewer MFMAs, else the larger Hermite dimension (more lanes in use); ties
+    // to the larger class index
     constexpr LBX_HD bool gradLaneFirst(int la, int lb, int lc, int ld)
     {
-        return nHerm(la + lb) > nHerm(lc + ld) ||
-               (nHerm(la + lb) == nHerm(lc + ld) && pairClassIdx(la, lb) >= pairClassIdx(lc, ld));
+        const bool tie = pairClassIdx(la, lb) >= pairClassIdx(lc, ld);
+        if (!gradUsesSlots(la, lb, lc, ld) && la <= 3 && lc <= 3)
+        {
+            const int x = gradWaveCost(la, lb, lc, ld), y = gradWaveCost(lc, ld, la, lb);
+            return x != y ? x < y : tie;
+        }
+        return nHerm(la + lb) > nHerm(lc + ld) || (nHerm(la + lb) == nHerm(lc + ld) && tie);
     }
 
     template <int LA, int LB, int LC, int LD>
@@ -76,17 +106,27 @@ namespace lbx
         static constexpr int HP = nHerm(LA + LB), HQ = nHerm(LC + LD), HL1 = nHerm(L1);
         static constexpr int SA = nSph(LA), SB = nSph(LB), SC = nSph(LC), SD = nSph(LD);
         static constexpr int SP = SA * SB, SQ = SC * SD;
-        static constexpr int kLds = 6144;   // doubles of LDS per wave (48 KiB)
-        static constexpr int perSlot = 2 * HL1 + SP * SQ;
-        static constexpr int G0 = 64 / (HP >= 64 ? 64 : pow2Ceil(HP));
-        static constexpr int gFit(int g) { return (g > 1 && g * perSlot > kLds) ? gFit(g / 2) : g; }
-        static constexpr int G = gFit(G0);
-        static constexpr int LPS = 64 / G;                 // lanes per slot
-        static constexpr int NH = ceilDiv(HP, LPS);        // h values per lane
-        static constexpr int NC = SQ < 8 ? SQ : 8;         // cd columns per pass
-        static constexpr int NPASS = ceilDiv(SQ, NC);
-        static_assert(G * perSlot <= kLds, "gradient LDS budget");
+        // lanes per slot: the Hermite rows (HR) times REP, REP groups of them taking the ket
+        // primitives of a lane-side primitive in turn (few rows would leave the long primitive loops
+        // of contracted s and p shells to one or four lanes)
+        static constexpr int HR = HP >= 64 ? 64 : pow2Ceil(HP);
+        static constexpr int REP = HP == 1 ? 4 : (HP == 4 ? 2 : 1);
+        static constexpr int LPS = HR * REP;
+        static constexpr int G = 64 / LPS;
+        static constexpr int NH = ceilDiv(HP, HR);         // h values per lane
+        static constexpr int NPASS = ceilDiv(SQ, 9);
+        static constexpr int NC = ceilDiv(SQ, NPASS);      // cd columns per pass, at most 9
+        static constexpr int RS = HL1 | 1;                 // LDS stride of one primitive quartet's R (odd)
     };
+
+    template <bool UNIFORM, typename T>
+    __device__ __forceinline__ auto uniformView(const T *p)
+    {
+        if constexpr (UNIFORM)
+            return constView(p);
+        else
+            return p;
+    }
 
     // sum over the LPS lanes of one slot (contiguous lane groups)
     template <int LPS>
@@ -110,38 +150,35 @@ namespace lbx
     // small-bound quartets of the mixed-precision gradient); Boys values, density weights and the
     // gradient sums stay double.
     template <int LA, int LB, int LC, int LD, typename T>
-    __global__ __launch_bounds__(64) void gradKernel(const GArgs A)
+    __global__ __launch_bounds__(64, 2) void gradKernel(const GArgs A)
     {
         using C = GCls<LA, LB, LC, LD>;
-        constexpr int L1 = C::L1, HP = C::HP, HQ = C::HQ, HL1 = C::HL1, SP = C::SP, SQ = C::SQ,
-                      SB = C::SB, SD = C::SD, G = C::G, LPS = C::LPS, NH = C::NH, NC = C::NC;
+        constexpr int L1 = C::L1, HP = C::HP, HQ = C::HQ, HL1 = C::HL1, SP = C::SP, SQ = C::SQ, SB = C::SB, SD = C::SD,
+                      G = C::G, LPS = C::LPS, HR = C::HR, REP = C::REP, NH = C::NH, NC = C::NC, RS = C::RS;
         constexpr bool F32 = sizeof(T) == 4;
-        __shared__ T sR[2][G][HL1];
-        __shared__ double sW[G][SP * SQ];
-        const int lane = threadIdx.x;
-        const int slot = lane / LPS, jl = lane % LPS;
+        __shared__ T sR[64 * RS];
+        __shared__ double sW[G * SP * SQ];
+        __shared__ unsigned short sTab[HP * HQ][4];   // R index of h + g, and of h + g + e_x
+        const int lane0 = threadIdx.x;
         const DPairs &LP = A.lane, &UP = A.unif;
         const long long n = A.nbf;
         const double *D = A.D;
-
-        // (t, u, v) of this lane's Hermite indices
-        int th[NH], uh[NH], vh[NH];
-        bool hv[NH];
-#pragma unroll
-        for (int r = 0; r < NH; r++)
-        {
-            const int h = jl + r * LPS;
-            hv[r] = h < HP;
-            const int tuv = hermTuv(hv[r] ? h : 0);
-            th[r] = tuv & 255;
-            uh[r] = (tuv >> 8) & 255;
-            vh[r] = tuv >> 16;
-        }
+        double *const grad = A.grad + static_cast<long long>(blockIdx.x % A.ncopy) * A.stride;
 
         const long long t0 = A.ntasks * blockIdx.x / gridDim.x;
         const long long t1 = A.ntasks * (blockIdx.x + 1) / gridDim.x;
         if (t0 >= t1)
             return;
+        for (int e = lane0; e < HP * HQ; e += 64)
+        {
+            const int a = hermTuv(e / HQ), b = hermTuv(e % HQ);
+            const int t = (a & 255) + (b & 255), u = ((a >> 8) & 255) + ((b >> 8) & 255), v = (a >> 16) + (b >> 16);
+            sTab[e][0] = static_cast<unsigned short>(hermIdx(t, u, v));
+            sTab[e][1] = static_cast<unsigned short>(hermIdx(t + 1, u, v));
+            sTab[e][2] = static_cast<unsigned short>(hermIdx(t, u + 1, v));
+            sTab[e][3] = static_cast<unsigned short>(hermIdx(t, u, v + 1));
+        }
+        waveFence();
         int q = uniform(findKet(A.prefix, A.nket, t0));
         long long base = A.prefix[q], next = A.prefix[q + 1];
         for (long long t = t0; t < t1; t++)
@@ -152,6 +189,8 @@ namespace lbx
                 base = next;
                 next = A.prefix[q + 1];
             }
+            const int lane = opaqueLane(lane0);
+            const int slot = lane / LPS, jl = lane % LPS, jh = jl % HR, rep = jl / HR;
             const int local = static_cast<int>(t - base);
             const int plo = uniform(A.plo[q]), phi = uniform(A.phi[q]);
             const int p = plo + local * G + slot;
@@ -172,178 +211,166 @@ namespace lbx
                 f *= 0.5;
 
             // density weights of this slot's quartet
+            double *const w0 = sW + slot * (SP * SQ);
             for (int e = jl; e < SP * SQ; e += LPS)
             {
                 const int ab = e / SQ, cd = e - ab * SQ;
                 const int al = ab / SB, be = ab - al * SB, ga = cd / SD, de = cd - ga * SD;
                 const long long ia = a0 + al, ib = b0 + be, ic = c0 + ga, id = d0 + de;
-                sW[slot][e] = active ? f * (4.0 * D[ia * n + ib] * D[ic * n + id] -
-                                            D[ia * n + ic] * D[ib * n + id] - D[ia * n + id] * D[ib * n + ic])
-                                     : 0.0;
+                w0[e] = active ? f * (4.0 * D[ia * n + ib] * D[ic * n + id] - D[ia * n + ic] * D[ib * n + id] -
+                                      D[ia * n + id] * D[ib * n + ic])
+                               : 0.0;
             }
-            __syncthreads();
+            waveFence();
 
             double gA[3] = {0, 0, 0}, gB[3] = {0, 0, 0}, gC[3] = {0, 0, 0};
+            // primitive quartets e = i ucnt + k of every slot, LPS of them at a time
+            const int emax = imax * ucnt;
 #pragma unroll 1
-            for (int pass = 0; pass < C::NPASS; pass++)
+            for (int e0 = 0; e0 < emax; e0 += LPS)
             {
-                const int cd0 = pass * NC;
-#pragma unroll 1
-                for (int i = 0; i < imax; i++)
                 {
-                    const bool valid = i < lcnt;
-                    const int ip = lpoff + (valid ? i : 0);
-                    // Y[h][c] = sum_ab Eb_i[h][ab] W[ab][cd0 + c]
-                    T Y[NH][NC], X[NH][NC];
-                    const T *eb;
-                    if constexpr (F32)
-                        eb = LP.eb32 + static_cast<size_t>(ip) * HP * SP;
-                    else
-                        eb = LP.eb + static_cast<size_t>(ip) * HP * SP;
-#pragma unroll
-                    for (int r = 0; r < NH; r++)
-#pragma unroll
-                        for (int c = 0; c < NC; c++)
-                        {
-                            Y[r][c] = T(0);
-                            X[r][c] = T(0);
-                        }
-                    for (int ab = 0; ab < SP; ab++)
+                    const int e = e0 + jl, i = e / ucnt, k = e - i * ucnt;
+                    waveFence();
+                    if (i < lcnt)
                     {
-                        T w[NC];
+                        const double4 Pl = LP.pp[lpoff + i], Pu = UP.pp[upoff + k];
+                        const double pq = Pl.x * Pu.x, ps = Pl.x + Pu.x, alpha = pq / ps;
+                        const double X = Pl.y - Pu.y, Y = Pl.z - Pu.z, Z = Pl.w - Pu.w;
+                        double F[L1 + 1];
+                        boysF<L1>(alpha * (X * X + Y * Y + Z * Z), A.boys, F);
+                        T R[HL1 + L1];
+                        double sc = kTwoPi52 / (pq * sqrt(ps));
 #pragma unroll
-                        for (int c = 0; c < NC; c++)
-                            w[c] = cd0 + c < SQ ? T(sW[slot][ab * SQ + cd0 + c]) : T(0);
+                        for (int m = 0; m <= L1; m++)
+                        {
+                            R[m] = T(F[m] * sc);
+                            sc *= -2.0 * alpha;
+                        }
+                        hermiteR<L1, T>(R, T(X), T(Y), T(Z));
+                        T *const out = sR + lane * RS;
+                        out[0] = R[0];
+#pragma unroll
+                        for (int h = 1; h < HL1; h++)
+                            out[h] = R[L1 + h];
+                    }
+                    waveFence();
+                }
+                const int e1 = min(e0 + LPS, emax);
+#pragma unroll 1
+                for (int pass = 0; pass < C::NPASS; pass++)
+                {
+                    const int cd0 = pass * NC;
+                    int e = e0;
+#pragma unroll 1
+                    while (e < e1)
+                    {
+                        // the run of one lane-side primitive pair in this batch
+                        const int i = e / ucnt, kBeg = e - i * ucnt, kEnd = min(ucnt, kBeg + e1 - e);
+                        const bool valid = i < lcnt;
+                        const int ip = lpoff + (valid ? i : 0);
+                        // Y[h][c] = sum_ab Eb_i[h][ab] W[ab][cd0 + c]
+                        T Y[NH][NC], X[NH][NC];
+                        const T *eb, *e1b;
+                        if constexpr (F32)
+                        {
+                            eb = LP.eb32 + static_cast<size_t>(ip) * HP * SP;
+                            e1b = LP.e1b32 + static_cast<size_t>(ip) * 3 * HP * SP;
+                        }
+                        else
+                        {
+                            eb = LP.eb + static_cast<size_t>(ip) * HP * SP;
+                            e1b = LP.e1b + static_cast<size_t>(ip) * 3 * HP * SP;
+                        }
 #pragma unroll
                         for (int r = 0; r < NH; r++)
-                        {
-                            const T e = hv[r] ? eb[(jl + r * LPS) * SP + ab] : T(0);
 #pragma unroll
                             for (int c = 0; c < NC; c++)
-                                Y[r][c] = fma(e, w[c], Y[r][c]);
+                            {
+                                Y[r][c] = T(0);
+                                X[r][c] = T(0);
+                            }
+#pragma unroll 3
+                        for (int ab = 0; ab < SP; ab++)
+                        {
+                            T w[NC];
+#pragma unroll
+                            for (int c = 0; c < NC; c++)
+                                w[c] = cd0 + c < SQ ? T(w0[ab * SQ + cd0 + c]) : T(0);
+#pragma unroll
+                            for (int r = 0; r < NH; r++)
+                            {
+                                const int h = jh + r * HR;
+                                const T ev = h < HP ? eb[h * SP + ab] : T(0);
+#pragma unroll
+                                for (int c = 0; c < NC; c++)
+                                    Y[r][c] = fma(ev, w[c], Y[r][c]);
+                            }
                         }
-                    }
-                    const double4 Pl = LP.pp[ip];
-                    double Ts[3] = {0, 0, 0};
-                    const cptr<double> ppU = constView(reinterpret_cast<const double *>(UP.pp + upoff));
-                    // Boys table row of ket primitive k + 1 fetched while k is computed
-                    auto argOf = [&](int k) {
-                        const double X_ = Pl.y - ppU[4 * k + 1], Y_ = Pl.z - ppU[4 * k + 2],
-                                     Z_ = Pl.w - ppU[4 * k + 3];
-                        const double pq = Pl.x * ppU[4 * k], ps = Pl.x + ppU[4 * k];
-                        return pq / ps * (X_ * X_ + Y_ * Y_ + Z_ * Z_);
-                    };
-                    BoysRow next;
-                    boysFetch<L1>(argOf(0), A.boys, next);
+                        double Ts[3] = {0, 0, 0};
 #pragma unroll 1
-                    for (int k = 0; k < ucnt; k++)
-                    {
-                        const BoysRow cur = next;
-                        if (k + 1 < ucnt)
-                            boysFetch<L1>(argOf(k + 1), A.boys, next);
-                        const double4 Pu{ppU[4 * k], ppU[4 * k + 1], ppU[4 * k + 2], ppU[4 * k + 3]};
-                        const double pq = Pl.x * Pu.x, ps = Pl.x + Pu.x, alpha = pq / ps;
-                        const double PX = Pl.y - Pu.y, PY = Pl.z - Pu.z, PZ = Pl.w - Pu.w;
-                        double F[L1 + 1];
-                        boysEval<L1>(cur, F);
-                        const double fac = kTwoPi52 / (pq * sqrt(ps));
-                        double init[L1 + 1];
+                        for (int kr = kBeg; kr < kEnd; kr += REP)
                         {
-                            double sc = fac;
-#pragma unroll
-                            for (int m = 0; m <= L1; m++)
-                            {
-                                init[m] = F[m] * sc;
-                                sc *= -2.0 * alpha;
-                            }
-                        }
-                        // levels n = L1 .. 0 of R^{(n)}_{tuv}, |tuv| <= L1 - n, ping-pong in LDS
-                        if (jl == 0)
-                            sR[L1 & 1][slot][0] = T(init[L1]);
-                        __syncthreads();
-#pragma unroll
-                        for (int lev = L1 - 1; lev >= 0; lev--)
-                        {
-                            const int nh = nHerm(L1 - lev);
-                            const T *in = sR[(lev + 1) & 1][slot];
-                            T *out = sR[lev & 1][slot];
-                            for (int h = jl; h < nh; h += LPS)
-                            {
-                                if (h == 0)
-                                {
-                                    out[0] = T(init[lev]);
-                                    continue;
-                                }
-                                const unsigned rt = kRecTab.v[h];
-                                const int s1 = rt & 2047, s2 = (rt >> 11) & 2047, ax = (rt >> 22) & 3,
-                                          cm = rt >> 24;
-                                const T xa = T(ax == 0 ? PX : (ax == 1 ? PY : PZ));
-                                out[h] = fma(xa, in[s1], T(cm) * in[s2]);
-                            }
-                            __syncthreads();
-                        }
-                        const T *R = sR[0][slot];
-                        if (valid)
-                        {
+                            const int k = min(kr + rep, kEnd - 1);   // past the end: not used
+                            const bool use = valid && kr + rep < kEnd;
+                            const T *R = sR + (slot * LPS + e - e0 + k - kBeg) * RS;
                             const size_t kk = static_cast<size_t>(upoff + k);
-                            const T *ekb, *e1b;
+                            const T *ekb, *e1kb;
                             if constexpr (F32)
                             {
                                 ekb = UP.ek32;
-                                e1b = UP.e1k32;
+                                e1kb = UP.e1k32;
                             }
                             else
                             {
                                 ekb = UP.ek;
-                                e1b = UP.e1k;
+                                e1kb = UP.e1k;
                             }
-                            const cptr<T> ek = constView(ekb + kk * HQ * SQ + cd0);
-                            const cptr<T> e1 = constView(e1b + kk * 3 * HQ * SQ + cd0);
+                            // wave-uniform (scalar loads) unless the groups are at different k
+                            const auto ek = uniformView<REP == 1>(ekb + kk * HQ * SQ + cd0);
+                            const auto e1 = uniformView<REP == 1>(e1kb + kk * 3 * HQ * SQ + cd0);
                             double tk[3] = {0, 0, 0};
+                            if (use)
 #pragma unroll
-                            for (int g = 0; g < HQ; g++)
-                            {
-                                const int tuvg = hermTuv(g);
-                                const int tg = tuvg & 255, ug = (tuvg >> 8) & 255, vg = tuvg >> 16;
-                                T ekv[NC], e1v[3][NC];
-#pragma unroll
-                                for (int c = 0; c < NC; c++)
+                                for (int g = 0; g < HQ; g++)
                                 {
-                                    const bool in = cd0 + c < SQ;
-                                    ekv[c] = in ? ek[g * SQ + c] : T(0);
-#pragma unroll
-                                    for (int x = 0; x < 3; x++)
-                                        e1v[x][c] = in ? e1[(x * HQ + g) * SQ + c] : T(0);
-                                }
-#pragma unroll
-                                for (int r = 0; r < NH; r++)
-                                {
-                                    if (!hv[r])
-                                        continue;
-                                    const int tt = th[r] + tg, uu = uh[r] + ug, vv = vh[r] + vg;
-                                    const T r0 = R[hermIdx(tt, uu, vv)];
-                                    const T rx = R[hermIdx(tt + 1, uu, vv)];
-                                    const T ry = R[hermIdx(tt, uu + 1, vv)];
-                                    const T rz = R[hermIdx(tt, uu, vv + 1)];
-                                    T z = T(0), zx = T(0), zy = T(0), zz = T(0);
+                                    T ekv[NC], e1v[3][NC];
 #pragma unroll
                                     for (int c = 0; c < NC; c++)
                                     {
-                                        z = fma(Y[r][c], ekv[c], z);
-                                        zx = fma(Y[r][c], e1v[0][c], zx);
-                                        zy = fma(Y[r][c], e1v[1][c], zy);
-                                        zz = fma(Y[r][c], e1v[2][c], zz);
-                                        X[r][c] = fma(r0, ekv[c], X[r][c]);
+                                        const bool in = cd0 + c < SQ;
+                                        ekv[c] = in ? ek[g * SQ + c] : T(0);
+#pragma unroll
+                                        for (int x = 0; x < 3; x++)
+                                            e1v[x][c] = in ? e1[(x * HQ + g) * SQ + c] : T(0);
                                     }
-                                    tk[0] = fma(double(z), double(rx), tk[0]);
-                                    tk[1] = fma(double(z), double(ry), tk[1]);
-                                    tk[2] = fma(double(z), double(rz), tk[2]);
-                                    gC[0] = fma(double(r0), double(zx), gC[0]);
-                                    gC[1] = fma(double(r0), double(zy), gC[1]);
-                                    gC[2] = fma(double(r0), double(zz), gC[2]);
+#pragma unroll
+                                    for (int r = 0; r < NH; r++)
+                                    {
+                                        const int h = jh + r * HR;
+                                        if (h >= HP)
+                                            continue;
+                                        const unsigned short *tab = sTab[h * HQ + g];
+                                        const T r0 = R[tab[0]], rx = R[tab[1]], ry = R[tab[2]], rz = R[tab[3]];
+                                        T z = T(0), zx = T(0), zy = T(0), zz = T(0);
+#pragma unroll
+                                        for (int c = 0; c < NC; c++)
+                                        {
+                                            z = fma(Y[r][c], ekv[c], z);
+                                            zx = fma(Y[r][c], e1v[0][c], zx);
+                                            zy = fma(Y[r][c], e1v[1][c], zy);
+                                            zz = fma(Y[r][c], e1v[2][c], zz);
+                                            X[r][c] = fma(r0, ekv[c], X[r][c]);
+                                        }
+                                        tk[0] = fma(double(z), double(rx), tk[0]);
+                                        tk[1] = fma(double(z), double(ry), tk[1]);
+                                        tk[2] = fma(double(z), double(rz), tk[2]);
+                                        gC[0] = fma(double(r0), double(zx), gC[0]);
+                                        gC[1] = fma(double(r0), double(zy), gC[1]);
+                                        gC[2] = fma(double(r0), double(zz), gC[2]);
+                                    }
                                 }
-                            }
-                            const double rc = constView(UP.ra)[upoff + k];   // c / q
+                            const double rc = uniformView<REP == 1>(UP.ra)[upoff + k];   // c / q
 #pragma unroll
                             for (int x = 0; x < 3; x++)
                             {
@@ -351,51 +378,47 @@ namespace lbx
                                 gC[x] = fma(-rc, tk[x], gC[x]);
                             }
                         }
-                        __syncthreads();
-                    }
-                    if (valid)
-                    {
-                        const double ra = LP.ra[ip];   // a / p
-#pragma unroll
-                        for (int x = 0; x < 3; x++)
+                        if (valid)
                         {
-                            gA[x] = fma(ra, Ts[x], gA[x]);
-                            gB[x] = fma(1.0 - ra, Ts[x], gB[x]);
-                        }
-                        // U_x = sum_ab sum_c W[ab][cd0 + c] sum_h Eb'_x[h][ab] X[h][c]
-                        const T *e1;
-                        if constexpr (F32)
-                            e1 = LP.e1b32 + static_cast<size_t>(ip) * 3 * HP * SP;
-                        else
-                            e1 = LP.e1b + static_cast<size_t>(ip) * 3 * HP * SP;
-                        double ux[3] = {0, 0, 0};
-                        for (int ab = 0; ab < SP; ab++)
-                        {
-                            T w[NC];
+                            const double ra = LP.ra[ip];   // a / p
 #pragma unroll
-                            for (int c = 0; c < NC; c++)
-                                w[c] = cd0 + c < SQ ? T(sW[slot][ab * SQ + cd0 + c]) : T(0);
-#pragma unroll
-                            for (int r = 0; r < NH; r++)
+                            for (int x = 0; x < 3; x++)
                             {
-                                if (!hv[r])
-                                    continue;
-                                T s = T(0);
+                                gA[x] = fma(ra, Ts[x], gA[x]);
+                                gB[x] = fma(1.0 - ra, Ts[x], gB[x]);
+                            }
+                            // U_x = sum_ab sum_c W[ab][cd0 + c] sum_h Eb'_x[h][ab] X[h][c]
+                            double ux[3] = {0, 0, 0};
+#pragma unroll 3
+                            for (int ab = 0; ab < SP; ab++)
+                            {
+                                T w[NC];
 #pragma unroll
                                 for (int c = 0; c < NC; c++)
-                                    s = fma(w[c], X[r][c], s);
-                                const int h = jl + r * LPS;
+                                    w[c] = cd0 + c < SQ ? T(w0[ab * SQ + cd0 + c]) : T(0);
 #pragma unroll
-                                for (int x = 0; x < 3; x++)
-                                    ux[x] = fma(double(e1[(x * HP + h) * SP + ab]), double(s), ux[x]);
+                                for (int r = 0; r < NH; r++)
+                                {
+                                    const int h = jh + r * HR;
+                                    if (h >= HP)
+                                        continue;
+                                    T s = T(0);
+#pragma unroll
+                                    for (int c = 0; c < NC; c++)
+                                        s = fma(w[c], X[r][c], s);
+#pragma unroll
+                                    for (int x = 0; x < 3; x++)
+                                        ux[x] = fma(double(e1b[(x * HP + h) * SP + ab]), double(s), ux[x]);
+                                }
+                            }
+#pragma unroll
+                            for (int x = 0; x < 3; x++)
+                            {
+                                gA[x] += ux[x];
+                                gB[x] -= ux[x];
                             }
                         }
-#pragma unroll
-                        for (int x = 0; x < 3; x++)
-                        {
-                            gA[x] += ux[x];
-                            gB[x] -= ux[x];
-                        }
+                        e += kEnd - kBeg;
                     }
                 }
             }
@@ -412,13 +435,13 @@ namespace lbx
 #pragma unroll
                 for (int x = 0; x < 3; x++)
                 {
-                    unsafeAtomicAdd(&A.grad[3 * at[0] + x], gA[x]);
-                    unsafeAtomicAdd(&A.grad[3 * at[1] + x], gB[x]);
-                    unsafeAtomicAdd(&A.grad[3 * at[2] + x], gC[x]);
-                    unsafeAtomicAdd(&A.grad[3 * at[3] + x], -(gA[x] + gB[x] + gC[x]));
+                    unsafeAtomicAdd(&grad[3 * at[0] + x], gA[x]);
+                    unsafeAtomicAdd(&grad[3 * at[1] + x], gB[x]);
+                    unsafeAtomicAdd(&grad[3 * at[2] + x], gC[x]);
+                    unsafeAtomicAdd(&grad[3 * at[3] + x], -(gA[x] + gB[x] + gC[x]));
                 }
             }
-            __syncthreads();   // sW of the next task
+            waveFence();   // sW of the next task
         }
     }
 

@@ -1,7 +1,7 @@
 // Instantiation unit of the gradient kernels, compiled once per LBX_GUNIT = lane-side main pair
 // class (order (0,0),(1,0),(1,1),(2,0),...): one kernel for every uniform-side class for which
 // this class is the lane side (gradLaneFirst).
-#include "grad.hpp"
+#include "grad_wave.hpp"
 
 #ifndef LBX_GUNIT
 #error "LBX_GUNIT must be defined"
@@ -24,7 +24,12 @@ namespace lbx
         void reg()
         {
             if constexpr (gradLaneFirst(PA, PB, LC, LD))
-                registerGrad<PA, PB, LC, LD>();
+            {
+                if constexpr (gradUsesSlots(PA, PB, LC, LD))
+                    registerGrad<PA, PB, LC, LD>();
+                else
+                    registerGradWave<PA, PB, LC, LD>();
+            }
         }
 
         struct Registrar

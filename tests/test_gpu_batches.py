@@ -1,0 +1,138 @@
+"""The kernels that work on batches of primitive quartets, at the edges of their batches and tiles,
+against the oracle: contractions longer than a batch, uneven contractions in one class, sizes around
+the 64 x 64 tiles of the density-fitting products, blocks in every order of their shells.
+
+Tolerances: FP64 sums of at most a few thousand terms in another order, 1e-12 relative with a floor
+of 1e-13 of the largest element (the other parity tests'); the gradient 1e-10 relative as in
+test_jk_grad."""
+import itertools
+
+import numpy as np
+import pytest
+
+from lible_amd import basis as B
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def lbx():
+    from lible_amd import lbx as L
+    L.lib()
+    return L
+
+
+@pytest.fixture(scope="module")
+def oracle():
+    from oracle import oracle as O
+    return O
+
+
+def close(gpu, ref, rel=1e-12, floor=1e-13):
+    gpu, ref = np.asarray(gpu), np.asarray(ref)
+    err, tol = np.abs(gpu - ref), rel * np.abs(ref) + floor * np.abs(ref).max()
+    assert (err <= tol).all(), f"{(err > tol).sum()} of {ref.size}, worst {(err / np.maximum(tol, 1e-300)).max():.2f} tol"
+
+
+def uneven_molecule(seed, contractions):
+    """Two atoms 1.6 bohr apart; contractions: [(l, K), ...] on the first, reversed on the second."""
+    rng = np.random.default_rng(seed)
+    per_atom = []
+    for order in (1, -1):
+        per_atom.append([(l, list(np.exp(rng.uniform(np.log(0.2), np.log(40.0), K))), list(rng.uniform(0.1, 1.0, K)))
+                         for l, K in contractions[::order]])
+    coords = np.array([[0.0, 0.1, -0.2], [0.9, 0.8, 1.1]])
+    return B.Molecule(coords, B.Shells.from_lists(per_atom))
+
+
+# (l, K) lists: K_ab up to 121 (s, s), 81 (p, p) and 25 (f, d), beyond every batch (64 primitive
+# quartets at low L, 3 at (ff|ff)), next to single primitives
+UNEVEN = [[(0, 11), (0, 1), (1, 2)], [(1, 9), (0, 2), (2, 1)], [(2, 5), (1, 1), (3, 1), (0, 1)],
+          [(3, 5), (2, 5), (0, 1), (1, 1)]]
+
+
+@pytest.mark.parametrize("contractions", UNEVEN)
+@pytest.mark.parametrize("variant", [None, 2, 6])
+def test_jk_uneven_contractions(lbx, oracle, contractions, variant):
+    import torch
+    m = uneven_molecule(5, contractions)
+    D = B.density_from_orbitals(3, m.shells.nbf, 3, 0.3)
+    Jr, Kr, _ = oracle.Structure(m).jk(D, thresh=0.0)
+    ctx = lbx.Context(m)
+    if variant is not None:
+        for la, lc in itertools.product(range(4), repeat=2):
+            for lb, ld in itertools.product(range(la + 1), range(lc + 1)):
+                ctx.set_variant((la, lb, lc, ld), variant)
+    J, K, _ = ctx.jk(torch.tensor(D, device="cuda"), schwarz=0.0)
+    close(J.cpu().numpy(), Jr)
+    close(K.cpu().numpy(), Kr)
+
+
+@pytest.mark.parametrize("contractions", UNEVEN)
+def test_jk_grad_uneven_contractions(lbx, oracle, contractions):
+    import torch
+    m = uneven_molecule(6, contractions)
+    D = B.density_from_orbitals(4, m.shells.nbf, 3, 0.3)
+    ref = oracle.Structure(m).jk_grad(D, thresh=0.0)
+    g, _ = lbx.Context(m).jk_grad(torch.tensor(D, device="cuda"), schwarz=0.0)
+    close(g.cpu().numpy(), ref, rel=1e-10, floor=1e-10)
+
+
+@pytest.mark.parametrize("natoms", [1, 3, 16])
+def test_dense_uneven(lbx, oracle, natoms):
+    """Dense eri4 / diagonal of 1 to 16 one-shell atoms (the largest has more pairs than lanes)."""
+    rng = np.random.default_rng(natoms)
+    per_atom = [[(k % 2, list(rng.uniform(0.3, 3.0, 1 + k % 3)), list(rng.uniform(0.2, 1.0, 1 + k % 3)))]
+                for k in range(natoms)]
+    m = B.Molecule(B.random_atoms(rng, natoms, 5.0, 0.8), B.Shells.from_lists(per_atom))
+    s, ctx = oracle.Structure(m), lbx.Context(m)
+    for _ in range(2):   # the second call reuses the task tables
+        close(ctx.eri4().cpu().numpy(), s.eri4(), floor=1e-14)
+        close(ctx.eri4_diag().cpu().numpy(), s.eri4_diag(), floor=1e-14)
+
+
+@pytest.fixture(scope="module")
+def block_case(oracle):
+    m = B.synthetic_molecule(77, 2, 3.0, B.RECIPE_MAIN)
+    return m, oracle.Structure(m).eri4()
+
+
+@pytest.mark.parametrize("perm", [(0, 1, 2, 3), (1, 0, 2, 3), (0, 1, 3, 2), (2, 3, 0, 1), (3, 2, 1, 0)])
+@pytest.mark.parametrize("ls", [(3, 1, 2, 0), (0, 0, 3, 2), (1, 1, 1, 1), (2, 0, 2, 2)])
+def test_eri4_block_orders(lbx, block_case, ls, perm):
+    """Blocks of shells in the caller's order, the side with the higher class first or last."""
+    m, e4 = block_case
+    off = np.concatenate([[0], np.cumsum(2 * m.shells.l + 1)])
+    rng = np.random.default_rng(8)
+    shells = np.stack([rng.choice(np.flatnonzero(m.shells.l == ls[p]), 67) for p in perm], 1).astype(np.int32)
+    got = lbx.Context(m).blocks(shells).cpu().numpy()[:, 0]
+    ref = np.stack([e4[tuple(slice(off[s], off[s + 1]) for s in q)] for q in shells])
+    close(got, ref, floor=1e-13 * np.abs(e4).max() / np.abs(ref).max())
+
+
+@pytest.mark.parametrize("nmain,naux", [(1, 1), (5, 3), (63, 7), (64, 2), (65, 9), (130, 5)])
+def test_ri_jk_sizes(lbx, oracle, nmain, naux):
+    """Density-fitted J and K at sizes around the 64 x 64 tiles and 16-step k loop, against numpy on
+    the library's own eri3 / eri2 (pinned to the oracle elsewhere).  s shells spread over a line, a
+    well-conditioned auxiliary set: 1e-11 of the largest element."""
+    import torch
+    from scipy.linalg import cho_solve, solve_triangular
+    rng = np.random.default_rng(nmain)
+    nat = max(nmain, naux)
+    coords = np.stack([1.5 * np.arange(nat), rng.uniform(0, 1, nat), rng.uniform(0, 1, nat)], 1)
+    main = B.Shells.from_lists([[(0, [0.8], [1.0])] if k < nmain else [] for k in range(nat)])
+    aux = B.Shells.from_lists([[(0, [1.1], [1.0])] if k < naux else [] for k in range(nat)])
+    m = B.Molecule(coords, main, aux)
+    ctx = lbx.Context(m)
+    e3, e2 = ctx.eri3().cpu().numpy(), ctx.eri2().cpu().numpy()
+    D = B.density_from_orbitals(2, nmain, 4, 0.3)
+    L = np.linalg.cholesky(e2)
+    Jr = e3 @ cho_solve((L, True), np.einsum("mnp,mn->p", e3, D))
+    W = solve_triangular(L, e3.reshape(nmain * nmain, naux).T, lower=True).reshape(naux, nmain, nmain)
+    Kr = np.einsum("pmn,nl,pkl->mk", W, D, W, optimize=True)
+    for _ in range(2):
+        J, K = ctx.ri_jk(torch.tensor(D, device="cuda"))
+        close(J.cpu().numpy(), Jr, rel=0.0, floor=1e-11)
+        close(K.cpu().numpy(), Kr, rel=0.0, floor=1e-11)
+    J, _ = ctx.ri_jk(torch.tensor(D, device="cuda"), exchange=False)
+    close(J.cpu().numpy(), Jr, rel=0.0, floor=1e-11)
