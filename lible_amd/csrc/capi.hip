@@ -5,6 +5,7 @@
 #include "quartet.hpp"
 #include "registry.hpp"
 #include "tasks.hpp"
+#include "variant_cost.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -464,69 +465,66 @@ namespace lbx
             return 2 * r;
         }
 
-        // Work estimate of a one-lane-per-quartet variant per quartet, from the primitive-pair
-        // counts (the lane side's as its waves see them, `divergent`; else its mean): ket
-        // transform and Boys + R per primitive quartet (R once per column pass), bra transform per
-        // lane-side primitive pair.
-        double valuCost(const PairClass &lane, const PairClass &unif, int nc, bool divergent = false)
+        // primitive pairs per shell pair of a class, as the time estimates take them
+        cost::Side costSide(const PairClass &pc)
         {
-            const double kmean = lane.n_pairs ? double(lane.n_ppairs) / lane.n_pairs : 1;
-            const double kl = divergent && lane.klane > 0 ? lane.klane : kmean;
-            const double ku = unif.n_pairs ? double(unif.n_ppairs) / unif.n_pairs : 1;
-            const double hl = nHerm(lane.la + lane.lb), hu = nHerm(unif.la + unif.lb);
-            const double sl = nSph(lane.la) * nSph(lane.lb), su = nSph(unif.la) * nSph(unif.lb);
-            const int L = lane.la + lane.lb + unif.la + unif.lb;
-            const double passes = std::ceil(su / nc);
-            return kl * ku * (hl * hu * su + passes * (60 + rFlopsHost(L))) + kl * sl * hl * su;
+            const double kmean = pc.n_pairs ? double(pc.n_ppairs) / pc.n_pairs : 1.0;
+            return {pc.la, pc.lb, kmean, pc.klane > 0 ? pc.klane : 0.5 * (kmean + pc.kmax), std::max<double>(pc.kmax, 1.0)};
         }
 
-        // A one-lane form whose waves wait on their longest lane for more than twice the work the
-        // mean contraction would give (long, uneven contractions on the lane side, as in the
-        // quadruple-zeta bases): for J/K the block form takes the class pair by default, whose
-        // workgroup runs one bra pair's primitives for a block of ket pairs (on def2-QZVP water
-        // clusters 7-25x faster there than the one-lane forms; on the evenly contracted bases
-        // the one-lane forms stay the default).
-        bool laneDivergent(const PairClass &lane, const PairClass &unif, int nc)
+        // Estimated time (ms) of one form over `quartets` quartets, which a one-lane form takes in
+        // `waves` tasks.
+        double variantTime(int mode, const PairClass &bra, const PairClass &ket, const KernelSlot &s, bool f32,
+                           double quartets, double waves)
         {
-            return valuCost(lane, unif, nc, true) > 2.0 * valuCost(lane, unif, nc);
+            const cost::Side b = costSide(bra), k = costSide(ket);
+            if (s.kind == KIND_LANE)
+                return cost::laneForm(s.swap ? k : b, s.swap ? b : k, s.nc, f32, waves, mode == MODE_JK);
+            return s.kind == KIND_WAVE ? cost::waveForm(b, k, f32, quartets) : cost::blockForm(b, k, f32, quartets);
         }
 
-        bool lane(const KernelSlot &s) { return s.fn && s.kind == KIND_LANE; }
-
-        // Default variant before tuning: the cheaper one-lane-per-quartet form by the work
-        // estimate (with the lane side's longest-lane contraction); MFMA when no such form fits the
-        // registers; for J/K the block form when the cheaper one-lane form diverges.
-        int defaultVariant(int mode, const PairClass &bra, const PairClass &ket)
+        // The form with the smallest estimate among the FP64 (or FP32) ones, and that estimate; -1
+        // when the class pair has none.  wavesBra, wavesKet: tasks of the one-lane forms with the
+        // bra (ket) pairs on the lanes.
+        int defaultVariant(int mode, const PairClass &bra, const PairClass &ket, bool f32, double quartets,
+                           double wavesBra, double wavesKet, double *ms = nullptr)
         {
-            const KernelSlot &vb = kernelSlot(mode, bra.la, bra.lb, ket.la, ket.lb, VAR_VALU_BRA);
-            const KernelSlot &vk = kernelSlot(mode, bra.la, bra.lb, ket.la, ket.lb, VAR_VALU_KET);
-            double cb = lane(vb) ? valuCost(bra, ket, vb.nc, true) : 1e300;
-            double ck = lane(vk) ? valuCost(ket, bra, vk.nc, true) : 1e300;
-            if (!lane(vb) && !lane(vk))
-                return VAR_MFMA;
-            const bool bra_lanes = cb <= ck;
-            if (mode == MODE_JK && kernelSlot(mode, bra.la, bra.lb, ket.la, ket.lb, VAR_BLOCK).fn &&
-                (bra_lanes ? laneDivergent(bra, ket, vb.nc) : laneDivergent(ket, bra, vk.nc)))
-                return VAR_BLOCK;
-            return bra_lanes ? VAR_VALU_BRA : VAR_VALU_KET;
+            int best = -1;
+            double tBest = 0.0;
+            for (int v = 0; v < N_VARIANTS; v++)
+            {
+                const KernelSlot &s = kernelSlot(mode, bra.la, bra.lb, ket.la, ket.lb, v);
+                const bool laneVariant = v != VAR_MFMA && v != VAR_MFMA32 && v != VAR_BLOCK && v != VAR_BLOCK32;
+                if (!s.fn || isF32Variant(v) != f32 || laneVariant != (s.kind == KIND_LANE))
+                    continue;   // (the one-wave form under a one-lane number is the same kernel)
+                const double t = variantTime(mode, bra, ket, s, f32, quartets, s.swap ? wavesKet : wavesBra);
+                if (best < 0 || t < tBest)
+                {
+                    best = v;
+                    tBest = t;
+                }
+            }
+            if (ms)
+                *ms = tBest;
+            return best;
         }
 
-        // Default for the FP32 tier of a mixed-precision J/K: the cheaper FP32 one-lane form by
-        // the same estimate (the FP32 block form when it diverges), else the FP32 MFMA form, or
-        // -1 when the class has neither (its quartets then stay FP64).
-        int defaultVariant32(const PairClass &bra, const PairClass &ket)
+        // Quartets of class pair (bra, ket) with lo <= Q_ab Q_cd < hi, from up to 64 evenly spaced
+        // ket positions (both classes sorted by Q).
+        double estimateQuartets(const PairClass &bra, const PairClass &ket, bool same, double lo, double hi)
         {
-            const KernelSlot &vb = kernelSlot(MODE_JK, bra.la, bra.lb, ket.la, ket.lb, VAR_VALU_BRA32);
-            const KernelSlot &vk = kernelSlot(MODE_JK, bra.la, bra.lb, ket.la, ket.lb, VAR_VALU_KET32);
-            if (!lane(vb) && !lane(vk))
-                return kernelSlot(MODE_JK, bra.la, bra.lb, ket.la, ket.lb, VAR_MFMA32).fn ? VAR_MFMA32 : -1;
-            double cb = lane(vb) ? valuCost(bra, ket, vb.nc, true) : 1e300;
-            double ck = lane(vk) ? valuCost(ket, bra, vk.nc, true) : 1e300;
-            const bool bra_lanes = cb <= ck;
-            if (kernelSlot(MODE_JK, bra.la, bra.lb, ket.la, ket.lb, VAR_BLOCK32).fn &&
-                (bra_lanes ? laneDivergent(bra, ket, vb.nc) : laneDivergent(ket, bra, vk.nc)))
-                return VAR_BLOCK32;
-            return bra_lanes ? VAR_VALU_BRA32 : VAR_VALU_KET32;
+            if (bra.Qs.empty() || ket.Qs.empty())
+                return double(bra.n_pairs) * ket.n_pairs * (same ? 0.5 : 1.0);
+            const int samples = std::min(64, ket.n_pairs);
+            double n = 0.0;
+            for (int i = 0; i < samples; i++)
+            {
+                const double q = ket.Qs[static_cast<size_t>(i) * ket.n_pairs / samples];
+                const int below = lo > 0 ? firstBelow(bra.Qs, q, lo) : bra.n_pairs;
+                const int above = hi < kNoUpper ? firstBelow(bra.Qs, q, hi) : 0;
+                n += std::max(0, below - above);
+            }
+            return n * ket.n_pairs / samples * (same ? 0.5 : 1.0);
         }
 
         __global__ void toFloatKernel(const double *__restrict__ in, float *__restrict__ out, long long n)
@@ -608,6 +606,16 @@ namespace lbx
             bool same;
             KArgs extra;
         };
+
+        // Whether every pair of main shells has primitive pairs above the screen: the dense drivers
+        // then write every element and need no zeroed output.
+        bool allPairs(const Context &c)
+        {
+            size_t n = 0;
+            for (const auto &pc : c.cls)
+                n += pc.n_pairs;
+            return n == c.shells.size() * (c.shells.size() + 1) / 2;
+        }
 
         // One kernel of a call whose kernels are independent
         struct QueuedLaunch
@@ -744,6 +752,7 @@ namespace lbx
         for (int i = 0; i < pc.n_pairs; i++)
             qs[i] = pc.Q[order[i]];
         pc.order = order;
+        pc.Qs = qs;
         double kl = 0.0;
         for (int b = 0; b < pc.n_pairs; b += 64)
         {
@@ -789,7 +798,13 @@ struct lbx_context : Context
             const PairClass &bra = *job.bra, &ket = *job.ket;
             if (bra.n_pairs == 0 || ket.n_pairs == 0)
                 continue;
-            const KernelSlot &s = slotFor(job.mode, bra, ket, defaultVariant(job.mode, bra, ket));
+            // tasks of a one-lane form: per uniform-side pair, its lane-side pairs in blocks of 64
+            const double nb = bra.n_pairs, nk = ket.n_pairs, half = job.same ? 0.5 : 1.0;
+            const bool diag = job.pairing == Pairing::Diagonal;
+            double ms = 0.0;
+            const int var = defaultVariant(job.mode, bra, ket, false, diag ? nb : half * nb * nk,
+                                           diag ? nb : nk * std::ceil(half * nb / 64), 0.0, &ms);
+            const KernelSlot &s = slotFor(job.mode, bra, ket, var);
             const auto key = std::make_tuple(&bra, &ket, static_cast<int>(job.pairing), job.same, s.width);
             auto it = plain_tasks.find(key);
             if (it == plain_tasks.end())
@@ -799,7 +814,7 @@ struct lbx_context : Context
             a.kind = job.extra.kind;
             a.qout = job.extra.qout;
             a.dout = job.extra.dout;
-            queue.push_back({s.fn, a, it->second.flops});
+            queue.push_back({s.fn, a, ms});
         }
         flushStaged();
         Fan fan(side, stream, queue.size() > 1);
@@ -849,21 +864,44 @@ struct lbx_context : Context
     // this device's scratch array (lbx_eri4_batch_static)
     int *d_scratch = nullptr;
 
-    int variantFor(int i, int j)
+    // the default forms, per class pair, bound range and tier, with their estimated times
+    struct Choice
     {
-        auto it = tuned.find({i, j});
-        return it != tuned.end() ? it->second : defaultVariant(MODE_JK, cls[i], cls[j]);
+        int variant;
+        double ms;
+    };
+    std::map<std::tuple<int, int, double, double, bool>, Choice> defaults;
+
+    Choice defaultFor(int i, int j, double lo, double hi, bool f32)
+    {
+        const auto key = std::make_tuple(i, j, lo, hi, f32);
+        auto it = defaults.find(key);
+        if (it == defaults.end())
+        {
+            const double n = estimateQuartets(cls[i], cls[j], i == j, lo, hi);
+            Choice ch{-1, 0.0};
+            ch.variant = defaultVariant(MODE_JK, cls[i], cls[j], f32, n, std::max(1.0, n / 64), std::max(1.0, n / 64), &ch.ms);
+            it = defaults.emplace(key, ch).first;
+        }
+        return it->second;
     }
 
-    // variant for the small-bound quartets of a mixed build: an FP32 form, or an FP64 one
+    // form of the FP64 quartets of class pair (i, j) with bounds in [lo, hi)
+    int variantFor(int i, int j, double lo, double hi)
+    {
+        auto it = tuned.find({i, j});
+        return it != tuned.end() ? it->second : defaultFor(i, j, lo, hi, false).variant;
+    }
+
+    // form of the small-bound quartets of a mixed build: an FP32 form, or an FP64 one
     // where the class has no FP32 form or tuning found the FP64 form faster
-    int variant32For(int i, int j)
+    int variant32For(int i, int j, double lo, double hi)
     {
         auto it = tuned32.find({i, j});
         if (it != tuned32.end())
             return it->second;
-        const int v = defaultVariant32(cls[i], cls[j]);
-        return v >= 0 ? v : variantFor(i, j);
+        const int v = defaultFor(i, j, lo, hi, true).variant;
+        return v >= 0 ? v : variantFor(i, j, lo, hi);
     }
 
     // Lane side of the one-lane J/K kernels, per pair class: Schwarz-order positions regrouped
@@ -1084,7 +1122,20 @@ struct lbx_context : Context
         auto it = tuned_sum.find({kind, il, iu});
         if (it != tuned_sum.end())
             return it->second;
-        return kernelSlot(MODE_SUM, lane.la, lane.lb, unif.la, unif.lb, VAR_VALU_BRA).fn ? VAR_VALU_BRA : VAR_MFMA;
+        // pairs per molecule on each side
+        std::vector<int> nl(nmol, 0), nu(nmol, 0);
+        for (int m : lane.mol)
+            nl[m]++;
+        for (int m : unif.mol)
+            nu[m]++;
+        double quartets = 0.0, waves = 0.0;
+        const double half = kind == 2 && il == iu ? 0.5 : 1.0;
+        for (int m = 0; m < nmol; m++)
+        {
+            quartets += half * nl[m] * nu[m];
+            waves += nu[m] * std::ceil(half * nl[m] / 64);
+        }
+        return defaultVariant(MODE_SUM, lane, unif, false, quartets, waves, 0.0);
     }
 
     // Times the FP64 sum kernels of every RI class pair (the one-lane form and the MFMA form,
@@ -1181,7 +1232,7 @@ struct lbx_context : Context
                     TaskTable t = buildTasksMol(*this, lane, unif, same, k.width, lo, hi);
                     KArgs a = baseArgs(*this, lane, unif, t, same);
                     a.kind = kind;
-                    launches.push_back({k.fn, a, t.flops});
+                    launches.push_back({k.fn, a, variantTime(MODE_SUM, lane, unif, k, fp32, t.quartets, double(t.ntasks))});
                     n[kind == 3 ? 0 : 1] += t.quartets;
                     n[2] += t.flops;
                     if (fp32)
@@ -1586,7 +1637,8 @@ extern "C"
                            Context &c = *ctx;
                            requireSingle(c, "lbx_eri4");
                            const long long n = static_cast<long long>(c.nbf);
-                           fill(out, n * n * n * n, 0.0, c.stream);
+                           if (!allPairs(c))
+                               fill(out, n * n * n * n, 0.0, c.stream);
                            KArgs extra{};
                            extra.out = out;
                            extra.kind = 4;
@@ -1640,7 +1692,8 @@ extern "C"
                            if (c.shells_aux.empty())
                                throw Error(LBX_ERR_STATE, "eri3(): RI approximation is not enabled");
                            const long long n = static_cast<long long>(c.nbf);
-                           fill(out, n * n * static_cast<long long>(c.nbf_aux), 0.0, c.stream);
+                           if (!allPairs(c))
+                               fill(out, n * n * static_cast<long long>(c.nbf_aux), 0.0, c.stream);
                            KArgs extra{};
                            extra.out = out;
                            extra.kind = 3;
@@ -2118,7 +2171,8 @@ extern "C"
                 st.quartets_fp32 += t.quartets;
             if (!prof_on)
             {
-                queue.push_back({l.fn, l.a, t.flops});
+                const KernelSlot &slot = kernelSlot(MODE_JK, bra.la, bra.lb, ket.la, ket.lb, var);
+                queue.push_back({l.fn, l.a, variantTime(MODE_JK, bra, ket, slot, isF32Variant(var), t.quartets, t.quartets / 64)});
                 return;
             }
             // one class pair at a time on the context stream, an event pair around each
@@ -2154,9 +2208,9 @@ extern "C"
                 const double lo0 = std::max(split, window_lo), hi0 = window_hi;
                 const double lo1 = std::max(schwarz_thresh, window_lo), hi1 = std::min(split, window_hi);
                 if (lo0 < hi0)
-                    launch(i, j, 0, variantFor(i, j), lo0, hi0);
+                    launch(i, j, 0, variantFor(i, j, lo0, hi0), lo0, hi0);
                 if (mixed && lo1 < hi1)
-                    launch(i, j, 1, variant32For(i, j), lo1, hi1);
+                    launch(i, j, 1, variant32For(i, j, lo1, hi1), lo1, hi1);
             }
         flushStaged();
         Fan fan(side, c.stream, queue.size() > 1);

@@ -64,7 +64,8 @@ namespace lbx
         std::vector<int> mol;              // molecule per pair (batched contexts)
         std::vector<int> prim_x, prim_y;   // surviving primitive pair -> primitive of a, of b
         std::vector<double> Q;          // Schwarz factor per pair (pair order)
-        std::vector<int> order;         // sorted by Q descending
+        std::vector<int> order;         // sorted by Q descending (within each molecule)
+        std::vector<double> Qs;         // Q in that order
         // mean over blocks of 64 consecutive sorted pairs of the block's largest primitive-pair
         // count: the primitive loop a wave of a one-lane form runs when its lanes take this class
         // (a wave waits for its longest lane); 0 until the pairs are sorted
