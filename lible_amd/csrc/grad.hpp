@@ -74,19 +74,25 @@ namespace lbx
     constexpr int kGradSlotL1 = 5;
     constexpr LBX_HD bool gradUsesSlots(int la, int lb, int lc, int ld) { return la + lb + lc + ld + 1 <= kGradSlotL1; }
 
-    // MFMAs of a quartet of the one-wave form with two primitive pairs a side when (la lb) takes
-    // the rows
+    // Work of a quartet of the one-wave form when (la lb) takes the rows, in quarters of an MFMA
+    // (64 cycles): per primitive quartet the products S and Q, the sums T (about 7 MFMAs' time per
+    // four row tiles of S) and V (3 per two of Q) and the loop; per row-side primitive Y, U and the
+    // turn of the accumulators; per column tile the weights.  Contraction depths fall with l: 4, 3,
+    // 1, 1 primitives for s, p, d, f.
     constexpr LBX_HD int gradWaveCost(int la, int lb, int lc, int ld)
     {
+        const int depth[5] = {4, 3, 1, 1, 1};
+        const int kb = depth[la] * depth[lb], kk = depth[lc] * depth[ld];
         const int hp = nHerm(la + lb), hp1 = nHerm(la + lb + 1), hq = nHerm(lc + ld);
         const int sp = nSph(la) * nSph(lb), sq = nSph(lc) * nSph(ld);
-        const int nq = ceilDiv(sq, 16);
-        return nq * (4 * (ceilDiv(hp1, 16) * ceilDiv(hq, 4) + ceilDiv(hq, 16) * ceilDiv(hp, 4)) +
-                     2 * (ceilDiv(hp, 16) * ceilDiv(sp, 4) + 3 * ceilDiv(sp, 16) * ceilDiv(hp, 4)));
+        const int tp1 = ceilDiv(hp1, 16), tq = ceilDiv(hq, 16);
+        const int prim = 4 * (tp1 * ceilDiv(hq, 4) + tq * ceilDiv(hp, 4)) + 7 * tp1 + 6 * tq + 12;
+        const int row = 4 * (ceilDiv(hp, 16) * ceilDiv(sp, 4) + 3 * ceilDiv(sp, 16) * ceilDiv(hp, 4)) + 32;
+        return ceilDiv(sq, 16) * (kb * kk * prim + kb * row + 8 * ceilDiv(sp, 4));
     }
 
     // lane side ("bra") chosen for an unordered class pair: in the one-wave form (main shells to f)
-    // the assignment with fewer MFMAs, else the larger Hermite dimension (more lanes in use); ties
+    // the assignment with less work, else the larger Hermite dimension (more lanes in use); ties
     // to the larger class index
     constexpr LBX_HD bool gradLaneFirst(int la, int lb, int lc, int ld)
     {
