@@ -527,6 +527,25 @@ namespace lbx
             return n * ket.n_pairs / samples * (same ? 0.5 : 1.0);
         }
 
+        // E matrices of a class interleaved over the lanes of each block of 64 lane positions
+        // (KArgs::le): perm maps lane position -> position in order
+        template <typename T>
+        __global__ __launch_bounds__(256) void interleaveKernel(const T *__restrict__ in, T *__restrict__ out,
+                                                                const int *order, const int *perm, const int *poff,
+                                                                const int *pcnt, const long long *base, int n, int hs)
+        {
+            const int lane = threadIdx.x & 63;
+            const int pos = 64 * static_cast<int>(blockIdx.x) + lane;
+            const int pair = pos < n ? order[perm[pos]] : -1;
+            const T *src = pair >= 0 ? in + static_cast<size_t>(poff[pair]) * hs : in;
+            const long long own = pair >= 0 ? static_cast<long long>(pcnt[pair]) * hs : 0;
+            const long long rows = (base[blockIdx.x + 1] - base[blockIdx.x]) / 64;
+            T *dst = out + base[blockIdx.x] + lane;
+            for (long long r = 4LL * blockIdx.y + (threadIdx.x >> 6); r < rows; r += 4LL * gridDim.y)
+                if (r < own)
+                    dst[r * 64] = src[r];
+        }
+
         __global__ void toFloatKernel(const double *__restrict__ in, float *__restrict__ out, long long n)
         {
             for (long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
@@ -753,12 +772,17 @@ namespace lbx
             qs[i] = pc.Q[order[i]];
         pc.order = order;
         pc.Qs = qs;
+        // the longest primitive loop of each 64-pair block, in the count order of lanePerm
+        std::vector<int> count(pc.n_pairs), none(pc.n_pairs, 0);
+        for (int i = 0; i < pc.n_pairs; i++)
+            count[i] = -pc.pcnt[order[i]];
+        const tasks::LaneOrder lo = tasks::laneOrder(qs, count, none);
         double kl = 0.0;
         for (int b = 0; b < pc.n_pairs; b += 64)
         {
             int m = 0;
             for (int i = b; i < std::min(b + 64, pc.n_pairs); i++)
-                m = std::max(m, pc.pcnt[order[i]]);
+                m = std::max(m, -count[lo.perm[i]]);
             kl += m;
         }
         pc.klane = kl / ((pc.n_pairs + 63) / 64);
@@ -905,19 +929,20 @@ struct lbx_context : Context
     }
 
     // Lane side of the one-lane J/K kernels, per pair class: Schwarz-order positions regrouped
-    // by shell within half-decade buckets of the Schwarz factor (lane position -> Schwarz-order
-    // position), so that lanes sharing the first shell are adjacent and combine their K updates,
-    // and the range of Schwarz-order positions each 64-lane block holds.
+    // within half-decade buckets of the Schwarz factor (lane position -> Schwarz-order position),
+    // and the range of Schwarz-order positions each 64-lane block holds.  Regrouped by primitive
+    // count when the kernel sums K in LDS, so that a wave's lanes run loops of one length; else by
+    // shell, so that lanes sharing the first shell are adjacent and combine their K updates.
     struct LanePerm
     {
         std::vector<int> perm, bqlo, bqhi;
         int *d_perm = nullptr, *d_bqlo = nullptr, *d_bqhi = nullptr;
     };
-    std::map<int, LanePerm> lane_perm;
+    std::map<std::pair<int, bool>, LanePerm> lane_perm;
 
-    const LanePerm &lanePerm(int idx)
+    const LanePerm &lanePerm(int idx, bool byCount)
     {
-        auto it = lane_perm.find(idx);
+        auto it = lane_perm.find({idx, byCount});
         if (it != lane_perm.end())
             return it->second;
         const PairClass &pc = cls[idx];
@@ -927,8 +952,9 @@ struct lbx_context : Context
         for (int p = 0; p < n; p++)
         {
             qs[p] = pc.Q.empty() ? 1.0 : pc.Q[pc.order[p]];
-            sa[p] = pc.sh_a[pc.order[p]];
-            sb[p] = pc.sh_b[pc.order[p]];
+            // longest primitive loops first
+            sa[p] = byCount ? -pc.pcnt[pc.order[p]] : pc.sh_a[pc.order[p]];
+            sb[p] = byCount ? 0 : pc.sh_b[pc.order[p]];
         }
         tasks::LaneOrder lo = tasks::laneOrder(qs, sa, sb);
         LanePerm lp;
@@ -939,7 +965,109 @@ struct lbx_context : Context
         lp.d_bqlo = stage(lp.bqlo);
         lp.d_bqhi = stage(lp.bqhi);
         lp.perm = std::move(perm);
-        return lane_perm.emplace(idx, std::move(lp)).first->second;
+        return lane_perm.emplace(std::make_pair(idx, byCount), std::move(lp)).first->second;
+    }
+
+    // Lane-interleaved E matrices (KArgs::le) per lane order and use (bra or ket).  The orders are
+    // made after the Schwarz order, which stays for the context's life.
+    struct LaneE
+    {
+        long long *base = nullptr;
+        double *e = nullptr;
+        float *e32 = nullptr;
+    };
+    std::map<std::pair<const LanePerm *, bool>, LaneE> lane_e;
+
+    // le / le32 / lbase of a lane side; the interleaved copies are made on first use
+    void setLaneE(KArgs &a, const PairClass &pc, bool ket, const LanePerm &lp, bool f32)
+    {
+        LaneE &le = lane_e[{&lp, ket}];
+        const int hs = nHerm(pc.la + pc.lb) * nSph(pc.la) * nSph(pc.lb), nblk = (pc.n_pairs + 63) / 64;
+        std::vector<long long> base(nblk + 1, 0);
+        if (f32 ? !le.e32 : !le.e)
+        {
+            for (int b = 0; b < nblk; b++)
+            {
+                int k = 0;
+                for (int p = 64 * b; p < std::min(64 * b + 64, pc.n_pairs); p++)
+                    k = std::max(k, pc.pcnt[pc.order[lp.perm[p]]]);
+                base[b + 1] = base[b] + 64LL * k * hs;
+            }
+            if (!le.base)
+                le.base = upload(base);
+            flushStaged();   // lp's arrays
+            const dim3 grid(nblk, 16);
+            auto run = [&](auto *out, auto *in) {
+                using T = std::remove_reference_t<decltype(*out)>;
+                hipLaunchKernelGGL(interleaveKernel<T>, grid, dim3(256), 0, stream, in, out, pc.d_order, lp.d_perm,
+                                   pc.d_poff, pc.d_pcnt, le.base, pc.n_pairs, hs);
+                LBX_HIP(hipGetLastError());
+            };
+            if (f32)
+            {
+                float *e = alloc<float>(base[nblk]);
+                run(e, ket ? pc.d_ek32 : pc.d_eb32);
+                le.e32 = e;
+            }
+            else
+            {
+                double *e = alloc<double>(base[nblk]);
+                run(e, ket ? pc.d_ek : pc.d_eb);
+                le.e = e;
+            }
+        }
+        a.le = le.e;
+        a.le32 = le.e32;
+        a.lbase = le.base;
+    }
+
+    // Columns of the K rows that the one-lane kernels sum in LDS, per lane-side class: the functions
+    // of its shells' angular momenta (KArgs::kcol_a ..)
+    struct KCols
+    {
+        int *d_a = nullptr, *d_b = nullptr, *d_ao = nullptr;
+        int n = 0;
+    };
+    std::map<int, KCols> k_cols;
+
+    int kColumns(const PairClass &pc) const
+    {
+        int n = 0;
+        for (const auto &s : shells)
+            n += (s.l == pc.la || s.l == pc.lb) ? nSph(s.l) : 0;
+        return n;
+    }
+
+    const KCols &kCols(int idx)
+    {
+        auto it = k_cols.find(idx);
+        if (it != k_cols.end())
+            return it->second;
+        const PairClass &pc = cls[idx];
+        std::vector<int> col(shells.size(), 0), ao, a(pc.n_pairs), b(pc.n_pairs);
+        for (int l : {pc.la, pc.lb})
+        {
+            for (size_t s = 0; s < shells.size(); s++)
+                if (shells[s].l == l)
+                {
+                    col[s] = static_cast<int>(ao.size());
+                    for (int m = 0; m < nSph(l); m++)
+                        ao.push_back(static_cast<int>(shells[s].ao) + m);
+                }
+            if (pc.la == pc.lb)
+                break;
+        }
+        for (int p = 0; p < pc.n_pairs; p++)
+        {
+            a[p] = col[pc.sh_a[p]];
+            b[p] = col[pc.sh_b[p]];
+        }
+        KCols k;
+        k.d_a = stage(a);
+        k.d_b = stage(b);
+        k.d_ao = stage(ao);
+        k.n = static_cast<int>(ao.size());
+        return k_cols.emplace(idx, k).first->second;
     }
 
     // The J/K kernel of class pair (i >= j) with the given variant, its arguments over the
@@ -986,7 +1114,14 @@ struct lbx_context : Context
             while (gshift < 6 && groupBytes * (2 << gshift) <= double(1 << 20))
                 gshift++;
         }
-        const LanePerm *lp = blockMajor && nlane > 0 ? &lanePerm(s.swap ? j : i) : nullptr;
+        // K rows of the uniform pair in LDS: up to 64 KiB, and at least three lane blocks to share
+        // them (a workgroup's four waves take four blocks of a group); else K by atomics alone, which
+        // bound the classes of low angular momentum (16 updates per (ps|ps) quartet at 23 G/s)
+        const PairClass &uside = s.swap ? bra : ket;
+        const bool kLds = blockMajor && nlane > 128 && (nSph(uside.la) + nSph(uside.lb)) * kColumns(lside) * 8 <= 65536;
+        if (kLds)
+            gshift = std::max(gshift, 2);
+        const LanePerm *lp = blockMajor && nlane > 0 ? &lanePerm(s.swap ? j : i, kLds) : nullptr;
         if (blockMajor && it->second.nblk == 0 && nlane > 0)
             buildBlockMajor(*this, it->second, nlane, 1, gshift, lp->perm, lp->bqlo, lp->bqhi);
         const TaskTable &t = it->second;
@@ -1006,6 +1141,15 @@ struct lbx_context : Context
             a.bprefix = t.d_bprefix;
             a.bq0 = t.d_bq0;
             a.ntasks = t.btasks;
+            setLaneE(a, lside, s.swap, *lp, isF32Variant(var));
+            if (kLds)
+            {
+                const KCols &k = kCols(s.swap ? j : i);
+                a.kcol_a = k.d_a;
+                a.kcol_b = k.d_b;
+                a.kao = k.d_ao;
+                a.kcols = k.n;
+            }
         }
         if (sample_quartets > 0 && a.block_major)
         {

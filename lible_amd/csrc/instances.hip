@@ -1,6 +1,6 @@
 // Instantiation unit of the quartet kernels.  Compiled once per LBX_UNIT:
 //   0..9   bra = main pair class LBX_UNIT (order (0,0),(1,0),(1,1),(2,0),...): eri4 J/K (FP64
-//          forms) and dense for every ket class <= bra class, the (ab|ab) diagonal, and eri3
+//          forms) and dense for every ket class <= bra class, and eri3
 //          (ab|c) against every auxiliary shell l = 0..5 not already covered;
 //   10, 11 bra = single auxiliary shell l = 4, 5: eri2 (a|b) for b <= l and the (a|a) diagonal;
 //   12..23 the FP32 forms of units 0..11: J/K and the batched RI sums.
@@ -104,8 +104,6 @@ namespace lbx
                 regEri2<3>();
                 regEri2<4>();
                 regEri2<5>();
-                if constexpr (mine(0) && !kF32Unit)
-                    registerQuartet<PA, PB, PA, PB, MODE_DIAG, 1>();
             }
         } registrar;
     }

@@ -23,7 +23,8 @@
 //             holds rows 4c..4c+3 across the lane groups, which is exactly the A-operand layout
 //             of K-chunk c.  R is built cooperatively in LDS.  Used where R alone would not fit
 //             a lane's registers (high total angular momentum).
-// Epilogues: J/K contraction with atomics, dense tensor scatter, or the (ab|ab) diagonal.
+// Epilogues: J/K contraction with atomics, dense tensor scatter, per-molecule sums, or (one-wave
+// form) the (ab|ab) diagonal and listed blocks.
 #pragma once
 
 #include <algorithm>
@@ -81,6 +82,18 @@ namespace lbx
         // MODE_DIAG
         double *qout;   // sqrt(max |(ab|ab)|) per pair (pair order)
         double *dout;   // (mn|mn) matrix (pair classes) or vector (single classes), may be null
+        // quartetV: the lane side's E matrices interleaved over the 64 lanes of a block, so that the
+        // lanes' loads of one element are one contiguous run (a pair's own matrix is contiguous: 64
+        // lanes would touch 64 lines per element, ~100 cycles a load against 4 an FMA): element e of
+        // primitive i of lane position pos at lbase[pos / 64] + (i H S + e) 64 + pos % 64
+        const double *le;
+        const float *le32;
+        const long long *lbase;
+        // J/K of quartetV with K rows in LDS (kcols > 0): column of the first function of each
+        // lane-side pair's shells a and b among the functions of their angular momenta, the AO of
+        // each column, and the number of columns
+        const int *kcol_a, *kcol_b, *kao;
+        int kcols;
     };
 
     constexpr LBX_HD int rFlops(int L)
@@ -217,6 +230,11 @@ namespace lbx
         return r;
     }
 
+    __device__ __forceinline__ void ldsAdd(double *p, double v)
+    {
+        __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+
     // Adds v of every lane of a run into one address, by the run's head lane (all lanes call).
     __device__ __forceinline__ void runAtomicAdd(const LaneRuns &r, double *addr, double v)
     {
@@ -245,19 +263,46 @@ namespace lbx
         }
     }
 
+    // Elements h * S + s of a pair's E matrix, without the structural zeros when SKIP
+    template <int La, int Lb, bool SKIP>
+    struct EList
+    {
+        static constexpr int S = nSph(La) * nSph(Lb), N = nHerm(La + Lb) * S;
+        int n = 0;
+        int e[N]{};
+        constexpr EList()
+        {
+            constexpr EPattern<La, Lb> P{};
+            for (int i = 0; i < N; i++)
+                if (!SKIP || P.nz[i / S][i % S])
+                    e[n++] = i;
+        }
+    };
+
+    template <int N, typename F, int... I>
+    __device__ __forceinline__ void forEachIntImpl(F &&f, std::integer_sequence<int, I...>)
+    {
+        (f(std::integral_constant<int, I>{}), ...);
+    }
+    template <int N, typename F>
+    __device__ __forceinline__ void forEachInt(F &&f)
+    {
+        forEachIntImpl<N>(f, std::make_integer_sequence<int, N>{});
+    }
+
     // ------------------------------------------------------------------------------- quartetV
     // One quartet per lane: lane-side pair l (64 consecutive sorted positions) against the
     // wave-uniform pair u.  SWAP = false: lanes = bra, u = ket; SWAP = true: lanes = ket, u = bra.
     // T: type of R, the E matrices and both transforms (double; float for the reduced-precision
     // J/K quartets, whose Boys values, epilogue and accumulation stay double).
     // jl (J/K only, SL entries per lane): this lane's J contributions to its lane-side pair,
-    // scaled by 2f.  CARRY = false: zeroed here and added to J at the end of the task; CARRY =
-    // true: accumulated into the caller's array, which adds it to J once for a run of tasks that
-    // share the lane-side pairs.
+    // scaled by 2f, accumulated over a run of tasks that share the lane-side pairs and added to J
+    // by the caller at its end.
     // MODE_SUM: the lane's weighted sums of |value| and value are added to jl[0] and jl[1], which
     // the caller adds to the molecule's sums once for a run of tasks of one molecule.
-    template <int LA, int LB, int LC, int LD, int MODE, bool SWAP, typename T, bool CARRY = false>
-    __device__ __forceinline__ void quartetVTask(const KArgs &A, int q, int local, int lane, double *jl)
+    template <int LA, int LB, int LC, int LD, int MODE, bool SWAP, typename T>
+    __device__ __forceinline__ void quartetVTask(const KArgs &A, int q, int local, int lane, double *jl,
+                                                 double *sK = nullptr)
     {
         using C = Cls<LA, LB, LC, LD>;
         constexpr int L = C::L, HL = C::HL;
@@ -302,16 +347,23 @@ namespace lbx
         if constexpr (F32)
         {
             eUb = SWAP ? UP.eb32 : UP.ek32;
-            eLb = SWAP ? LP.ek32 : LP.eb32;
+            eLb = MODE == MODE_JK ? A.le32 : LP.eb32;
         }
         else
         {
             eUb = SWAP ? UP.eb : UP.ek;
-            eLb = SWAP ? LP.ek : LP.eb;
+            eLb = MODE == MODE_JK ? A.le : LP.eb;
         }
         const cptr<T> eU = constView(eUb + static_cast<size_t>(upoff) * HU * SU);
         const cptr<double> ppU = constView(reinterpret_cast<const double *>(UP.pp + upoff));
-        const T *__restrict__ eL = eLb + static_cast<size_t>(lpoff) * HLn * SL;
+        // the lane side's E: J/K interleaved over the block's lanes (wave-uniform base + lane), the
+        // other modes, whose lanes are not aligned to the blocks, as stored
+        constexpr int ES = MODE == MODE_JK ? 64 : 1;
+        const T *__restrict__ eL;
+        if constexpr (MODE == MODE_JK)
+            eL = eLb + uniform(A.lbase[local >> 6]);
+        else
+            eL = eLb + static_cast<size_t>(lpoff) * HLn * SL;
 
         const int l0 = active ? LP.ao_a[l] : 0, l1 = active ? LP.ao_b[l] : 0;
         const int u0 = uniform(UP.ao_a[u]), u1 = uniform(UP.ao_b[u]);
@@ -329,28 +381,44 @@ namespace lbx
         }
         const long long n = A.nbf;
         const double *D = A.D;
-        // K updates on the columns of the lane pair's first shell: with a shell-ordered lane side
-        // the lanes of one shell add their sum once (runs of adjacent lanes), else each lane
-        // adds its own
+        // K rows of the uniform pair's functions (r: first shell 0 .. SUa - 1, then the second) on the
+        // columns of the lane pair's shells: summed in LDS over the workgroup's lanes (kcols > 0),
+        // else added to K, where with a shell-ordered lane side the lanes of one first shell add
+        // their sum once (runs of adjacent lanes)
         LaneRuns runs{};
-        int la0 = l0;
+        int la0 = l0, ca = 0, cb = 0;
         if constexpr (MODE == MODE_JK)
-            if (permuted)
+        {
+            if (A.kcols > 0)
+            {
+                ca = A.kcol_a[l];
+                cb = A.kcol_b[l];
+            }
+            else if (permuted)
             {
                 la0 = LP.ao_a[l];
                 runs = laneRuns(la0, active, lane);
             }
-        auto addA = [&](long long row, int al, double v) {
-            if (permuted)
+        }
+        auto addA = [&](int r, long long row, int al, double v) {
+            if (A.kcols > 0)
+            {
+                if (active)
+                    ldsAdd(&sK[r * A.kcols + ca + al], v);
+            }
+            else if (permuted)
                 runAtomicAdd(runs, &A.K[row * n + la0 + al], v);
             else if (active)
                 unsafeAtomicAdd(&A.K[row * n + l0 + al], v);
         };
-        if constexpr (MODE == MODE_JK && !CARRY)
-#pragma unroll
-            for (int s = 0; s < SL; s++)
-                jl[s] = 0.0;
-        double dmax = 0.0;
+        auto addB = [&](int r, long long row, int be, double v) {
+            if (!active)
+                return;
+            if (A.kcols > 0)
+                ldsAdd(&sK[r * A.kcols + cb + be], v);
+            else
+                unsafeAtomicAdd(&A.K[row * n + l1 + be], v);
+        };
         double sabs = 0.0, ssum = 0.0;   // MODE_SUM
 
         // Passes stay a runtime loop (unrolling them lets the compiler overlap the live ranges of
@@ -409,27 +477,76 @@ namespace lbx
                                     X[h * NC + c] = fma(r, ek[g * SU + pass * NC + c], X[h * NC + c]);
                         }
                 }
-                const T *el = eL + static_cast<size_t>(i) * HLn * SL;
-                // structural zeros of the lane side's E (about half the entries) are skipped
-                constexpr EPattern<La, Lb> PL{};
+                // Elements of the lane side's E (about half are structural zeros, skipped) in groups,
+                // the next group's loads in flight over this one's FMAs: left to itself the compiler
+                // waits for each load before it issues the next.  The two groups take the registers
+                // that R held.
+                typedef const T __attribute__((address_space(1))) *Row;
+                constexpr EList<La, Lb, kSkipL> EL{};
+                constexpr int G = (HL + L) / 2 < 2 ? 2 : ((HL + L) / 2 > 16 ? 16 : (HL + L) / 2);
+                constexpr int NG = ceilDiv(EL.n, G);
+                T eb[2][G];
+                auto load = [&](auto gC) {
+                    constexpr int g = decltype(gC)::value;
+                    // J/K: the group's (uniform) address anew, else all of them are formed ahead
+                    Row er = (Row)(eL + (static_cast<size_t>(i) * (HLn * SL) + EL.e[g * G]) * ES);
+                    if constexpr (MODE == MODE_JK)
+                        asm("" : "+s"(er));
 #pragma unroll
-                for (int h = 0; h < HLn; h++)
+                    for (int j = 0; j < G; j++)
+                        if (g * G + j < EL.n)
+                            eb[g & 1][j] = er[(EL.e[g * G + j] - EL.e[g * G]) * ES + (MODE == MODE_JK ? lane : 0)];
+                };
+                load(std::integral_constant<int, 0>{});
+                forEachInt<NG>([&](auto gC) {
+                    constexpr int g = decltype(gC)::value;
+                    if constexpr (g + 1 < NG)
+                        load(std::integral_constant<int, g + 1>{});
+                    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int s = 0; s < SL; s++)
-                    {
-                        if (kSkipL && !PL.nz[h][s])
-                            continue;
-                        const T e = el[h * SL + s];
+                    for (int j = 0; j < G; j++)
+                        if (g * G + j < EL.n)
+                        {
+                            const int h = EL.e[g * G + j] / SL, s = EL.e[g * G + j] % SL;
 #pragma unroll
-                        for (int c = 0; c < NC; c++)
-                            I[s * NC + c] = fma(e, X[h * NC + c], I[s * NC + c]);
-                    }
+                            for (int c = 0; c < NC; c++)
+                                I[s * NC + c] = fma(eb[g & 1][j], X[h * NC + c], I[s * NC + c]);
+                        }
+                    __builtin_amdgcn_sched_barrier(0);
+                });
             }
 
             // ---- epilogue for the columns of this pass: I[s][c] = (l s | u pass*NC + c)
             if constexpr (MODE == MODE_JK)
             {
+                // The lanes' density blocks once per pass, into the registers that X and R held: read
+                // where they are used they are read again for every component of the other shells
+                // (the additions in between may alias them), a line per lane each time.
+                auto readD = [&](auto &d, auto rows, auto cols, auto &&at, auto &&wanted) {
+#pragma unroll
+                    for (int r = 0; r < decltype(rows)::value; r++)
+#pragma unroll
+                        for (int c = 0; c < decltype(cols)::value; c++)
+                            if (wanted(r))
+                                d[r * decltype(cols)::value + c] = at(r, c);
+                    __builtin_amdgcn_sched_barrier(0);
+                };
+                using ia = std::integral_constant<int, SLa>;
+                using ib = std::integral_constant<int, SLb>;
+                using ua = std::integral_constant<int, SUa>;
+                using ub = std::integral_constant<int, SUb>;
+                auto every = [](int) { return true; };
+                // first index ga of some column of this pass
+                auto inPass = [&](int ga) {
+                    bool any = false;
+#pragma unroll
+                    for (int de = 0; de < SUb; de++)
+                        any |= (ga * SUb + de) / NC == pass;
+                    return any;
+                };
                 // J_l += 2f I D_u (accumulated over passes); J_u += 2f I^T D_l (wave sum)
+                double dl[SL];
+                readD(dl, ia{}, ib{}, [&](int al, int be) { return active ? D[(l0 + al) * n + l1 + be] : 0.0; }, every);
 #pragma unroll
                 for (int c = 0; c < NC; c++)
                 {
@@ -442,10 +559,9 @@ namespace lbx
 #pragma unroll
                     for (int s = 0; s < SL; s++)
                     {
-                        const int al = s / SLb, be = s % SLb;
                         const double iv = I[s * NC + c];
                         jl[s] = fma(iv, du, jl[s]);
-                        ju = fma(iv, active ? D[(l0 + al) * n + l1 + be] : 0.0, ju);
+                        ju = fma(iv, dl[s], ju);
                     }
                     ju = waveSum(2.0 * f * ju);
                     if (lane == 0)
@@ -460,15 +576,13 @@ namespace lbx
                     // unique-quartet contributions are symmetrised at the end (K + K^T), so
                     // either triangle may receive them, and with the row fixed across the wave
                     // its atomics and loads stay on a few rows that remain in L2.
+                    double dbb[SUb * SLb], dba[SUb * SLa];   // D[u1 + de][l1 + be], D[u1 + de][l0 + al]
+                    readD(dbb, ub{}, ib{}, [&](int de, int be) { return D[(u1 + de) * n + l1 + be]; }, every);
+                    readD(dba, ub{}, ia{}, [&](int de, int al) { return D[(u1 + de) * n + l0 + al]; }, every);
 #pragma unroll
                     for (int ga = 0; ga < SUa; ga++)
                     {
-                        // columns of this pass with first index ga
-                        bool any = false;
-#pragma unroll
-                        for (int de = 0; de < SUb; de++)
-                            any |= (ga * SUb + de) / NC == pass;
-                        if (!any)
+                        if (!inPass(ga))
                             continue;
 #pragma unroll
                         for (int al = 0; al < SLa; al++)
@@ -483,9 +597,9 @@ namespace lbx
                                     if (su / NC != pass)
                                         continue;
                                     s = fma(double(I[(al * SLb + be) * NC + su % NC]),
-                                            D[(u1 + de) * n + l1 + be], s);
+                                            dbb[de * SLb + be], s);
                                 }
-                            addA(u0 + ga, al, f * s);
+                            addA(ga, u0 + ga, al, f * s);
                         }
 #pragma unroll
                         for (int be = 0; be < SLb; be++)
@@ -500,12 +614,14 @@ namespace lbx
                                     if (su / NC != pass)
                                         continue;
                                     s = fma(double(I[(al * SLb + be) * NC + su % NC]),
-                                            D[(u1 + de) * n + l0 + al], s);
+                                            dba[de * SLa + al], s);
                                 }
-                            if (active)
-                                unsafeAtomicAdd(&A.K[(u0 + ga) * n + l1 + be], f * s);
+                            addB(ga, u0 + ga, be, f * s);
                         }
                     }
+                    double dab[SUa * SLb], daa[SUa * SLa];   // D[u0 + ga][l1 + be], D[u0 + ga][l0 + al]
+                    readD(dab, ua{}, ib{}, [&](int ga, int be) { return D[(u0 + ga) * n + l1 + be]; }, inPass);
+                    readD(daa, ua{}, ia{}, [&](int ga, int al) { return D[(u0 + ga) * n + l0 + al]; }, inPass);
 #pragma unroll
                     for (int de = 0; de < SUb; de++)
                     {
@@ -528,9 +644,9 @@ namespace lbx
                                     if (su / NC != pass)
                                         continue;
                                     s = fma(double(I[(al * SLb + be) * NC + su % NC]),
-                                            D[(u0 + ga) * n + l1 + be], s);
+                                            dab[ga * SLb + be], s);
                                 }
-                            addA(u1 + de, al, f * s);
+                            addA(SUa + de, u1 + de, al, f * s);
                         }
 #pragma unroll
                         for (int be = 0; be < SLb; be++)
@@ -545,10 +661,9 @@ namespace lbx
                                     if (su / NC != pass)
                                         continue;
                                     s = fma(double(I[(al * SLb + be) * NC + su % NC]),
-                                            D[(u0 + ga) * n + l0 + al], s);
+                                            daa[ga * SLa + al], s);
                                 }
-                            if (active)
-                                unsafeAtomicAdd(&A.K[(u1 + de) * n + l1 + be], f * s);
+                            addB(SUa + de, u1 + de, be, f * s);
                         }
                     }
                 }
@@ -564,9 +679,9 @@ namespace lbx
                             if (pass * NC + c < SU)
                                 denseStore<C>(A, I[s * NC + c], s, pass * NC + c, l0, l1, u0, u1);
             }
-            else if constexpr (MODE == MODE_SUM)
+            else
             {
-                static_assert(!SWAP, "sums keep the bra on the lanes");
+                static_assert(MODE == MODE_SUM && !SWAP, "sums keep the bra on the lanes");
                 if (active)
 #pragma unroll
                     for (int s = 0; s < SL; s++)
@@ -579,48 +694,10 @@ namespace lbx
                                 ssum += v;
                             }
             }
-            else
-            {
-                static_assert(MODE != MODE_DIAG || (LA == LC && LB == LD && !SWAP),
-                              "diagonal needs ab == cd");
-                if (active)
-#pragma unroll
-                    for (int c = 0; c < NC; c++)
-                    {
-                        const int s = pass * NC + c;
-                        if (s >= SU)
-                            continue;
-                        const double v = I[s * NC + c];
-                        dmax = fmax(dmax, fabs(v));
-                        if (A.dout)
-                        {
-                            const int mu = s / SLb, nu = s % SLb;
-                            if (A.kind == 2)
-                                A.dout[l0 + mu] = v;
-                            else
-                            {
-                                A.dout[(l0 + mu) * A.nbf + l1 + nu] = v;
-                                A.dout[(l1 + nu) * A.nbf + l0 + mu] = v;
-                            }
-                        }
-                    }
-            }
         };
         forEachPass<NPASS>(passBody);
 
-        if constexpr (MODE == MODE_JK && !CARRY)
-        {
-            if (active)
-#pragma unroll
-                for (int s = 0; s < SL; s++)
-                    unsafeAtomicAdd(&A.J[(l0 + s / SLb) * n + l1 + s % SLb], jl[s]);
-        }
-        else if constexpr (MODE == MODE_DIAG)
-        {
-            if (active)
-                A.qout[l] = sqrt(dmax);
-        }
-        else if constexpr (MODE == MODE_SUM)
+        if constexpr (MODE == MODE_SUM)
         {
             // images in the dense tensor: (ab|P) and (ba|P) for distinct shells; (P|Q), (Q|P)
             const bool one = A.kind == 3 ? LP.sh_a[l] == LP.sh_b[l] : (A.same_class && p == q);
@@ -650,82 +727,114 @@ namespace lbx
         double jl[MODE == MODE_SUM ? 2 : SL];
         if constexpr (MODE == MODE_JK)
         {
-            if (A.block_major)
-            {
-                const DPairs &LP = SWAP ? A.ket : A.bra;
-                auto flushJ = [&](int b) {
-                    const int p = 64 * b + lane;
-                    if (p < LP.n)
-                    {
-                        const int l = LP.order[A.lperm ? A.lperm[p] : p];
-                        const long long r0 = LP.ao_a[l], r1 = LP.ao_b[l];
-#pragma unroll
-                        for (int s = 0; s < SL; s++)
-                            unsafeAtomicAdd(&A.J[(r0 + s / SLb) * A.nbf + r1 + s % SLb], jl[s]);
-                    }
-                };
-                const int gs = A.gshift;
-                const int ng = (A.nblk + (1 << gs) - 1) >> gs;
-                int g = 0, q0 = 0, b = -1;
-                long long base = 0, next = 0;
-                for (long long t = w; t < A.ntasks; t += nw)
+            const DPairs &LP = SWAP ? A.ket : A.bra;
+            auto flushJ = [&](int b) {
+                const int p = 64 * b + lane;
+                if (p < LP.n)
                 {
-                    if (t >= next)
-                    {
-                        g = uniform(findKet(A.bprefix, ng, t));
-                        base = A.bprefix[g];
-                        next = A.bprefix[g + 1];
-                        q0 = uniform(A.bq0[g]);
-                    }
-                    const long long local = t - base;
-                    const int bt = (g << gs) + static_cast<int>(local & ((1LL << gs) - 1));
-                    if (bt != b)
-                    {
-                        if (b >= 0)
-                            flushJ(b);
+                    const int l = LP.order[A.lperm ? A.lperm[p] : p];
+                    const long long r0 = LP.ao_a[l], r1 = LP.ao_b[l];
 #pragma unroll
-                        for (int s = 0; s < SL; s++)
-                            jl[s] = 0.0;
-                        b = bt;
-                    }
-                    quartetVTask<LA, LB, LC, LD, MODE, SWAP, T, true>(A, q0 + static_cast<int>(local >> gs), 64 * b,
-                                                                      lane, jl);
+                    for (int s = 0; s < SL; s++)
+                        unsafeAtomicAdd(&A.J[(r0 + s / SLb) * A.nbf + r1 + s % SLb], jl[s]);
                 }
-                if (b >= 0)
-                    flushJ(b);
-                return;
-            }
-        }
-        const long long t0 = A.ntasks * w / nw, t1 = A.ntasks * (w + 1) / nw;
-        if (t0 >= t1)
-            return;
-        int q = uniform(findKet(A.prefix, A.nket, t0));
-        long long base = A.prefix[q], next = A.prefix[q + 1];
-        int mol = -1;   // MODE_SUM: the molecule of the sums in jl
-        for (long long t = t0; t < t1; t++)
-        {
-            while (t >= next)
+            };
+            const int gs = A.gshift;
+            const int ng = (A.nblk + (1 << gs) - 1) >> gs;
+            int g = 0, q0 = 0, b = -1;
+            long long base = 0, next = 0;
+            // K rows in LDS: the workgroup's four waves take four blocks of one uniform pair
+            // (G >= 4), so after each round of tasks its rows are complete and go to K
+            extern __shared__ double sKrows[];
+            constexpr int SUa = nSph(SWAP ? LA : LC), SUb = nSph(SWAP ? LB : LD);
+            const int nK = (SUa + SUb) * A.kcols;
+            if (A.kcols > 0)
             {
-                q++;
-                base = next;
-                next = A.prefix[q + 1];
+                for (int e = threadIdx.x; e < nK; e += 256)
+                    sKrows[e] = 0.0;
+                __syncthreads();
+            }
+            for (long long t = w; t < A.ntasks; t += nw)
+            {
+                if (t >= next)
+                {
+                    g = uniform(findKet(A.bprefix, ng, t));
+                    base = A.bprefix[g];
+                    next = A.bprefix[g + 1];
+                    q0 = uniform(A.bq0[g]);
+                }
+                const long long local = t - base;
+                const int bt = (g << gs) + static_cast<int>(local & ((1LL << gs) - 1));
+                const int q = q0 + static_cast<int>(local >> gs);
+                if (bt != b)
+                {
+                    if (b >= 0)
+                        flushJ(b);
+#pragma unroll
+                    for (int s = 0; s < SL; s++)
+                        jl[s] = 0.0;
+                    b = bt;
+                }
+                quartetVTask<LA, LB, LC, LD, MODE, SWAP, T>(A, q, 64 * b, lane, jl, sKrows);
+                if (A.kcols > 0)
+                {
+                    __syncthreads();
+                    const DPairs &UP = SWAP ? A.bra : A.ket;
+                    const int u = uniform(UP.order[q]);
+                    const long long u0 = uniform(UP.ao_a[u]), u1 = uniform(UP.ao_b[u]);
+                    for (int r = 0; r < SUa + SUb; r++)
+                    {
+                        double *row = A.K + (r < SUa ? u0 + r : u1 + r - SUa) * A.nbf;
+                        for (int e = threadIdx.x; e < A.kcols; e += 256)
+                        {
+                            const double v = sKrows[r * A.kcols + e];
+                            if (v != 0.0)
+                            {
+                                sKrows[r * A.kcols + e] = 0.0;
+                                unsafeAtomicAdd(row + A.kao[e], v);
+                            }
+                        }
+                    }
+                    __syncthreads();
+                }
+            }
+            if (b >= 0)
+                flushJ(b);
+            return;
+        }
+        else
+        {
+            const long long t0 = A.ntasks * w / nw, t1 = A.ntasks * (w + 1) / nw;
+            if (t0 >= t1)
+                return;
+            int q = uniform(findKet(A.prefix, A.nket, t0));
+            long long base = A.prefix[q], next = A.prefix[q + 1];
+            int mol = -1;   // MODE_SUM: the molecule of the sums in jl
+            for (long long t = t0; t < t1; t++)
+            {
+                while (t >= next)
+                {
+                    q++;
+                    base = next;
+                    next = A.prefix[q + 1];
+                }
+                if constexpr (MODE == MODE_SUM)
+                {
+                    const int m = uniform(A.ket.mol[A.ket.order[q]]);
+                    if (m != mol)
+                    {
+                        if (mol >= 0)
+                            flushSums(A, mol, lane, jl[0], jl[1]);
+                        mol = m;
+                        jl[0] = jl[1] = 0.0;
+                    }
+                }
+                quartetVTask<LA, LB, LC, LD, MODE, SWAP, T>(A, q, uniform(A.plo[q]) + 64 * static_cast<int>(t - base),
+                                                            lane, jl);
             }
             if constexpr (MODE == MODE_SUM)
-            {
-                const int m = uniform(A.ket.mol[A.ket.order[q]]);
-                if (m != mol)
-                {
-                    if (mol >= 0)
-                        flushSums(A, mol, lane, jl[0], jl[1]);
-                    mol = m;
-                    jl[0] = jl[1] = 0.0;
-                }
-            }
-            quartetVTask<LA, LB, LC, LD, MODE, SWAP, T>(A, q, uniform(A.plo[q]) + 64 * static_cast<int>(t - base),
-                                                        lane, jl);
+                flushSums(A, mol, lane, jl[0], jl[1]);
         }
-        if constexpr (MODE == MODE_SUM)
-            flushSums(A, mol, lane, jl[0], jl[1]);
     }
 
     template <int LA, int LB, int LC, int LD, int MODE, bool SWAP, typename T>
@@ -736,21 +845,31 @@ namespace lbx
         // uniform-major: contiguous task ranges per wave, up to 8192 workgroups of 4 waves;
         // lane-block-major: as many workgroups as are resident at once, so that one sweep of the
         // waves over the task order keeps them all on the same few lane blocks
-        static const int resident = [] {
+        struct Residency
+        {
+            int blocks, cus;
+        };
+        static const Residency resident = [] {
             int per_cu = 0, dev = 0, ncu = 0;
             if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
                         &per_cu, reinterpret_cast<const void *>(&quartetV<LA, LB, LC, LD, MODE, SWAP, T>), 256, 0) !=
                         hipSuccess ||
                 hipGetDevice(&dev) != hipSuccess ||
                 hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-                return 8192;
-            return std::max(1, per_cu) * std::max(1, ncu);
+                return Residency{8192, 256};
+            return Residency{std::max(1, per_cu) * std::max(1, ncu), std::max(1, ncu)};
         }();
-        // per-molecule sums: four rounds of them, each wave ending in one addition per molecule
-        const long long cap = A.block_major ? std::min(resident, 8192) : MODE == MODE_SUM ? std::min(4 * resident, 8192) : 8192;
+        // K rows of the uniform pair in LDS
+        constexpr int SUa = nSph(SWAP ? LA : LC), SUb = nSph(SWAP ? LB : LD);
+        const size_t lds = MODE == MODE_JK ? sizeof(double) * (SUa + SUb) * A.kcols : 0;
+        long long cap = 8192;
+        if (A.block_major)
+            cap = std::min<long long>({resident.blocks, cap, lds ? resident.cus * static_cast<long long>(163840 / lds) : cap});
+        else if (MODE == MODE_SUM)
+            cap = std::min<long long>(4 * resident.blocks, cap);   // each wave ends in one addition per molecule
         long long wg = (A.ntasks + 3) / 4;
         int grid = static_cast<int>(wg < cap ? wg : cap);
-        hipLaunchKernelGGL((quartetV<LA, LB, LC, LD, MODE, SWAP, T>), dim3(grid), dim3(256), 0, s, A);
+        hipLaunchKernelGGL((quartetV<LA, LB, LC, LD, MODE, SWAP, T>), dim3(grid), dim3(256), lds, s, A);
     }
 
     // The FP32 forms (J/K and RI sums).
@@ -778,7 +897,7 @@ namespace lbx
     }
 
     // Registers the one-lane variants the class supports in this mode.  The ket-on-lanes form
-    // only serves J/K between different classes (dense and diagonal outputs keep the bra on
+    // only serves J/K between different classes (dense outputs and sums keep the bra on
     // the lanes; for one class both forms coincide).
     // FORMS: 1 the FP64 forms, 2 the FP32 forms, 3 both (lets the build compile them apart).
     template <int LA, int LB, int LC, int LD, int MODE, int FORMS = 3>

@@ -136,3 +136,29 @@ def test_ri_jk_sizes(lbx, oracle, nmain, naux):
         close(K.cpu().numpy(), Kr, rel=0.0, floor=1e-11)
     J, _ = ctx.ri_jk(torch.tensor(D, device="cuda"), exchange=False)
     close(J.cpu().numpy(), Jr, rel=0.0, floor=1e-11)
+
+
+@pytest.mark.parametrize("ns", [14, 15, 16, 19, 23])
+@pytest.mark.parametrize("variant", [0, 1, 3, 4])
+def test_jk_one_lane_pair_counts(lbx, oracle, ns, variant):
+    """One-lane J/K at pair counts around those where K rows move to LDS (more than two 64-pair
+    blocks: 105, 120 | 136, 190, 276 (ss) pairs), the last blocks of a group past the end, uneven
+    contractions among a block's lanes.  FP32 forms: 1e-5 of the largest element (the other parity
+    tests')."""
+    import torch
+    rng = np.random.default_rng(ns)
+    per_atom = [[(0, list(rng.uniform(0.2, 4.0, 1 + k % 4)), list(rng.uniform(0.2, 1.0, 1 + k % 4)))] for k in range(ns)]
+    for l in (1, 2, 3):
+        per_atom[l].append((l, [0.7, 1.3], [0.6, 0.5]))
+    m = B.Molecule(B.random_atoms(rng, ns, 5.0, 0.8), B.Shells.from_lists(per_atom))
+    D = B.density_from_orbitals(9, m.shells.nbf, 3, 0.3)
+    Jr, Kr, _ = oracle.Structure(m).jk(D, thresh=1e-10)
+    ctx = lbx.Context(m)
+    for la, lc in itertools.product(range(4), repeat=2):
+        for lb, ld in itertools.product(range(la + 1), range(lc + 1)):
+            ctx.set_variant((la, lb, lc, ld), variant)
+    mixed = dict(precision=lbx.LBX_MIXED, mixed_thresh=1e9) if variant >= 3 else {}
+    for _ in range(2):
+        J, K, _ = ctx.jk(torch.tensor(D, device="cuda"), schwarz=1e-10, **mixed)
+        for got, ref in ((J, Jr), (K, Kr)):
+            close(got.cpu().numpy(), ref, **(dict(rel=0.0, floor=1e-5) if variant >= 3 else dict(floor=1e-12)))
