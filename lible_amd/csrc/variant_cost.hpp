@@ -7,11 +7,13 @@
 // once), and a constant for the launch.  The coefficients (milliseconds per 10^6 of a count, on
 // the MI355X) are a non-negative fit of the logarithm of 2900 timed launches: every form of every class
 // pair to (ff|ff) on water clusters of 1 to 10 molecules in def2-SVP, -TZVP and -QZVP and on 2 to
-// 19 atoms of the synthetic s to f shells, 0.03 to 200 ms each, typically within 40%.  J/K time summed over the class pairs, ms,
-// by this rule / by the fastest form of each / by the mean-contraction estimate it replaces:
-//   H2O SVP 0.77 / 0.76 / 1.7, (H2O)8 SVP 7.4 / 7.1 / 12.2, (H2O)10 TZVP 53 / 47 / 72,
-//   7 atoms s-f 11.0 / 9.7 / 19, 19 atoms s-f 181 / 178 / 233;
-//   FP32 forms: 0.67 / 0.65 / 2.3, 7.2 / 6.8 / 11.6, 45 / 40 / 74, 9.8 / 8.8 / 14, 134 / 127 / 149.
+// 19 atoms of the synthetic s to f shells, 0.03 to 200 ms each, typically within 45%.  J/K time
+// summed over the class pairs, ms, by this rule / by the fastest form of each:
+//   H2O SVP 0.77 / 0.74, (H2O)8 SVP 5.5 / 4.9, (H2O)10 TZVP 40 / 35, 7 atoms s-f 9.8 / 8.3,
+//   19 atoms s-f 155 / 154;
+//   FP32 forms: 0.67 / 0.64, 5.2 / 4.9, 30 / 28, 8.6 / 7.4, 89 / 88
+// (the estimate from the mean contraction alone that it replaced, with the one-lane kernels of that
+// time: 1.7, 12.2, 72, 19 and 233; FP32 2.3, 11.6, 74, 14 and 149).
 #pragma once
 
 #include <algorithm>
@@ -45,30 +47,40 @@ namespace lbx
         }
 
         // One lane per quartet: `waves` tasks of 64 lane-side pairs against one uniform pair, in
-        // column passes of nc (R and Boys again in each).  sums: J/K, whose epilogue sums each
-        // uniform-side column over the wave.
-        inline double laneForm(const Side &lane, const Side &unif, int nc, bool f32, double waves, bool sums)
+        // column passes of nc (R and Boys again in each).  jk: E interleaved over the lanes, K rows
+        // and wave sums in the epilogue; the other modes read E a line per lane.
+        inline double laneForm(const Side &lane, const Side &unif, int nc, bool f32, double waves, bool jk)
         {
             const int L = lane.L() + unif.L(), su = unif.S(), sl = lane.S();
             const double passes = ceilDiv(su, nc), step = passes * (recursionSteps(L) + 100);
-            const double hlsl = double(lane.H()) * sl;
-            const double fma = lane.klane * (unif.kmean * lane.H() * unif.H() * su + hlsl * su);
+            const double hlsl = double(lane.H()) * sl, hlhu = double(lane.H()) * unif.H();
+            const double fma = lane.klane * (unif.kmean * hlhu * su + hlsl * su);
             const double rec = lane.klane * unif.kmean * step;
             const double eLane = lane.klane * hlsl * passes;   // lane-side E elements (a load per lane)
-            const double chain = lane.kmax * (unif.kmax * (double(lane.H()) * unif.H() * su + step) + hlsl * su);
-            // more than three passes share one instance of the pass body, which then spills
-            const double shared = passes > 3 ? 1.0 : 0.0, big = hlsl > 700 ? 1.0 : 0.0;
-            const double runs = (nSph(unif.la) + nSph(unif.lb)) * nSph(lane.lb);
+            const double chain = lane.kmax * (unif.kmax * (hlhu * su + step) + hlsl * su);
+            // more than three passes share one instance of the pass body, which then spills (in the
+            // J/K forms those with a long body)
+            const double shared = passes > 3 && (!jk || nc * (hlhu + hlsl) > (f32 ? 4500 : 1400)) ? 1.0 : 0.0;
+            const double big = hlsl > 700 ? 1.0 : 0.0;
+            const double rows = nSph(unif.la) + nSph(unif.lb);
             double t;
-            if (f32)
-                t = waves * (0.0033 * rec + (0.0177 + 0.0388 * big) * eLane + 0.0027 * shared * (fma + rec) +
-                             (sums ? 4.97 * su + 1.64 * runs + 0.56 * su * sl : 0.0)) +
+            // an (ss) lane side: each FMA takes a new scalar load of the uniform side's E
+            const double steps = lane.H() == 1 ? lane.klane * unif.kmean : 0.0, uLoads = steps * unif.H() * su;
+            if (jk && f32)
+                t = waves * (0.0022 * rec + (0.0119 + 0.013 * big) * eLane + 0.0039 * shared * (fma + rec) +
+                             0.0036 * uLoads + 0.328 * passes * steps + 1.37 * rows + 0.197 * su * su + 10.3) +
+                    (2.41 + 1.74 * shared) * chain;
+            else if (jk)
+                t = waves * (0.0021 * rec + (0.0212 + 0.0248 * big) * eLane + 0.0179 * shared * (fma + rec) +
+                             0.013 * uLoads + 0.207 * passes * steps + 0.5 * rows + 0.353 * su * su + 7.27) +
+                    (3.40 + 15.7 * shared) * chain;
+            else if (f32)
+                t = waves * (0.0033 * rec + (0.0177 + 0.0388 * big) * eLane + 0.0027 * shared * (fma + rec)) +
                     (2.68 + 2.60 * shared) * chain;
             else
-                t = waves * (0.0024 * rec + (0.0422 + 0.0176 * big) * eLane + 0.0122 * shared * (fma + rec) +
-                             (sums ? 10.99 * su : 0.0)) +
+                t = waves * (0.0024 * rec + (0.0422 + 0.0176 * big) * eLane + 0.0122 * shared * (fma + rec)) +
                     (3.91 + 9.28 * shared) * chain;
-            return 1e-6 * t + (f32 ? 0.073 : 0.061);
+            return 1e-6 * t + (jk && !f32 ? 0.05 : 0.06);
         }
 
         // One wave per quartet (MFMA).
