@@ -409,7 +409,8 @@ namespace lbx
                 t.phi[q] = b;
                 t.prefix[q] = acc;
                 const long long cnt = b - a;
-                acc += (cnt + width - 1) / width;
+                // the one-lane form's tasks are the aligned blocks of 64 positions
+                acc += width == 64 && cnt > 0 ? (b - (a & ~63) + 63) / 64 : (cnt + width - 1) / width;
                 if (cnt > 0)
                 {
                     const double kq = unif.pcnt[unif.order[q]];
@@ -528,7 +529,7 @@ namespace lbx
         }
 
         // E matrices of a class interleaved over the lanes of each block of 64 lane positions
-        // (KArgs::le): perm maps lane position -> position in order
+        // (KArgs::le): perm maps lane position -> position in order (null: the same)
         template <typename T>
         __global__ __launch_bounds__(256) void interleaveKernel(const T *__restrict__ in, T *__restrict__ out,
                                                                 const int *order, const int *perm, const int *poff,
@@ -536,7 +537,7 @@ namespace lbx
         {
             const int lane = threadIdx.x & 63;
             const int pos = 64 * static_cast<int>(blockIdx.x) + lane;
-            const int pair = pos < n ? order[perm[pos]] : -1;
+            const int pair = pos < n ? order[perm ? perm[pos] : pos] : -1;
             const T *src = pair >= 0 ? in + static_cast<size_t>(poff[pair]) * hs : in;
             const long long own = pair >= 0 ? static_cast<long long>(pcnt[pair]) * hs : 0;
             const long long rows = (base[blockIdx.x + 1] - base[blockIdx.x]) / 64;
@@ -978,44 +979,92 @@ struct lbx_context : Context
     };
     std::map<std::pair<const LanePerm *, bool>, LaneE> lane_e;
 
-    // le / le32 / lbase of a lane side; the interleaved copies are made on first use
+    // le / le32 / lbase of a J/K lane side; the interleaved copies are made on first use
     void setLaneE(KArgs &a, const PairClass &pc, bool ket, const LanePerm &lp, bool f32)
     {
         LaneE &le = lane_e[{&lp, ket}];
+        interleave(le, pc, ket, pc.order, &lp.perm, pc.d_order, lp.d_perm, f32);
+        a.le = le.e;
+        a.le32 = le.e32;
+        a.lbase = le.base;
+    }
+
+    void interleave(LaneE &le, const PairClass &pc, bool ket, const std::vector<int> &order,
+                    const std::vector<int> *perm, const int *d_order, const int *d_perm, bool f32)
+    {
+        if (f32 ? le.e32 != nullptr : le.e != nullptr)
+            return;
         const int hs = nHerm(pc.la + pc.lb) * nSph(pc.la) * nSph(pc.lb), nblk = (pc.n_pairs + 63) / 64;
         std::vector<long long> base(nblk + 1, 0);
-        if (f32 ? !le.e32 : !le.e)
+        for (int b = 0; b < nblk; b++)
         {
-            for (int b = 0; b < nblk; b++)
-            {
-                int k = 0;
-                for (int p = 64 * b; p < std::min(64 * b + 64, pc.n_pairs); p++)
-                    k = std::max(k, pc.pcnt[pc.order[lp.perm[p]]]);
-                base[b + 1] = base[b] + 64LL * k * hs;
-            }
-            if (!le.base)
-                le.base = upload(base);
-            flushStaged();   // lp's arrays
-            const dim3 grid(nblk, 16);
-            auto run = [&](auto *out, auto *in) {
-                using T = std::remove_reference_t<decltype(*out)>;
-                hipLaunchKernelGGL(interleaveKernel<T>, grid, dim3(256), 0, stream, in, out, pc.d_order, lp.d_perm,
-                                   pc.d_poff, pc.d_pcnt, le.base, pc.n_pairs, hs);
-                LBX_HIP(hipGetLastError());
-            };
-            if (f32)
-            {
-                float *e = alloc<float>(base[nblk]);
-                run(e, ket ? pc.d_ek32 : pc.d_eb32);
-                le.e32 = e;
-            }
-            else
-            {
-                double *e = alloc<double>(base[nblk]);
-                run(e, ket ? pc.d_ek : pc.d_eb);
-                le.e = e;
-            }
+            int k = 0;
+            for (int p = 64 * b; p < std::min(64 * b + 64, pc.n_pairs); p++)
+                k = std::max(k, pc.pcnt[order[perm ? (*perm)[p] : p]]);
+            base[b + 1] = base[b] + 64LL * k * hs;
         }
+        if (!le.base)
+            le.base = upload(base);
+        flushStaged();   // the orders
+        const dim3 grid(nblk, 16);
+        auto run = [&](auto *out, auto *in) {
+            using T = std::remove_reference_t<decltype(*out)>;
+            hipLaunchKernelGGL(interleaveKernel<T>, grid, dim3(256), 0, stream, in, out, d_order, d_perm, pc.d_poff,
+                               pc.d_pcnt, le.base, pc.n_pairs, hs);
+            LBX_HIP(hipGetLastError());
+        };
+        if (f32)
+        {
+            float *e = alloc<float>(base[nblk]);
+            run(e, ket ? pc.d_ek32 : pc.d_eb32);
+            le.e32 = e;
+        }
+        else
+        {
+            double *e = alloc<double>(base[nblk]);
+            run(e, ket ? pc.d_ek : pc.d_eb);
+            le.e = e;
+        }
+    }
+
+    // Pair order of the RI sums without a bound range: by molecule, then the longest primitive
+    // loops first.  Unlike the classes' order it does not change when the Schwarz factors are made,
+    // so launches prepared before that stay good.
+    struct SumOrder
+    {
+        std::vector<int> order;
+        int *d_order = nullptr;
+    };
+    std::map<const PairClass *, SumOrder> sum_orders;
+    // the lane sides' interleaved E in that order or (true) in the Schwarz order
+    std::map<std::pair<const PairClass *, bool>, LaneE> sum_e;
+
+    const SumOrder &sumOrder(const PairClass &pc)
+    {
+        SumOrder &so = sum_orders[&pc];
+        if (!so.d_order)
+        {
+            so.order = pc.order;
+            std::stable_sort(so.order.begin(), so.order.end(), [&](int x, int y) {
+                return pc.mol[x] != pc.mol[y] ? pc.mol[x] < pc.mol[y] : pc.pcnt[x] > pc.pcnt[y];
+            });
+            so.d_order = stage(so.order);
+        }
+        return so;
+    }
+
+    // orders and (one-lane forms) the lane side's E of an RI sum launch
+    void setSumSides(KArgs &a, const PairClass &lane, const PairClass &unif, bool bounded, int kind, bool f32)
+    {
+        if (!bounded)
+        {
+            a.bra.order = sumOrder(lane).d_order;
+            a.ket.order = sumOrder(unif).d_order;
+        }
+        if (kind != KIND_LANE)
+            return;
+        LaneE &le = sum_e[{&lane, bounded}];
+        interleave(le, lane, false, bounded ? lane.order : sumOrder(lane).order, nullptr, a.bra.order, nullptr, f32);
         a.le = le.e;
         a.le32 = le.e32;
         a.lbase = le.base;
@@ -1116,7 +1165,8 @@ struct lbx_context : Context
         }
         // K rows of the uniform pair in LDS: up to 64 KiB, and at least three lane blocks to share
         // them (a workgroup's four waves take four blocks of a group); else K by atomics alone, which
-        // bound the classes of low angular momentum (16 updates per (ps|ps) quartet at 23 G/s)
+        // bound the classes of low angular momentum (16 updates per (ps|ps) quartet at 23 G/s:
+        // (H2O)10 def2-TZVP (ps|ps) 2.3 ms, with the rows in LDS 1.1)
         const PairClass &uside = s.swap ? bra : ket;
         const bool kLds = blockMajor && nlane > 128 && (nSph(uside.la) + nSph(uside.lb)) * kColumns(lside) * 8 <= 65536;
         if (kLds)
@@ -1305,6 +1355,8 @@ struct lbx_context : Context
                 KArgs a = baseArgs(*this, lane, unif, t, same);
                 a.kind = kind;
                 a.out = scratch.p;
+                setSumSides(a, lane, unif, false, k.kind, false);
+                flushStaged();
                 k.fn(a, stream);   // loads the code
                 LBX_HIP(hipEventRecord(e0, stream));
                 k.fn(a, stream);
@@ -1376,6 +1428,7 @@ struct lbx_context : Context
                     TaskTable t = buildTasksMol(*this, lane, unif, same, k.width, lo, hi);
                     KArgs a = baseArgs(*this, lane, unif, t, same);
                     a.kind = kind;
+                    setSumSides(a, lane, unif, split > 0.0, k.kind, fp32);
                     launches.push_back({k.fn, a, variantTime(MODE_SUM, lane, unif, k, fp32, t.quartets, double(t.ntasks))});
                     n[kind == 3 ? 0 : 1] += t.quartets;
                     n[2] += t.flops;

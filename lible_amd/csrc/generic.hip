@@ -1,5 +1,6 @@
-// Quartet kernels for the class pairs with a g shell in the main basis: one kernel for all of
-// them, with the angular momenta at run time (the reference's generic-L kernels,
+// Quartet kernels for the class pairs with a g shell in the main basis: dense tensors, diagonals,
+// sums and the gradient of all of them and J/K of (gg|gg) and (gg|gf) (the other J/K class pairs
+// run the compiled one-wave form), one kernel with the angular momenta at run time (the reference's generic-L kernels,
 // eri_kernel_funs.cpp:7-101, serve every class above its rolled-out ones the same way).
 //
 // One wave per shell quartet (the task tables of the one-wave MFMA form, so every J/K, dense,

@@ -8,21 +8,21 @@
 // (-1)^{t'+u'+v'} folded into Ek) and Eb, Ek the spherical Hermite-expansion matrices of the
 // primitive pairs.
 //
-// Two kernels:
-//   quartetV  one lane per quartet, everything in registers.  A wave holds 64 pairs of one side
-//             (the "lane" side) against one pair of the other (the "uniform" side), so every
-//             uniform-side operand is a scalar load and the transforms are VALU FMAs with an
-//             SGPR operand.  Registers are bounded by splitting the uniform side's spherical
-//             components into column passes (Boys + R recomputed per pass); which side runs on
-//             the lanes is chosen per class to minimise work.
-//   quartetM  one wave per quartet, both transforms on FP64 MFMA (v_mfma_f64_16x16x4f64).  The
-//             bra primitive pairs are stacked along M, (prim, tuv) rows, so one GEMM per ket
-//             primitive covers all bra primitives: X[(i,tuv), kl] += R[(i,tuv), t'u'v'] Ek[t'u'v', kl];
-//             the bra transform contracts over the stacked rows, I^T = X^T Eb_stack, reading X^T
-//             straight out of the accumulator registers: accumulator element c of a 16-row tile
-//             holds rows 4c..4c+3 across the lane groups, which is exactly the A-operand layout
-//             of K-chunk c.  R is built cooperatively in LDS.  Used where R alone would not fit
-//             a lane's registers (high total angular momentum).
+// quartetV: one lane per quartet, everything in registers.  A wave holds 64 pairs of one side (the
+// "lane" side) against one pair of the other (the "uniform" side), so every uniform-side operand is
+// a scalar load and the transforms are VALU FMAs with an SGPR operand.  Registers are bounded by
+// splitting the uniform side's spherical components into column passes (Boys + R recomputed per
+// pass); which side runs on the lanes is chosen per class pair (variant_cost.hpp).
+//
+// What bounds it: the loads of the lane side's E, one element per FMA of a column.  As stored, each
+// is a line per lane (about 100 cycles against 4 for the FMA), and the compiler waits for it before
+// it issues the next; interleaved over the lanes (512 contiguous bytes) and loaded a group ahead
+// they cost J/K of 19 atoms (570 functions): (dp|ps) 5.1 -> 2.7 ms, (dp|ds) 5.4 -> 2.7, (fp|ps)
+// 9.4 -> 8.4, FP32 (fd|ps) 11.6 -> 1.2, (dd|dp) 4.8 -> 1.6.  At low angular momentum the K atomics
+// (16 updates per (ps|ps) quartet at 23 G lines/s): K rows in LDS take J/K of (H2O)10 def2-TZVP
+// from (pp|ps) 2.4 -> 1.1 ms, (ps|ps) 2.3 -> 1.1, (ds|ps) 2.2 -> 0.95.  (ss|ss) is left at its Boys
+// functions: 4.5e8 in 2.8 ms.
+// The other forms: quartet_wave.hpp (one wave per quartet on MFMA), quartet_block.hpp.
 // Epilogues: J/K contraction with atomics, dense tensor scatter, per-molecule sums, or (one-wave
 // form) the (ab|ab) diagonal and listed blocks.
 #pragma once
@@ -57,7 +57,7 @@ namespace lbx
         int nket;
         long long ntasks;
         int same_class;            // bra class == ket class: quartet p == q is its own image
-        int bra_major;             // quartetM: q indexes bra pairs, p ket pairs (classes differ)
+        int bra_major;             // one-wave form: q indexes bra pairs, p ket pairs (classes differ)
         // quartetV lane-block-major order: lane block b = lane positions 64b .. 64b+63; group g =
         // blocks g G .. g G + G - 1 (G = 2^gshift).  Group g's tasks pair its uniform positions
         // q = bq0[g], bq0[g] + 1, ... with its G blocks in turn (bprefix[g+1] - bprefix[g] = G x
@@ -65,9 +65,10 @@ namespace lbx
         int block_major, nblk, gshift;
         const long long *bprefix;
         const int *bq0;
-        // lane-block-major J/K: lane position -> Schwarz-order position (the lane side ordered by
-        // shell within Schwarz-factor buckets, so lanes sharing a shell are adjacent), and per
-        // lane block the range [bqlo, bqhi) of Schwarz-order positions it holds; null otherwise
+        // lane-block-major J/K: lane position -> Schwarz-order position (within Schwarz-factor
+        // buckets by primitive count when kcols > 0, else by shell, so lanes sharing a shell are
+        // adjacent), and per lane block the range [bqlo, bqhi) of Schwarz-order positions it holds;
+        // null otherwise
         const int *lperm, *bqlo, *bqhi;
         const double *boys;
         // MODE_JK
@@ -318,14 +319,18 @@ namespace lbx
         // Skipping structural zeros scatters the loads of E (no wide contiguous loads); it pays
         // where each loaded value feeds several FMAs: lane side with >= 2 columns per pass,
         // uniform side with >= 4 Hermite rows of X.
+        // The lane side's E interleaved over the block's lanes (wave-uniform base + lane); dense
+        // tensors, whose lanes are not aligned to the blocks, read it as stored.
+        constexpr bool kInter = MODE != MODE_DENSE;
+        constexpr int ES = kInter ? 64 : 1;
         constexpr bool kSkipL = NC >= 2;
         constexpr bool kSkipU = HLn >= 4;
         static_assert(!F32 || MODE == MODE_JK || MODE == MODE_SUM, "FP32 forms: J/K and RI sums");
         const DPairs &LP = SWAP ? A.ket : A.bra;
         const DPairs &UP = SWAP ? A.bra : A.ket;
 
-        // lanes cover lane positions pbase .. pbase + 63 (pbase = `local`); p is the lane's
-        // Schwarz-order position (through A.lperm when the lane side is shell-ordered)
+        // lanes cover lane positions local .. local + 63; p is the lane's Schwarz-order position
+        // (through A.lperm for J/K)
         const int plo = uniform(A.plo[q]), phi = uniform(A.phi[q]);
         const bool permuted = A.lperm != nullptr;
         // the last group of a lane-block-major table runs G blocks, some past the lane side
@@ -347,20 +352,17 @@ namespace lbx
         if constexpr (F32)
         {
             eUb = SWAP ? UP.eb32 : UP.ek32;
-            eLb = MODE == MODE_JK ? A.le32 : LP.eb32;
+            eLb = A.le32;
         }
         else
         {
             eUb = SWAP ? UP.eb : UP.ek;
-            eLb = MODE == MODE_JK ? A.le : LP.eb;
+            eLb = kInter ? A.le : LP.eb;
         }
         const cptr<T> eU = constView(eUb + static_cast<size_t>(upoff) * HU * SU);
         const cptr<double> ppU = constView(reinterpret_cast<const double *>(UP.pp + upoff));
-        // the lane side's E: J/K interleaved over the block's lanes (wave-uniform base + lane), the
-        // other modes, whose lanes are not aligned to the blocks, as stored
-        constexpr int ES = MODE == MODE_JK ? 64 : 1;
         const T *__restrict__ eL;
-        if constexpr (MODE == MODE_JK)
+        if constexpr (kInter)
             eL = eLb + uniform(A.lbase[local >> 6]);
         else
             eL = eLb + static_cast<size_t>(lpoff) * HLn * SL;
@@ -488,14 +490,14 @@ namespace lbx
                 T eb[2][G];
                 auto load = [&](auto gC) {
                     constexpr int g = decltype(gC)::value;
-                    // J/K: the group's (uniform) address anew, else all of them are formed ahead
+                    // the group's (uniform) address anew, else all of them are formed ahead
                     Row er = (Row)(eL + (static_cast<size_t>(i) * (HLn * SL) + EL.e[g * G]) * ES);
-                    if constexpr (MODE == MODE_JK)
+                    if constexpr (kInter)
                         asm("" : "+s"(er));
 #pragma unroll
                     for (int j = 0; j < G; j++)
                         if (g * G + j < EL.n)
-                            eb[g & 1][j] = er[(EL.e[g * G + j] - EL.e[g * G]) * ES + (MODE == MODE_JK ? lane : 0)];
+                            eb[g & 1][j] = er[(EL.e[g * G + j] - EL.e[g * G]) * ES + (kInter ? lane : 0)];
                 };
                 load(std::integral_constant<int, 0>{});
                 forEachInt<NG>([&](auto gC) {
@@ -829,7 +831,9 @@ namespace lbx
                         jl[0] = jl[1] = 0.0;
                     }
                 }
-                quartetVTask<LA, LB, LC, LD, MODE, SWAP, T>(A, q, uniform(A.plo[q]) + 64 * static_cast<int>(t - base),
+                // sums: aligned blocks of 64 positions (the interleaved E's)
+                const int first = MODE == MODE_SUM ? uniform(A.plo[q]) & ~63 : uniform(A.plo[q]);
+                quartetVTask<LA, LB, LC, LD, MODE, SWAP, T>(A, q, first + 64 * static_cast<int>(t - base),
                                                             lane, jl);
             }
             if constexpr (MODE == MODE_SUM)
