@@ -480,7 +480,7 @@ namespace lbx
         {
             const cost::Side b = costSide(bra), k = costSide(ket);
             if (s.kind == KIND_LANE)
-                return cost::laneForm(s.swap ? k : b, s.swap ? b : k, s.nc, f32, waves, mode == MODE_JK);
+                return cost::laneForm(s.swap ? k : b, s.swap ? b : k, s.nc, f32, waves, mode == MODE_JK || mode == MODE_SUM, mode == MODE_JK);
             return s.kind == KIND_WAVE ? cost::waveForm(b, k, f32, quartets) : cost::blockForm(b, k, f32, quartets);
         }
 

@@ -47,9 +47,9 @@ namespace lbx
         }
 
         // One lane per quartet: `waves` tasks of 64 lane-side pairs against one uniform pair, in
-        // column passes of nc (R and Boys again in each).  jk: E interleaved over the lanes, K rows
-        // and wave sums in the epilogue; the other modes read E a line per lane.
-        inline double laneForm(const Side &lane, const Side &unif, int nc, bool f32, double waves, bool jk)
+        // column passes of nc (R and Boys again in each).  inter: E interleaved over the lanes (J/K and
+        // sums; the other modes read it a line per lane); jk: K rows and wave sums in the epilogue.
+        inline double laneForm(const Side &lane, const Side &unif, int nc, bool f32, double waves, bool inter, bool jk)
         {
             const int L = lane.L() + unif.L(), su = unif.S(), sl = lane.S();
             const double passes = ceilDiv(su, nc), step = passes * (recursionSteps(L) + 100);
@@ -59,20 +59,20 @@ namespace lbx
             const double eLane = lane.klane * hlsl * passes;   // lane-side E elements (a load per lane)
             const double chain = lane.kmax * (unif.kmax * (hlhu * su + step) + hlsl * su);
             // more than three passes share one instance of the pass body, which then spills (in the
-            // J/K forms those with a long body)
-            const double shared = passes > 3 && (!jk || nc * (hlhu + hlsl) > (f32 ? 4500 : 1400)) ? 1.0 : 0.0;
+            // interleaved forms those with a long body)
+            const double shared = passes > 3 && (!inter || nc * (hlhu + hlsl) > (f32 ? 4500 : 1400)) ? 1.0 : 0.0;
             const double big = hlsl > 700 ? 1.0 : 0.0;
             const double rows = nSph(unif.la) + nSph(unif.lb);
             double t;
             // an (ss) lane side: each FMA takes a new scalar load of the uniform side's E
             const double steps = lane.H() == 1 ? lane.klane * unif.kmean : 0.0, uLoads = steps * unif.H() * su;
-            if (jk && f32)
+            if (inter && f32)
                 t = waves * (0.0022 * rec + (0.0119 + 0.013 * big) * eLane + 0.0039 * shared * (fma + rec) +
-                             0.0036 * uLoads + 0.328 * passes * steps + 1.37 * rows + 0.197 * su * su + 10.3) +
+                             0.0036 * uLoads + 0.328 * passes * steps + (jk ? 1.37 * rows + 0.197 * su * su + 10.3 : 0.0)) +
                     (2.41 + 1.74 * shared) * chain;
-            else if (jk)
+            else if (inter)
                 t = waves * (0.0021 * rec + (0.0212 + 0.0248 * big) * eLane + 0.0179 * shared * (fma + rec) +
-                             0.013 * uLoads + 0.207 * passes * steps + 0.5 * rows + 0.353 * su * su + 7.27) +
+                             0.013 * uLoads + 0.207 * passes * steps + (jk ? 0.5 * rows + 0.353 * su * su + 7.27 : 0.0)) +
                     (3.40 + 15.7 * shared) * chain;
             else if (f32)
                 t = waves * (0.0033 * rec + (0.0177 + 0.0388 * big) * eLane + 0.0027 * shared * (fma + rec)) +
@@ -80,7 +80,7 @@ namespace lbx
             else
                 t = waves * (0.0024 * rec + (0.0422 + 0.0176 * big) * eLane + 0.0122 * shared * (fma + rec)) +
                     (3.91 + 9.28 * shared) * chain;
-            return 1e-6 * t + (jk && !f32 ? 0.05 : 0.06);
+            return 1e-6 * t + (inter && !f32 ? 0.05 : 0.06);
         }
 
         // One wave per quartet (MFMA).
