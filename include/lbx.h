@@ -208,8 +208,8 @@ int lbx_ri_sums(lbx_context *ctx, double *out, int precision, double mixed_thres
  *                   f (4 D_mn D_kl - D_mk D_nl - D_ml D_nk) d(mn|kl)/dR_{A,x}
  * with f the permutational weight.  D: device (nbf, nbf) symmetric; grad: device 3 natoms
  * (atom-major, x y z), Eh/bohr.  precision LBX_FP64, or LBX_MIXED: quartets with bound below
- * mixed_thresh in FP32 arithmetic (R, E, E', transforms) with FP64 Boys values and sums; stats
- * count the quartets and those in FP32. */
+ * mixed_thresh with R, E and E' in FP32 (for class pairs of total angular momentum up to 4 the
+ * transforms too) and FP64 Boys values and sums; stats count the quartets and those in FP32. */
 int lbx_jk_grad(lbx_context *ctx, const double *D, double *grad, double schwarz_thresh,
                 int precision, double mixed_thresh, lbx_jk_stats *stats);
 

@@ -20,17 +20,11 @@
 
 namespace lbx
 {
-    typedef float gv4f __attribute__((ext_vector_type(4)));
-
-    // 16x16x4 MFMA, A[j][g] and B[g][j] from lane (g, j) = (lane / 16, lane % 16); accumulator
-    // element r of that lane holds D[4 r + g][j] for FP64 and D[4 g + r][j] for FP32.
+    // 16x16x4 FP64 MFMA, A[j][g] and B[g][j] from lane (g, j) = (lane / 16, lane % 16); accumulator
+    // element r of that lane holds D[4 r + g][j].
     __device__ __forceinline__ v4d gmfma(double a, double b, v4d c)
     {
         return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-    }
-    __device__ __forceinline__ gv4f gmfma(float a, float b, gv4f c)
-    {
-        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
     }
 
     template <int LA, int LB, int LC, int LD, typename T>
@@ -41,10 +35,8 @@ namespace lbx
         static constexpr int SB = nSph(LB), SD = nSph(LD), SP = nSph(LA) * SB, SQ = nSph(LC) * SD;
         static constexpr int NQ = ceilDiv(SQ, 16), KQ = ceilDiv(HQ, 4);
         static constexpr int TP = ceilDiv(HP, 16), TP1 = ceilDiv(HP1, 16), TQ = ceilDiv(HQ, 16), TS = ceilDiv(SP, 16);
-        // K steps over accumulator rows: FP64 element r of a tile holds rows 4 r .. 4 r + 3, FP32
-        // rows r, 4 + r, 8 + r, 12 + r
-        static constexpr bool F32 = sizeof(T) == 4;
-        static constexpr int KP = F32 ? 4 * TP : ceilDiv(HP, 4), KS = F32 ? 4 * TS : ceilDiv(SP, 4);
+        // K steps over accumulator rows: element r of a tile holds rows 4 r .. 4 r + 3
+        static constexpr int KP = ceilDiv(HP, 4), KS = ceilDiv(SP, 4);
         // primitive quartets whose R is held at a time: 10 KiB of LDS
         static constexpr int PB0 = 10240 / (HL1 * static_cast<int>(sizeof(T)));
         static constexpr int PB = PB0 < 1 ? 1 : (PB0 > 64 ? 64 : PB0);
@@ -52,6 +44,11 @@ namespace lbx
         static constexpr int YS = 17;        // row stride of Y in LDS
     };
 
+    // T: type of R, the E and the E' matrices (float: the small-bound quartets of a mixed build).
+    // Every product and sum is FP64 in both, on the FP64 MFMA: T_ik is the difference of two totals
+    // over the ket primitives, and in FP32 accumulators the share of a small primitive was rounded at
+    // the size of the ones before it.  7 atoms (s to f), every quartet in the float form: 36.9 ms (FP32
+    // accumulators 33.9, the double form 41.9); 19 atoms 1058 ms (1017, 1207).
     template <int LA, int LB, int LC, int LD, typename T>
     __global__ __launch_bounds__(64, 2) void gradWave(const GArgs A)
     {
@@ -59,14 +56,13 @@ namespace lbx
         constexpr int L1 = P::L1, HL1 = P::HL1, HP = P::HP, HP1 = P::HP1, HQ = P::HQ, SP = P::SP, SQ = P::SQ;
         constexpr int SB = P::SB, SD = P::SD, NQ = P::NQ, KQ = P::KQ, TP = P::TP, TP1 = P::TP1, TQ = P::TQ, TS = P::TS;
         constexpr int KP = P::KP, KS = P::KS, PB = P::PB, TW = P::TW, YS = P::YS;
-        constexpr bool F32 = P::F32;
-        using Acc = std::conditional_t<F32, gv4f, v4d>;
+        constexpr bool F32 = sizeof(T) == 4;
         __shared__ T sR[PB * HL1];
         __shared__ T sInit[PB * (L1 + 1)];
         __shared__ T sPQ[4 * PB];
         __shared__ unsigned short sTab[16 * TP1 * TW]; // R index of (h', g); 0 past HP1, HQ
         __shared__ unsigned short sDn[16 * TP1][4];    // Y row of h' - e_x times YS; the zero row when there is none
-        __shared__ T sY[(HP + 1) * YS];
+        __shared__ double sY[(HP + 1) * YS];
 
         const int lane0 = threadIdx.x;
         const long long t0 = A.ntasks * blockIdx.x / gridDim.x;
@@ -100,7 +96,7 @@ namespace lbx
             sDn[e][2] = static_cast<unsigned short>((v > 0 ? hermIdx(t, u, v - 1) : HP) * YS);
         }
         if (lane0 < YS)
-            sY[HP * YS + lane0] = T(0);
+            sY[HP * YS + lane0] = 0.0;
         waveFence();
 
         int q = uniform(findKet(A.prefix, A.nket, t0));
@@ -115,9 +111,7 @@ namespace lbx
             }
             const int lane = opaqueLane(lane0);
             const int g4 = lane >> 4, j = lane & 15;
-            // row of accumulator element (K step) kk held by this lane: rowBase(kk) + rowLane
-            const int rowLane = F32 ? 4 * g4 : g4;
-            auto rowBase = [](int kk) { return F32 ? 16 * (kk >> 2) + (kk & 3) : 4 * kk; };
+            // accumulator element (K step) kk of this lane holds row 4 kk + g4
             const int p = uniform(A.plo[q] + static_cast<int>(t - base));
             const int u = uniform(UP.order[q]), l = uniform(LP.order[p]);
             const int upoff = uniform(UP.poff[u]), ucnt = uniform(UP.pcnt[u]);
@@ -151,10 +145,10 @@ namespace lbx
                     {
                         const int col = 16 * pass + j;
                         const bool inC = col < SQ;
-                        const unsigned ekOff = g4 * SQ + col, e1kOff = rowLane * SQ + col;
-                        const int yOff = rowLane * YS + j;
+                        const unsigned ekOff = g4 * SQ + col, e1kOff = g4 * SQ + col;
+                        const int yOff = g4 * YS + j;
                         // density weights: this lane's B-operand elements
-                        T wB[KS];
+                        double wB[KS];
                         {
                             const int ga = inC ? col / SD : 0, de = inC ? col % SD : 0;
                             const long long ic = c0 + ga, id = d0 + de;
@@ -162,13 +156,13 @@ namespace lbx
 #pragma unroll
                             for (int kk = 0; kk < KS; kk++)
                             {
-                                const int ab = rowBase(kk) + rowLane;
+                                const int ab = 4 * kk + g4;
                                 const bool in = inC && ab < SP;
                                 const int al = in ? ab / SB : 0, be = in ? ab % SB : 0;
                                 const long long ia = a0 + al, ib = b0 + be;
                                 const double w = f * (D[ia * n + ib] * dcd - D[ia * n + ic] * D[ib * n + id] -
                                                       D[ia * n + id] * D[ib * n + ic]);
-                                wB[kk] = in ? T(w) : T(0);
+                                wB[kk] = in ? w : 0.0;
                             }
                         }
 #pragma unroll 1
@@ -186,20 +180,20 @@ namespace lbx
                                 eb = LP.eb + static_cast<size_t>(ip) * HP * SP;
                                 e1b = LP.e1b + static_cast<size_t>(ip) * 3 * HP * SP;
                             }
-                            const unsigned ebOff = j * SP + rowLane, e1bOff = rowLane * SP + j;
-                            Acc y[TP];
+                            const unsigned ebOff = j * SP + g4, e1bOff = g4 * SP + j;
+                            v4d y[TP];
 #pragma unroll
                             for (int tp = 0; tp < TP; tp++)
-                                y[tp] = Acc{0, 0, 0, 0};
+                                y[tp] = v4d{0, 0, 0, 0};
 #pragma unroll
                             for (int kk = 0; kk < KS; kk++)
                             {
-                                const int ab0 = rowBase(kk);
+                                const int ab0 = 4 * kk;
 #pragma unroll
                                 for (int tp = 0; tp < TP; tp++)
                                 {
-                                    const bool in = 16 * tp + j < HP && ab0 + rowLane < SP;
-                                    const T a = in ? (eb + 16 * tp * SP + ab0)[ebOff] : T(0);
+                                    const bool in = 16 * tp + j < HP && ab0 + g4 < SP;
+                                    const double a = in ? (eb + 16 * tp * SP + ab0)[ebOff] : T(0);
                                     y[tp] = gmfma(a, wB[kk], y[tp]);
                                 }
                             }
@@ -209,16 +203,16 @@ namespace lbx
 #pragma unroll
                                 for (int r = 0; r < 4; r++)
                                 {
-                                    const int row = rowBase(4 * tp + r);
-                                    if (row + rowLane < HP)
+                                    const int row = 4 * (4 * tp + r);
+                                    if (row + g4 < HP)
                                         sY[row * YS + yOff] = y[tp][r];
                                 }
                             waveFence();
 
-                            Acc s[TP1];
+                            v4d s[TP1];
 #pragma unroll
                             for (int tp = 0; tp < TP1; tp++)
-                                s[tp] = Acc{0, 0, 0, 0};
+                                s[tp] = v4d{0, 0, 0, 0};
                             double dsum[3] = {0, 0, 0};   // sum over the k so far of T_ik (this lane's part)
 #pragma unroll 1
                             for (int k = 0; k < nk; k++)
@@ -227,7 +221,7 @@ namespace lbx
                                 const T *R = sR + (i * nk + k) * HL1;
                                 // opaque again: nothing in this loop writes LDS, so its table and Y reads
                                 // would all move in front of it
-                                const int jk = opaqueLane(j), rk = opaqueLane(rowLane);
+                                const int jk = opaqueLane(j), rk = opaqueLane(g4);
                                 const int tabS = jk * TW + g4, tabQ = rk * TW + jk;
                                 const T *ek, *e1k;
                                 if constexpr (F32)
@@ -244,7 +238,7 @@ namespace lbx
                                 for (int kt = 0; kt < KQ; kt++)
                                 {
                                     const bool in = 4 * kt + g4 < HQ && inC;
-                                    const T b = in ? (ek + 4 * kt * SQ)[ekOff] : T(0);
+                                    const double b = in ? (ek + 4 * kt * SQ)[ekOff] : T(0);
 #pragma unroll
                                     for (int tp = 0; tp < TP1; tp++)
                                         s[tp] = gmfma(R[sTab[tabS + 16 * tp * TW + 4 * kt]], b, s[tp]);
@@ -252,16 +246,16 @@ namespace lbx
                                 // keep the phases apart: left alone the scheduler fetches all their operands
                                 // first, and the registers for that cost more than the latency
                                 __builtin_amdgcn_sched_barrier(0);
-                                Acc qa[TQ];
+                                v4d qa[TQ];
 #pragma unroll
                                 for (int tq = 0; tq < TQ; tq++)
-                                    qa[tq] = Acc{0, 0, 0, 0};
+                                    qa[tq] = v4d{0, 0, 0, 0};
 #pragma unroll
                                 for (int kt = 0; kt < KP; kt++)
                                 {
 #pragma unroll
                                     for (int tq = 0; tq < TQ; tq++)
-                                        qa[tq] = gmfma(R[sTab[tabQ + rowBase(kt) * TW + 16 * tq]], y[kt >> 2][kt & 3], qa[tq]);
+                                        qa[tq] = gmfma(R[sTab[tabQ + 4 * kt * TW + 16 * tq]], y[kt >> 2][kt & 3], qa[tq]);
                                 }
                                 // V
 #pragma unroll
@@ -269,8 +263,8 @@ namespace lbx
 #pragma unroll
                                     for (int r = 0; r < 4; r++)
                                     {
-                                        const int gg = rowBase(4 * tq + r);
-                                        const bool in = gg + rowLane < HQ && inC;
+                                        const int gg = 4 * (4 * tq + r);
+                                        const bool in = gg + g4 < HQ && inC;
                                         const double qv = qa[tq][r];
 #pragma unroll
                                         for (int x = 0; x < 3; x++)
@@ -288,11 +282,11 @@ namespace lbx
 #pragma unroll
                                     for (int r = 0; r < 4; r++)
                                     {
-                                        const unsigned short *dn = sDn[rowBase(4 * tp + r) + rk];
+                                        const unsigned short *dn = sDn[4 * (4 * tp + r) + rk];
                                         const double sv = s[tp][r];
 #pragma unroll
                                         for (int x = 0; x < 3; x++)
-                                            d[x] = fma(sv, static_cast<double>(sY[dn[x] + jk]), d[x]);
+                                            d[x] = fma(sv, sY[dn[x] + jk], d[x]);
                                     }
                                 }
                                 const double rc = UP.ra[kp];   // c / q
@@ -315,20 +309,20 @@ namespace lbx
 #pragma unroll
                                 for (int ts = 0; ts < TS; ts++)
                                 {
-                                    Acc gx = Acc{0, 0, 0, 0};
+                                    v4d gx = v4d{0, 0, 0, 0};
                                     const int ab = 16 * ts + j;
 #pragma unroll
                                     for (int kt = 0; kt < KP; kt++)
                                     {
-                                        const int h = rowBase(kt);
-                                        const bool in = h + rowLane < HP && ab < SP;
-                                        const T a = in ? (e1b + (x * HP + h) * SP + 16 * ts)[e1bOff] : T(0);
+                                        const int h = 4 * kt;
+                                        const bool in = h + g4 < HP && ab < SP;
+                                        const double a = in ? (e1b + (x * HP + h) * SP + 16 * ts)[e1bOff] : T(0);
                                         gx = gmfma(a, s[kt >> 2][kt & 3], gx);
                                     }
 #pragma unroll
                                     for (int r = 0; r < 4; r++)
                                         if (4 * ts + r < KS)
-                                            ux = fma(static_cast<double>(gx[r]), static_cast<double>(wB[4 * ts + r]), ux);
+                                            ux = fma(gx[r], wB[4 * ts + r], ux);
                                 }
                                 gA[x] += ux;
                                 gB[x] -= ux;

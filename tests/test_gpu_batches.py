@@ -78,6 +78,37 @@ def test_jk_grad_uneven_contractions(lbx, oracle, contractions):
     close(g.cpu().numpy(), ref, rel=1e-10, floor=1e-10)
 
 
+@pytest.mark.parametrize("contractions", [[(2, 5), (3, 2)], [(2, 9)], [(3, 4), (2, 1), (3, 1)]])
+def test_jk_grad_fp32_sums(lbx, contractions):
+    """The FP32 tier sums over primitives in FP64 (class pairs of d and f shells: the one-wave form):
+    every primitive listed twice with half its coefficient is the same function, its E matrices scale
+    by exact powers of two, and the gradients differ by the rounding of FP64 sums of up to 1e6 terms
+    that cancel to about a tenth: 1e-11 of the largest component (FP32 sums: 1e-8 and more).  Against
+    FP64: R and E rounded to FP32, about 20 roundings of 6e-8 per term: 1e-5 of the largest component."""
+    import torch
+    m = uneven_molecule(7, contractions)
+
+    def doubled(exps, coeffs, nprim):
+        e, c, at = [], [], 0
+        for k in nprim:
+            e += [np.tile(exps[at:at + k], 2)]
+            c += [np.tile(0.5 * coeffs[at:at + k], 2)]
+            at += k
+        return np.concatenate(e), np.concatenate(c)
+
+    sh = m.shells
+    e2, c2 = doubled(sh.exps, sh.coeffs, sh.nprim)
+    m2 = B.Molecule(m.coords, B.Shells(sh.atom, sh.l, 2 * sh.nprim, e2, c2))
+    D = torch.tensor(B.density_from_orbitals(4, m.shells.nbf, 3, 0.3), device="cuda")
+    mixed = dict(schwarz=0.0, precision=lbx.LBX_MIXED, mixed_thresh=1e30)
+    ref, _ = lbx.Context(m).jk_grad(D, schwarz=0.0)
+    g, st = lbx.Context(m).jk_grad(D, **mixed)
+    g2, _ = lbx.Context(m2).jk_grad(D, **mixed)
+    assert st["quartets_fp32"] == st["quartets"]
+    close(g2.cpu().numpy(), g.cpu().numpy(), rel=0.0, floor=1e-11)
+    close(g.cpu().numpy(), ref.cpu().numpy(), rel=0.0, floor=1e-5)
+
+
 @pytest.mark.parametrize("natoms", [1, 3, 16])
 def test_dense_uneven(lbx, oracle, natoms):
     """Dense eri4 / diagonal of 1 to 16 one-shell atoms (the largest has more pairs than lanes)."""
