@@ -145,8 +145,8 @@ int lbx_jk(lbx_context *ctx, const double *D, double *J, double *K, double schwa
  * reference's eri3() / eri2(), eri3.cpp:7-46, eri2.cpp:27-72): with V = (P|Q) = L L^T,
  *   J_mn = sum_PQ (mn|P) (V^-1)_PQ sum_kl (Q|kl) D_kl
  *   K_mk = sum_P sum_nl W_P(mn) D_nl W_P(kl),   W_P = sum_Q (L^-1)_PQ (Q|..)
- * D, J, K: device (nbf, nbf) row-major, D symmetric; K may be NULL (J only).  Needs an
- * auxiliary basis.  The first call builds the fitted 3-index tensor W (8 nbf^2 naux bytes of
+ * D, J, K: device (nbf, nbf) row-major; K may be NULL (J only).  D need not be symmetric (then
+ * neither is K, which takes a third more work).  Needs an auxiliary basis.  The first call builds the fitted 3-index tensor W (8 nbf^2 naux bytes of
  * device memory, plus a work buffer of the same size while it is built or once K is asked for)
  * and the context keeps both until lbx_destroy, so later calls (an SCF loop) cost only the
  * products with D.  LBX_ERR_NOMEM when they do not fit; LBX_ERR_STATE when (P|Q) is not

@@ -121,6 +121,7 @@ namespace lbx
         // built on the first lbx_ri_jk call and kept, and the exchange work buffer (same size,
         // made on the first call with K); both in allocations
         double *ri_w = nullptr, *ri_t = nullptr, *ri_h = nullptr;   // ri_h: naux doubles
+        int *ri_flags = nullptr;                                    // whether D is symmetric
         bool ri_ready = false;
         std::mutex ri_mu;
 

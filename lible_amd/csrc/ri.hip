@@ -3,7 +3,7 @@
 // eri2.cpp:27-72; the reference has no J/K build).  With B_P(mn) = (mn|P), V = (P|Q) = L L^T
 // and the fitted tensor W_P = sum_Q (L^-1)_PQ B_Q (so that sum_P W_P W_P^T = B V^-1 B^T):
 //   J = sum_P W_P h_P,   h_P = sum_mn W_P(mn) D_mn
-//   K = sum_P W_P D W_P
+//   K = sum_P W_P D W_P   (also of a D that is not symmetric)
 // W depends on the geometry only: the first call builds it (eri3, a transpose to P-major, eri2,
 // the Cholesky factorisation, one triangular solve) and the context keeps it, so every later
 // call (an SCF iteration) costs one or two passes over W for J and, for K, the products
@@ -109,9 +109,36 @@ namespace lbx
                 p[i] = 0.0;
         }
 
-        // upper triangle from the lower one
-        __global__ void mirrorKernel(double *K, int n)
+        // Whether D is symmetric to rounding, per block: flags[blockIdx.x] = 1 where it is not.  K is then
+        // not symmetric either, and its upper triangle is made too.
+        __global__ __launch_bounds__(256) void asymmetryKernel(const double *__restrict__ D, int n, int *flags)
         {
+            const long long tot = static_cast<long long>(n) * n;
+            bool differ = false;
+            for (long long e = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x; e < tot;
+                 e += static_cast<long long>(gridDim.x) * 256)
+            {
+                const int i = static_cast<int>(e / n), j = static_cast<int>(e % n);
+                if (j < i)
+                {
+                    const double a = D[e], b = D[static_cast<long long>(j) * n + i];
+                    differ |= fabs(a - b) > 1e-14 * fmax(fabs(a), fabs(b));
+                }
+            }
+            const int any = __syncthreads_or(differ);
+            if (threadIdx.x == 0)
+                flags[blockIdx.x] = any;
+        }
+
+        // the flags of asymmetryKernel's kFlagBlocks workgroups (all 256 threads call)
+        constexpr int kFlagBlocks = 256;
+        __device__ __forceinline__ bool asymmetric(const int *flags) { return __syncthreads_or(flags[threadIdx.x]); }
+
+        // upper triangle from the lower one, unless it has been made (D not symmetric)
+        __global__ __launch_bounds__(256) void mirrorKernel(double *K, int n, const int *flags)
+        {
+            if (asymmetric(flags))
+                return;
             const long long tot = static_cast<long long>(n) * n;
             for (long long e = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; e < tot;
                  e += static_cast<long long>(gridDim.x) * blockDim.x)
@@ -131,13 +158,15 @@ namespace lbx
         //     blockIdx.y = P)
         //   SPLIT = true:  K = sum_P T_P W_P^T with k = (P, l) running over n naux: for a small n
         //     the n x n tiles alone leave the chip idle (nine tiles at n = 192), so k is split over
-        //     gridDim.y workgroups per tile that add into C by atomics, and only the tiles with
-        //     row >= column are made (K is symmetric).
+        //     gridDim.y workgroups per tile that add into C by atomics.  The tiles with row >= column
+        //     come first (K of a symmetric D is symmetric), then the others, which return at once
+        //     unless the flags say that D is not symmetric.
         // At n = 192, naux = 904 (k = 1.7e5) a J and K call takes 0.68 ms, 38 TFLOP/s over both
         // products (library GEMMs, whose few tiles left the chip idle: 19.5 ms).
         template <bool SPLIT>
         __global__ __launch_bounds__(256) void panelGemm(const double *__restrict__ A, const double *__restrict__ B,
-                                                         double *__restrict__ C, int n, long long kTotal, long long kChunk)
+                                                         double *__restrict__ C, int n, long long kTotal, long long kChunk,
+                                                         int splits, const int *flags)
         {
             const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
             const int g = lane >> 4, j = lane & 15;
@@ -146,14 +175,28 @@ namespace lbx
             long long k0, k1;
             if constexpr (SPLIT)
             {
-                // blockIdx.y = lower-triangle tile, blockIdx.x = split: the tiles of one split are
-                // gridDim.x apart (a multiple of 8), so one XCD's L2 serves them
-                tr = 0;
-                int t = blockIdx.y;
-                while (t > tr)
-                    t -= ++tr;
-                tc = t;
-                k0 = blockIdx.x * kChunk;
+                // the tiles of one split are `splits` workgroups apart (a multiple of 8), so one XCD's
+                // L2 serves them
+                const int tile = blockIdx.x / splits, lower = nt * (nt + 1) / 2;
+                if (tile < lower)
+                {
+                    int t = tile;
+                    tr = 0;
+                    while (t > tr)
+                        t -= ++tr;
+                    tc = t;
+                }
+                else
+                {
+                    if (!asymmetric(flags))
+                        return;
+                    int t = tile - lower;
+                    tc = 1;
+                    while (t >= tc)
+                        t -= tc++;
+                    tr = t;
+                }
+                k0 = (blockIdx.x % splits) * kChunk;
                 k1 = min(kTotal, k0 + kChunk);
             }
             else
@@ -278,6 +321,8 @@ namespace lbx
         const long long n2 = n * n;
         if (K && !c.ri_t)
             c.ri_t = c.alloc<double>(static_cast<size_t>(n2 * naux));
+        if (K && !c.ri_flags)
+            c.ri_flags = c.alloc<int>(kFlagBlocks);
         if (!c.ri_ready)
         {
             Handle h(stream);
@@ -335,14 +380,15 @@ namespace lbx
         auto blocks1d = [](long long m) { return dim3(static_cast<int>(std::min<long long>((m + 255) / 256, 65536))); };
         if (K)
         {
-            // T_P = W_P D (W_P and D symmetric, so row- and column-major readings agree); blockIdx.y
-            // holds at most 65535 auxiliary functions
+            hipLaunchKernelGGL(asymmetryKernel, dim3(kFlagBlocks), dim3(256), 0, stream, D, ni, c.ri_flags);
+            // T_P = D^T W_P as panelGemm reads its operands; blockIdx.y holds at most 65535 auxiliary
+            // functions
             const int nt = (ni + 63) / 64;
             for (long long p0 = 0; p0 < naux; p0 += 65535)
             {
                 const int np = static_cast<int>(std::min<long long>(65535, naux - p0));
                 hipLaunchKernelGGL((panelGemm<false>), dim3(nt * nt, np), dim3(256), 0, stream, D, c.ri_w + p0 * n2,
-                                   c.ri_t + p0 * n2, ni, n, n);
+                                   c.ri_t + p0 * n2, ni, n, n, 1, nullptr);
             }
             // K = sum_P T_P W_P^T
             hipLaunchKernelGGL(zeroKernel, blocks1d(n2), dim3(256), 0, stream, K, n2);
@@ -351,9 +397,9 @@ namespace lbx
             splits = std::min(splits, (kTotal + 255) / 256);   // at least 256 k per workgroup
             splits = (splits + 7) / 8 * 8;
             const long long chunk = ((kTotal + splits - 1) / splits + 15) / 16 * 16;
-            hipLaunchKernelGGL((panelGemm<true>), dim3(static_cast<int>(splits), static_cast<int>(tiles)), dim3(256), 0,
-                               stream, c.ri_t, c.ri_w, K, ni, kTotal, chunk);
-            hipLaunchKernelGGL(mirrorKernel, blocks1d(n2), dim3(256), 0, stream, K, ni);
+            hipLaunchKernelGGL((panelGemm<true>), dim3(static_cast<unsigned>(splits * nt * nt)), dim3(256), 0, stream,
+                               c.ri_t, c.ri_w, K, ni, kTotal, chunk, static_cast<int>(splits), c.ri_flags);
+            hipLaunchKernelGGL(mirrorKernel, blocks1d(n2), dim3(256), 0, stream, K, ni, c.ri_flags);
             hipLaunchKernelGGL(fitTraceKernel, dim3(static_cast<int>(naux)), dim3(256), 0, stream, c.ri_t, c.ri_h, n);
         }
         else

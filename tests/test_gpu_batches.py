@@ -141,20 +141,24 @@ def test_eri4_block_orders(lbx, block_case, ls, perm):
     close(got, ref, floor=1e-13 * np.abs(e4).max() / np.abs(ref).max())
 
 
-@pytest.mark.parametrize("nmain,naux", [(1, 1), (5, 3), (63, 7), (64, 2), (65, 9), (130, 5)])
-def test_ri_jk_sizes(lbx, oracle, nmain, naux):
-    """Density-fitted J and K at sizes around the 64 x 64 tiles and 16-step k loop, against numpy on
-    the library's own eri3 / eri2 (pinned to the oracle elsewhere).  s shells spread over a line, a
-    well-conditioned auxiliary set: 1e-11 of the largest element."""
-    import torch
-    from scipy.linalg import cho_solve, solve_triangular
+def ri_line_molecule(nmain, naux):
+    """s shells spread over a line, a well-conditioned auxiliary set."""
     rng = np.random.default_rng(nmain)
     nat = max(nmain, naux)
     coords = np.stack([1.5 * np.arange(nat), rng.uniform(0, 1, nat), rng.uniform(0, 1, nat)], 1)
     main = B.Shells.from_lists([[(0, [0.8], [1.0])] if k < nmain else [] for k in range(nat)])
     aux = B.Shells.from_lists([[(0, [1.1], [1.0])] if k < naux else [] for k in range(nat)])
-    m = B.Molecule(coords, main, aux)
-    ctx = lbx.Context(m)
+    return B.Molecule(coords, main, aux)
+
+
+@pytest.mark.parametrize("nmain,naux", [(1, 1), (5, 3), (63, 7), (64, 2), (65, 9), (130, 5)])
+def test_ri_jk_sizes(lbx, oracle, nmain, naux):
+    """Density-fitted J and K at sizes around the 64 x 64 tiles and 16-step k loop, against numpy on
+    the library's own eri3 / eri2 (pinned to the oracle elsewhere): 1e-11 of the
+    largest element."""
+    import torch
+    from scipy.linalg import cho_solve, solve_triangular
+    ctx = lbx.Context(ri_line_molecule(nmain, naux))
     e3, e2 = ctx.eri3().cpu().numpy(), ctx.eri2().cpu().numpy()
     D = B.density_from_orbitals(2, nmain, 4, 0.3)
     L = np.linalg.cholesky(e2)
@@ -167,6 +171,25 @@ def test_ri_jk_sizes(lbx, oracle, nmain, naux):
         close(K.cpu().numpy(), Kr, rel=0.0, floor=1e-11)
     J, _ = ctx.ri_jk(torch.tensor(D, device="cuda"), exchange=False)
     close(J.cpu().numpy(), Jr, rel=0.0, floor=1e-11)
+
+
+@pytest.mark.parametrize("nmain,naux", [(5, 3), (65, 9), (130, 5)])
+def test_ri_jk_density_not_symmetric(lbx, nmain, naux):
+    """J and K of a density that is not symmetric (all of it, or one element of it), in both triangles;
+    tolerance as above."""
+    import torch
+    from scipy.linalg import solve_triangular
+    ctx = lbx.Context(ri_line_molecule(nmain, naux))
+    e3, e2 = ctx.eri3().cpu().numpy(), ctx.eri2().cpu().numpy()
+    W = solve_triangular(np.linalg.cholesky(e2), e3.reshape(nmain * nmain, naux).T, lower=True).reshape(naux, nmain, nmain)
+    one = B.density_from_orbitals(2, nmain, 4, 0.3)
+    one[0, nmain - 1] += 0.5
+    for D in (np.random.default_rng(3).normal(size=(nmain, nmain)), one):
+        Jr = np.einsum("pmn,p->mn", W, np.einsum("pmn,mn->p", W, D))
+        Kr = np.einsum("pmn,nl,pkl->mk", W, D, W, optimize=True)
+        J, K = ctx.ri_jk(torch.tensor(D, device="cuda"))
+        close(J.cpu().numpy(), Jr, rel=0.0, floor=1e-11)
+        close(K.cpu().numpy(), Kr, rel=0.0, floor=1e-11)
 
 
 @pytest.mark.parametrize("ns", [14, 15, 16, 19, 23])
