@@ -122,6 +122,7 @@ namespace lbx
         // made on the first call with K); both in allocations
         double *ri_w = nullptr, *ri_t = nullptr, *ri_h = nullptr;   // ri_h: naux doubles
         int *ri_flags = nullptr;                                    // whether D is symmetric
+        double *ri_part = nullptr;                                  // parts of K and of J
         bool ri_ready = false;
         std::mutex ri_mu;
 

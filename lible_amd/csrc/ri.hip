@@ -87,9 +87,9 @@ namespace lbx
                 h[blockIdx.x] = s;
         }
 
-        // J += sum over the P of group blockIdx.y of W_P h_P
+        // out = sum over the P of group blockIdx.y of W_P h_P; each group has an n2-sized output of its own
         __global__ __launch_bounds__(256) void fitCoulombKernel(const double *__restrict__ W, const double *__restrict__ h,
-                                                                double *__restrict__ J, long long n2, int naux, int group)
+                                                                double *__restrict__ out, long long n2, int naux, int group)
         {
             const long long i = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
             if (i >= n2)
@@ -99,14 +99,21 @@ namespace lbx
 #pragma unroll 8
             for (int p = p0; p < p1; p++)
                 s = fma(W[p * n2 + i], h[p], s);
-            unsafeAtomicAdd(&J[i], s);
+            out[blockIdx.y * n2 + i] = s;
         }
 
-        __global__ void zeroKernel(double *p, long long n)
+        // out[i] = sum of the groups' outputs, in order
+        __global__ __launch_bounds__(256) void sumGroupsKernel(const double *__restrict__ in, double *__restrict__ out,
+                                                               long long n2, int groups)
         {
-            for (long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-                 i += static_cast<long long>(gridDim.x) * blockDim.x)
-                p[i] = 0.0;
+            const long long i = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
+            if (i >= n2)
+                return;
+            double s = 0.0;
+#pragma unroll 8
+            for (int g = 0; g < groups; g++)
+                s += in[g * n2 + i];
+            out[i] = s;
         }
 
         // Whether D is symmetric to rounding, per block: flags[blockIdx.x] = 1 where it is not.  K is then
@@ -134,6 +141,59 @@ namespace lbx
         constexpr int kFlagBlocks = 256;
         __device__ __forceinline__ bool asymmetric(const int *flags) { return __syncthreads_or(flags[threadIdx.x]); }
 
+        // tile number -> tile: the tiles with row >= column first, then the others
+        __device__ __forceinline__ void tileOf(int tile, int nt, int &tr, int &tc)
+        {
+            const int lower = nt * (nt + 1) / 2;
+            if (tile < lower)
+            {
+                int t = tile;
+                tr = 0;
+                while (t > tr)
+                    t -= ++tr;
+                tc = t;
+            }
+            else
+            {
+                int t = tile - lower;
+                tc = 1;
+                while (t >= tc)
+                    t -= tc++;
+                tr = t;
+            }
+        }
+
+        // K from the splits' parts of each 64 x 64 tile, added in order (one workgroup per row of a tile,
+        // its waves a quarter of the splits each); the upper triangle from the lower one unless D is not
+        // symmetric.
+        __global__ __launch_bounds__(256) void sumTilesKernel(const double *__restrict__ parts, double *__restrict__ K, int n,
+                                                              int splits, const int *flags)
+        {
+            const bool full = asymmetric(flags);
+            const int nt = (n + 63) / 64, tile = blockIdx.x / 64, r = blockIdx.x % 64;
+            if (!full && tile >= nt * (nt + 1) / 2)
+                return;
+            int tr, tc;
+            tileOf(tile, nt, tr, tc);
+            __shared__ double quarter[4][64];
+            const int j = threadIdx.x & 63, w = threadIdx.x >> 6;
+            const int s0 = splits * w / 4, s1 = splits * (w + 1) / 4;
+            const double *in = parts + (static_cast<long long>(tile) * splits * 64 + r) * 64 + j;
+            double v = 0.0;
+#pragma unroll 8
+            for (int k = s0; k < s1; k++)
+                v += in[k * 4096LL];
+            quarter[w][j] = v;
+            __syncthreads();
+            const int row = tr * 64 + r, col = tc * 64 + j;
+            if (w > 0 || row >= n || col >= n || (!full && col > row))
+                return;
+            v = (quarter[0][j] + quarter[1][j]) + (quarter[2][j] + quarter[3][j]);
+            K[static_cast<long long>(row) * n + col] = v;
+            if (!full)
+                K[static_cast<long long>(col) * n + row] = v;
+        }
+
         // upper triangle from the lower one, unless it has been made (D not symmetric)
         __global__ __launch_bounds__(256) void mirrorKernel(double *K, int n, const int *flags)
         {
@@ -158,9 +218,11 @@ namespace lbx
         //     blockIdx.y = P)
         //   SPLIT = true:  K = sum_P T_P W_P^T with k = (P, l) running over n naux: for a small n
         //     the n x n tiles alone leave the chip idle (nine tiles at n = 192), so k is split over
-        //     gridDim.y workgroups per tile that add into C by atomics.  The tiles with row >= column
-        //     come first (K of a symmetric D is symmetric), then the others, which return at once
-        //     unless the flags say that D is not symmetric.
+        //     `splits` workgroups per tile, each with a part of its own that sumTilesKernel adds up
+        //     (atomics into K took the same time and made its last bits differ from call to call);
+        //     one split: C is K itself.  The tiles with row >= column come first (K of a symmetric D
+        //     is symmetric), then the others, which return at once unless the flags say that D is not
+        //     symmetric.
         // At n = 192, naux = 904 (k = 1.7e5) a J and K call takes 0.68 ms, 38 TFLOP/s over both
         // products (library GEMMs, whose few tiles left the chip idle: 19.5 ms).
         template <bool SPLIT>
@@ -177,25 +239,10 @@ namespace lbx
             {
                 // the tiles of one split are `splits` workgroups apart (a multiple of 8), so one XCD's
                 // L2 serves them
-                const int tile = blockIdx.x / splits, lower = nt * (nt + 1) / 2;
-                if (tile < lower)
-                {
-                    int t = tile;
-                    tr = 0;
-                    while (t > tr)
-                        t -= ++tr;
-                    tc = t;
-                }
-                else
-                {
-                    if (!asymmetric(flags))
-                        return;
-                    int t = tile - lower;
-                    tc = 1;
-                    while (t >= tc)
-                        t -= tc++;
-                    tr = t;
-                }
+                const int tile = blockIdx.x / splits;
+                if (tile >= nt * (nt + 1) / 2 && !asymmetric(flags))
+                    return;
+                tileOf(tile, nt, tr, tc);
                 k0 = (blockIdx.x % splits) * kChunk;
                 k1 = min(kTotal, k0 + kChunk);
             }
@@ -260,6 +307,9 @@ namespace lbx
                 }
             }
             // accumulator element r of lane (g, j): row 4 r + g, column j
+            const bool parts = SPLIT && splits > 1;
+            if (parts)
+                C += blockIdx.x * 4096LL;
 #pragma unroll
             for (int x = 0; x < 2; x++)
 #pragma unroll
@@ -268,14 +318,10 @@ namespace lbx
                     for (int r = 0; r < 4; r++)
                     {
                         const int row = r0 + 16 * x + 4 * r + g, col = c0 + 16 * y + j;
-                        if (row < n && col < n)
-                        {
-                            double *dst = &C[static_cast<long long>(row) * n + col];
-                            if constexpr (SPLIT)
-                                unsafeAtomicAdd(dst, acc[x][y][r]);
-                            else
-                                *dst = acc[x][y][r];
-                        }
+                        if (parts)
+                            C[(row & 63) * 64 + (col & 63)] = acc[x][y][r];
+                        else if (row < n && col < n)
+                            C[static_cast<long long>(row) * n + col] = acc[x][y][r];
                     }
         }
 
@@ -377,6 +423,34 @@ namespace lbx
             c.ri_ready = true;
         }
         const int ni = static_cast<int>(n);
+        // K in splits of k, so that about 1024 workgroups share it, at least 256 k each; J in groups of
+        // P, so that about 2048 share the pass over W
+        const long long nt2 = (n + 63) / 64 * ((n + 63) / 64), tiles = (nt2 + (n + 63) / 64) / 2;
+        long long splits = std::min(std::max<long long>(1, 1024 / tiles), (n * naux + 255) / 256);
+        splits = (splits + 7) / 8 * 8;
+        long long jGroup = std::max<long long>(8, naux * ((n2 + 255) / 256) / 2048);
+        if (!c.ri_part)
+        {
+            // one buffer for the parts of K, then of J: up to 80 MiB at 1000 functions, 8 nbf^2 values
+            // where tiles are many.  Without it K and J are made in one part.
+            void *p = nullptr;
+            const long long parts = std::max(nt2 * splits * 4096, (naux + jGroup - 1) / jGroup * n2);
+            const hipError_t e = hipMalloc(&p, sizeof(double) * parts);
+            if (e == hipSuccess)
+            {
+                c.allocations.push_back(p);
+                c.ri_part = static_cast<double *>(p);
+            }
+            else if (e != hipErrorOutOfMemory)
+                LBX_HIP(e);
+            else
+                (void)hipGetLastError();
+        }
+        if (!c.ri_part)
+        {
+            splits = 1;
+            jGroup = naux;
+        }
         auto blocks1d = [](long long m) { return dim3(static_cast<int>(std::min<long long>((m + 255) / 256, 65536))); };
         if (K)
         {
@@ -391,26 +465,26 @@ namespace lbx
                                    c.ri_t + p0 * n2, ni, n, n, 1, nullptr);
             }
             // K = sum_P T_P W_P^T
-            hipLaunchKernelGGL(zeroKernel, blocks1d(n2), dim3(256), 0, stream, K, n2);
-            const long long tiles = static_cast<long long>(nt) * (nt + 1) / 2, kTotal = n * naux;
-            long long splits = std::max<long long>(1, 1024 / tiles);
-            splits = std::min(splits, (kTotal + 255) / 256);   // at least 256 k per workgroup
-            splits = (splits + 7) / 8 * 8;
+            const long long kTotal = n * naux;
             const long long chunk = ((kTotal + splits - 1) / splits + 15) / 16 * 16;
             hipLaunchKernelGGL((panelGemm<true>), dim3(static_cast<unsigned>(splits * nt * nt)), dim3(256), 0, stream,
-                               c.ri_t, c.ri_w, K, ni, kTotal, chunk, static_cast<int>(splits), c.ri_flags);
-            hipLaunchKernelGGL(mirrorKernel, blocks1d(n2), dim3(256), 0, stream, K, ni, c.ri_flags);
+                               c.ri_t, c.ri_w, splits > 1 ? c.ri_part : K, ni, kTotal, chunk, static_cast<int>(splits),
+                               c.ri_flags);
+            if (splits > 1)
+                hipLaunchKernelGGL(sumTilesKernel, dim3(nt * nt * 64), dim3(256), 0, stream, c.ri_part, K, ni,
+                                   static_cast<int>(splits), c.ri_flags);
+            else
+                hipLaunchKernelGGL(mirrorKernel, blocks1d(n2), dim3(256), 0, stream, K, ni, c.ri_flags);
             hipLaunchKernelGGL(fitTraceKernel, dim3(static_cast<int>(naux)), dim3(256), 0, stream, c.ri_t, c.ri_h, n);
         }
         else
             hipLaunchKernelGGL(fitDotKernel, dim3(static_cast<int>(naux)), dim3(256), 0, stream, c.ri_w, D, c.ri_h, n2);
         {
-            // J: groups of P so that about 2048 workgroups share the pass over W
-            const long long bx = (n2 + 255) / 256;
-            const int group = static_cast<int>(std::max<long long>(8, naux * bx / 2048));
-            hipLaunchKernelGGL(zeroKernel, blocks1d(n2), dim3(256), 0, stream, J, n2);
-            hipLaunchKernelGGL(fitCoulombKernel, dim3(static_cast<int>(bx), static_cast<int>((naux + group - 1) / group)),
-                               dim3(256), 0, stream, c.ri_w, c.ri_h, J, n2, static_cast<int>(naux), group);
+            const int bx = static_cast<int>((n2 + 255) / 256), groups = static_cast<int>((naux + jGroup - 1) / jGroup);
+            hipLaunchKernelGGL(fitCoulombKernel, dim3(bx, groups), dim3(256), 0, stream, c.ri_w, c.ri_h,
+                               groups > 1 ? c.ri_part : J, n2, static_cast<int>(naux), static_cast<int>(jGroup));
+            if (groups > 1)
+                hipLaunchKernelGGL(sumGroupsKernel, dim3(bx), dim3(256), 0, stream, c.ri_part, J, n2, groups);
         }
         LBX_HIP(hipGetLastError());
         LBX_HIP(hipStreamSynchronize(stream));

@@ -192,6 +192,20 @@ def test_ri_jk_density_not_symmetric(lbx, nmain, naux):
         close(K.cpu().numpy(), Kr, rel=0.0, floor=1e-11)
 
 
+@pytest.mark.parametrize("nmain,naux", [(30, 56), (65, 200), (180, 90)])
+def test_ri_jk_repeats(lbx, nmain, naux):
+    """The same density gives the same bits again (K and J are added up from parts in a fixed order)."""
+    import torch
+    ctx = lbx.Context(ri_line_molecule(nmain, naux))
+    D = torch.tensor(B.density_from_orbitals(2, nmain, 4, 0.3), device="cuda")
+    J, K = ctx.ri_jk(D)
+    Jo, _ = ctx.ri_jk(D, exchange=False)
+    for _ in range(5):
+        J2, K2 = ctx.ri_jk(D)
+        assert torch.equal(J, J2) and torch.equal(K, K2)
+        assert torch.equal(Jo, ctx.ri_jk(D, exchange=False)[0])
+
+
 @pytest.mark.parametrize("ns", [14, 15, 16, 19, 23])
 @pytest.mark.parametrize("variant", [0, 1, 3, 4])
 def test_jk_one_lane_pair_counts(lbx, oracle, ns, variant):
