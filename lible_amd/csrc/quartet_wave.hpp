@@ -479,7 +479,7 @@ namespace lbx
 
     // The one-wave forms of a class pair: FP64 in every mode, FP32 for J/K (FORMS as in
     // registerQuartet).  For J/K they also stand in for the one-lane forms that would fit the
-    // registers but are not built (Cls::laneBuilt).
+    // registers but are not built (Cls::laneBuilt; main shells to f only).
     template <int LA, int LB, int LC, int LD, int MODE, int FORMS = 3>
     void registerWave()
     {
@@ -495,9 +495,9 @@ namespace lbx
         if constexpr (FORMS & 1)
         {
             put(VAR_MFMA, &launchMfma<LA, LB, LC, LD, MODE>);
-            if constexpr (MODE == MODE_JK && C::NC0 > 0 && !C::kLane0)
+            if constexpr (MODE == MODE_JK && LA <= 3 && C::NC0 > 0 && !C::kLane0)
                 put(VAR_VALU_BRA, &launchMfma<LA, LB, LC, LD, MODE>);
-            if constexpr (MODE == MODE_JK && C::NC1 > 0 && !C::kLane1 && !same)
+            if constexpr (MODE == MODE_JK && LA <= 3 && C::NC1 > 0 && !C::kLane1 && !same)
                 put(VAR_VALU_KET, &launchMfma<LA, LB, LC, LD, MODE>);
         }
         if constexpr ((FORMS & 2) && MODE == MODE_JK)

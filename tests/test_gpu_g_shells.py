@@ -58,6 +58,16 @@ def test_g_jk(lbx, oracle):
     assert abs(dE) <= 1e-9, dE
 
 
+def test_g_variants(lbx):
+    """A class pair with a main g shell has one J/K form (2): every other number is refused."""
+    ctx = lbx.Context(B.synthetic_molecule(402, 1, 4.5, RECIPE_G))
+    pairs = [(l, m) for l in range(5) for m in range(l + 1)]
+    for i, bra in enumerate(pairs):
+        for ket in pairs[:i + 1]:
+            if bra[0] == 4:
+                assert [v for v in range(8) if ctx.set_variant(bra + ket, v)] == [2], (bra, ket)
+
+
 def test_g_eri3_eri2_sums(lbx, oracle):
     """(ab|P) with g main shells against h auxiliary shells, (P|Q), and the per-molecule sums."""
     m = B.synthetic_molecule(403, 2, 3.5, RECIPE_G1, RECIPE_AUX_H)
