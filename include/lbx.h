@@ -55,6 +55,10 @@ int lbx_dims(const lbx_context *ctx, long *nbf, long *nbf_aux, long *natoms);
 /* All work of a context is queued on this stream (default: the null stream).  hipStream_t. */
 int lbx_set_stream(lbx_context *ctx, void *stream);
 int lbx_synchronize(lbx_context *ctx);
+/* Upper bound on the device memory that the context holds between calls (bytes; 0: none, the
+ * default).  A call that would go past it returns LBX_ERR_NOMEM, as when the device is full, and
+ * the context stays usable: a later call with more room gives the same results. */
+int lbx_set_memory_limit(lbx_context *ctx, long bytes);
 
 /* Boys function F_0..F_n at count points (device x[count] -> device out[count*(n+1)]).
  * Replaces calcBoysF (boys_function.cpp:71-117); n <= 17. */

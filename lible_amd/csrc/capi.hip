@@ -342,13 +342,13 @@ namespace lbx
             {
                 throw Error(LBX_ERR_STATE, e.what());
             }
-            t.nblk = b.nblk;
             t.gshift = gshift;
             t.bprefix = std::move(b.bprefix);
             t.bq0 = std::move(b.bq0);
             t.btasks = b.ntasks;
             t.d_bprefix = c.stage(t.bprefix);
             t.d_bq0 = c.stage(t.bq0);
+            t.nblk = b.nblk;   // the table is there (staging may run out of memory)
             return b.quartets;
         }
 
@@ -557,6 +557,19 @@ namespace lbx
                 out[i] = static_cast<float>(in[i]);
         }
 
+        // FP32 copies b32, k32 of n doubles each; b32, whose presence says that both are there, last
+        void toFloat(Context &c, const double *b, const double *k, float *&b32, float *&k32, long long n)
+        {
+            if (!k32)
+                k32 = c.alloc<float>(n);
+            float *out = c.alloc<float>(n);
+            const int grid = static_cast<int>(std::min<long long>((n + 255) / 256, 65536));
+            hipLaunchKernelGGL(toFloatKernel, dim3(grid), dim3(256), 0, c.stream, b, out, n);
+            hipLaunchKernelGGL(toFloatKernel, dim3(grid), dim3(256), 0, c.stream, k, k32, n);
+            LBX_HIP(hipGetLastError());
+            b32 = out;
+        }
+
         // FP32 copies of the E matrices, made once per context on first mixed-precision use
         void ensureF32(Context &c)
         {
@@ -564,13 +577,7 @@ namespace lbx
             {
                 if (pc.d_eb32 || pc.n_ppairs == 0)
                     continue;
-                const long long n = static_cast<long long>(pc.eCount());
-                pc.d_eb32 = c.alloc<float>(n);
-                pc.d_ek32 = c.alloc<float>(n);
-                const int grid = static_cast<int>(std::min<long long>((n + 255) / 256, 65536));
-                hipLaunchKernelGGL(toFloatKernel, dim3(grid), dim3(256), 0, c.stream, pc.d_eb, pc.d_eb32, n);
-                hipLaunchKernelGGL(toFloatKernel, dim3(grid), dim3(256), 0, c.stream, pc.d_ek, pc.d_ek32, n);
-                LBX_HIP(hipGetLastError());
+                toFloat(c, pc.d_eb, pc.d_ek, pc.d_eb32, pc.d_ek32, static_cast<long long>(pc.eCount()));
             }
         }
 
@@ -581,13 +588,7 @@ namespace lbx
             {
                 if (pc.d_eb32 || pc.n_ppairs == 0)
                     continue;
-                const long long n = static_cast<long long>(pc.eCount());
-                pc.d_eb32 = c.alloc<float>(n);
-                pc.d_ek32 = c.alloc<float>(n);
-                const int grid = static_cast<int>(std::min<long long>((n + 255) / 256, 65536));
-                hipLaunchKernelGGL(toFloatKernel, dim3(grid), dim3(256), 0, c.stream, pc.d_eb, pc.d_eb32, n);
-                hipLaunchKernelGGL(toFloatKernel, dim3(grid), dim3(256), 0, c.stream, pc.d_ek, pc.d_ek32, n);
-                LBX_HIP(hipGetLastError());
+                toFloat(c, pc.d_eb, pc.d_ek, pc.d_eb32, pc.d_ek32, static_cast<long long>(pc.eCount()));
             }
         }
 
@@ -598,13 +599,7 @@ namespace lbx
             {
                 if (pc.d_e1b32 || pc.n_ppairs == 0 || !pc.d_e1b)
                     continue;
-                const long long n = 3 * static_cast<long long>(pc.eCount());
-                pc.d_e1b32 = c.alloc<float>(n);
-                pc.d_e1k32 = c.alloc<float>(n);
-                const int grid = static_cast<int>(std::min<long long>((n + 255) / 256, 65536));
-                hipLaunchKernelGGL(toFloatKernel, dim3(grid), dim3(256), 0, c.stream, pc.d_e1b, pc.d_e1b32, n);
-                hipLaunchKernelGGL(toFloatKernel, dim3(grid), dim3(256), 0, c.stream, pc.d_e1k, pc.d_e1k32, n);
-                LBX_HIP(hipGetLastError());
+                toFloat(c, pc.d_e1b, pc.d_e1k, pc.d_e1b32, pc.d_e1k32, 3 * static_cast<long long>(pc.eCount()));
             }
         }
 
@@ -1377,14 +1372,7 @@ struct lbx_context : Context
                 for (void *p : {static_cast<void *>(t.d_prefix), static_cast<void *>(t.d_plo),
                                 static_cast<void *>(t.d_phi), static_cast<void *>(t.d_bprefix),
                                 static_cast<void *>(t.d_bq0)})
-                {
-                    auto it = std::find(allocations.begin(), allocations.end(), p);
-                    if (p && it != allocations.end())
-                    {
-                        (void)hipFree(p);
-                        allocations.erase(it);
-                    }
-                }
+                    giveBack(p);
             }
             if (best >= 0)
                 tuned_sum[{kind, il, iu}] = best;
@@ -1803,6 +1791,18 @@ extern "C"
         }
         ctx->stream = static_cast<hipStream_t>(stream);
         return LBX_OK;
+    }
+
+    int lbx_set_memory_limit(lbx_context *ctx, long bytes)
+    {
+        return guarded([&]
+                       {
+                           if (!ctx || bytes < 0)
+                               throw Error(LBX_ERR_INVALID, "lbx_set_memory_limit: null context or negative limit");
+                           std::lock_guard<std::mutex> lk(ctx->mu);
+                           std::lock_guard<std::mutex> la(ctx->alloc_mu);
+                           ctx->limit = static_cast<size_t>(bytes);
+                       });
     }
 
     int lbx_synchronize(lbx_context *ctx)

@@ -826,20 +826,26 @@ namespace lbx
     {
         if (pc.d_e1b || pc.n_pairs == 0)
             return;
-        pc.d_atom_a = c.upload(pc.atom_a);
-        pc.d_atom_b = c.upload(pc.atom_b);
+        // d_e1b last: a call that ran out of memory on the way goes on from what is there
+        if (!pc.d_atom_a)
+            pc.d_atom_a = c.upload(pc.atom_a);
+        if (!pc.d_atom_b)
+            pc.d_atom_b = c.upload(pc.atom_b);
         std::vector<PrimIn> prim(pc.n_ppairs);
         LBX_HIP(hipMemcpy(prim.data(), pc.d_prim, prim.size() * sizeof(PrimIn), hipMemcpyDeviceToHost));
         std::vector<double> ra(pc.n_ppairs);
         for (int o = 0; o < pc.n_ppairs; o++)
             ra[o] = prim[o].a / (prim[o].a + prim[o].b);
-        pc.d_ra = c.upload(ra);
+        if (!pc.d_ra)
+            pc.d_ra = c.upload(ra);
         const size_t ne = 3 * pc.eCount();
-        pc.d_e1b = c.alloc<double>(ne);
-        pc.d_e1k = c.alloc<double>(ne);
-        ecoefD1Fn(pc.la, pc.lb)(pc.n_ppairs, pc.d_prim, pc.d_centers, pc.d_norms, pc.d_e1b, pc.d_e1k,
+        if (!pc.d_e1k)
+            pc.d_e1k = c.alloc<double>(ne);
+        double *e1b = c.alloc<double>(ne);
+        ecoefD1Fn(pc.la, pc.lb)(pc.n_ppairs, pc.d_prim, pc.d_centers, pc.d_norms, e1b, pc.d_e1k,
                                 c.stream);
         LBX_HIP(hipGetLastError());
+        pc.d_e1b = e1b;
     }
 
     // Dense overlap, kinetic-energy and point-charge attraction matrices (any may be null),

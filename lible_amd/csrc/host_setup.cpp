@@ -322,8 +322,9 @@ namespace lbx
 
     void Context::release()
     {
-        for (void *p : allocations)
-            (void)hipFree(p);
+        for (auto &a : allocations)
+            (void)hipFree(a.first);
         allocations.clear();
+        held = 0;
     }
 }

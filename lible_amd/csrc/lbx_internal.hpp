@@ -7,6 +7,7 @@
 #include <algorithm>
 #include <array>
 #include <cstring>
+#include <map>
 #include <mutex>
 #include <stdexcept>
 #include <string>
@@ -116,7 +117,11 @@ namespace lbx
         // within a molecule.  Empty for an ordinary (one-molecule) context.
         std::vector<int> atom_mol;
         int nmol = 1;
-        std::vector<void *> allocations;
+        // device memory held until release(), with its sizes (alloc_mu: density fitting allocates
+        // without mu)
+        std::map<void *, size_t> allocations;
+        size_t held = 0, limit = 0;   // bytes; limit 0: none
+        std::mutex alloc_mu;
         // density fitting (ri.hip): the fitted 3-index tensor W (nbf^2 naux doubles, P-major),
         // built on the first lbx_ri_jk call and kept, and the exchange work buffer (same size,
         // made on the first call with K); both in allocations
@@ -126,14 +131,45 @@ namespace lbx
         bool ri_ready = false;
         std::mutex ri_mu;
 
+        // null when the device or the limit has no room
+        void *take(size_t bytes)
+        {
+            std::lock_guard<std::mutex> lk(alloc_mu);
+            if (limit > 0 && held + bytes > limit)
+                return nullptr;
+            void *p = nullptr;
+            const hipError_t e = hipMalloc(&p, bytes);
+            if (e == hipErrorOutOfMemory)
+            {
+                (void)hipGetLastError();   // not the next launch's error
+                return nullptr;
+            }
+            LBX_HIP(e);
+            allocations.emplace(p, bytes);
+            held += bytes;
+            return p;
+        }
+
+        void giveBack(void *p)
+        {
+            std::lock_guard<std::mutex> lk(alloc_mu);
+            auto it = allocations.find(p);
+            if (it == allocations.end())
+                return;
+            held -= it->second;
+            allocations.erase(it);
+            (void)hipFree(p);
+        }
+
+        // Whoever keeps the pointer for later calls stores it once everything that goes with it is
+        // there: a call may end here.
         template <class T>
         T *alloc(size_t n)
         {
-            void *p = nullptr;
-            if (n == 0)
-                n = 1;
-            LBX_HIP(hipMalloc(&p, n * sizeof(T)));
-            allocations.push_back(p);
+            const size_t bytes = std::max<size_t>(n, 1) * sizeof(T);
+            void *p = take(bytes);
+            if (!p)
+                throw Error(LBX_ERR_NOMEM, "device memory: no room for " + std::to_string(bytes) + " bytes");
             return static_cast<T *>(p);
         }
 

@@ -433,18 +433,8 @@ namespace lbx
         {
             // one buffer for the parts of K, then of J: up to 80 MiB at 1000 functions, 8 nbf^2 values
             // where tiles are many.  Without it K and J are made in one part.
-            void *p = nullptr;
             const long long parts = std::max(nt2 * splits * 4096, (naux + jGroup - 1) / jGroup * n2);
-            const hipError_t e = hipMalloc(&p, sizeof(double) * parts);
-            if (e == hipSuccess)
-            {
-                c.allocations.push_back(p);
-                c.ri_part = static_cast<double *>(p);
-            }
-            else if (e != hipErrorOutOfMemory)
-                LBX_HIP(e);
-            else
-                (void)hipGetLastError();
+            c.ri_part = static_cast<double *>(c.take(sizeof(double) * parts));
         }
         if (!c.ri_part)
         {

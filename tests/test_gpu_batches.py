@@ -206,6 +206,43 @@ def test_ri_jk_repeats(lbx, nmain, naux):
         assert torch.equal(Jo, ctx.ri_jk(D, exchange=False)[0])
 
 
+def until_it_fits(ctx, call, lbx):
+    """call() under a memory limit raised in steps of a tenth until it goes through -> its result and
+    the number of calls that ran out of memory."""
+    limit, refused = 1 << 10, 0
+    while True:
+        ctx.set_memory_limit(limit)
+        try:
+            return call(), refused, limit
+        except lbx.LbxError as e:
+            assert "lbx error -3" in str(e)
+            refused += 1
+            limit = limit * 11 // 10
+
+
+@pytest.mark.parametrize("what", ["jk", "grad", "one_electron_grad", "ri_jk", "sums"])
+def test_calls_after_running_out_of_memory(lbx, what):
+    """A call that ran out of memory leaves a context on which a later one gives the results of a fresh
+    context.  Tolerances: the order of atomic additions (1e-12), FP32 tiers the same kernels."""
+    import torch
+    mixed = dict(precision=lbx.LBX_MIXED, mixed_thresh=1e-2)
+    m = B.synthetic_molecule(78, 2, 3.0, B.RECIPE_MAIN, B.RECIPE_AUX)
+    D = torch.tensor(B.density_from_orbitals(3, m.shells.nbf, 6, 0.2), device="cuda")
+    charges = np.column_stack([m.coords, [6.0, 7.0]])
+    calls = {"jk": lambda c: c.jk(D, schwarz=0.0, **mixed)[:2], "grad": lambda c: c.jk_grad(D, schwarz=0.0, **mixed)[:1],
+             "one_electron_grad": lambda c: c.one_electron_grad(D, D, charges), "ri_jk": lambda c: c.ri_jk(D),
+             "sums": lambda c: c.ri_sums(**mixed)[:1]}
+    make = lambda: lbx.Context.batch([m, m]) if what == "sums" else lbx.Context(m)
+    ref = calls[what](make())
+    ctx = make()
+    got, refused, _ = until_it_fits(ctx, lambda: calls[what](ctx), lbx)
+    assert refused > 10
+    ctx.set_memory_limit(0)
+    for out in (got, calls[what](ctx)):
+        for a, b in zip(out, ref):
+            close(a.cpu().numpy(), b.cpu().numpy(), rel=0.0, floor=1e-12)
+
+
 @pytest.mark.parametrize("ns", [14, 15, 16, 19, 23])
 @pytest.mark.parametrize("variant", [0, 1, 3, 4])
 def test_jk_one_lane_pair_counts(lbx, oracle, ns, variant):
