@@ -57,7 +57,9 @@ int lbx_set_stream(lbx_context *ctx, void *stream);
 int lbx_synchronize(lbx_context *ctx);
 /* Upper bound on the device memory that the context holds between calls (bytes; 0: none, the
  * default).  A call that would go past it returns LBX_ERR_NOMEM, as when the device is full, and
- * the context stays usable: a later call with more room gives the same results. */
+ * the context stays usable: a later call with more room gives the same results.  What only saves
+ * time (copies of the E matrices for the one-lane kernels, parts of J: at most a quarter of the
+ * device's memory) is left out where there is no room, and freed before a call fails. */
 int lbx_set_memory_limit(lbx_context *ctx, long bytes);
 
 /* Boys function F_0..F_n at count points (device x[count] -> device out[count*(n+1)]).

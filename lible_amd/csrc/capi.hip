@@ -977,21 +977,65 @@ struct lbx_context : Context
     };
     std::map<std::pair<const LanePerm *, bool>, LaneE> lane_e;
 
-    // le / le32 / lbase of a J/K lane side; the interleaved copies are made on first use
-    void setLaneE(KArgs &a, const PairClass &pc, bool ket, const LanePerm &lp, bool f32)
+    // Device memory that only saves time: the interleaved copies of E and the parts of J.  At most a
+    // quarter of the device's; where there is no room for one, the call takes forms that need none,
+    // and a call that runs out of memory frees them all and is made again without (guardedIn).
+    std::vector<void *> extras;
+    size_t extra_bytes = 0, extra_cap = 0;
+    bool no_extras = false;   // after such a call
+    bool capturing = false;   // a capture allocates nothing: it takes what the eager call before it took
+
+    template <class T>
+    T *takeExtra(size_t n)
     {
-        LaneE &le = lane_e[{&lp, ket}];
-        interleave(le, pc, ket, pc.order, &lp.perm, pc.d_order, lp.d_perm, f32);
-        a.le = le.e;
-        a.le32 = le.e32;
-        a.lbase = le.base;
+        if (no_extras || capturing)
+            return nullptr;
+        if (extra_cap == 0)
+        {
+            size_t total = 0;
+            LBX_HIP(hipDeviceTotalMem(&total, device));
+            extra_cap = total / 4;
+        }
+        const size_t bytes = std::max<size_t>(n, 1) * sizeof(T);
+        void *p = extra_bytes + bytes <= extra_cap ? take(bytes) : nullptr;
+        if (p)
+        {
+            extras.push_back(p);
+            extra_bytes += bytes;
+        }
+        return static_cast<T *>(p);
     }
 
-    void interleave(LaneE &le, const PairClass &pc, bool ket, const std::vector<int> &order,
+    // Frees them (between calls) with the graphs and launches that were made with them.
+    bool freeExtras()
+    {
+        if (extras.empty())
+            return false;
+        LBX_HIP(hipStreamSynchronize(stream));
+        dropJKGraphs();
+        dropRiGraph();
+        ri_prepared.clear();
+        ri_launches.clear();
+        for (auto &kv : lane_e)
+            kv.second.e = nullptr, kv.second.e32 = nullptr;
+        for (auto &kv : sum_e)
+            kv.second.e = nullptr, kv.second.e32 = nullptr;
+        j_parts = nullptr;
+        for (void *p : extras)
+            giveBack(p);
+        extras.clear();
+        extra_bytes = 0;
+        return true;
+    }
+
+    // The interleaved E of a lane side, made on first use; false when there is no room for it.
+    bool interleave(LaneE &le, const PairClass &pc, bool ket, const std::vector<int> &order,
                     const std::vector<int> *perm, const int *d_order, const int *d_perm, bool f32)
     {
         if (f32 ? le.e32 != nullptr : le.e != nullptr)
-            return;
+            return true;
+        if (capturing)
+            return false;
         const int hs = nHerm(pc.la + pc.lb) * nSph(pc.la) * nSph(pc.lb), nblk = (pc.n_pairs + 63) / 64;
         std::vector<long long> base(nblk + 1, 0);
         for (int b = 0; b < nblk; b++)
@@ -1001,6 +1045,10 @@ struct lbx_context : Context
                 k = std::max(k, pc.pcnt[order[perm ? (*perm)[p] : p]]);
             base[b + 1] = base[b] + 64LL * k * hs;
         }
+        float *e32 = f32 ? takeExtra<float>(base[nblk]) : nullptr;
+        double *e = f32 ? nullptr : takeExtra<double>(base[nblk]);
+        if (!e && !e32)
+            return false;
         if (!le.base)
             le.base = upload(base);
         flushStaged();   // the orders
@@ -1013,16 +1061,15 @@ struct lbx_context : Context
         };
         if (f32)
         {
-            float *e = alloc<float>(base[nblk]);
-            run(e, ket ? pc.d_ek32 : pc.d_eb32);
-            le.e32 = e;
+            run(e32, ket ? pc.d_ek32 : pc.d_eb32);
+            le.e32 = e32;
         }
         else
         {
-            double *e = alloc<double>(base[nblk]);
             run(e, ket ? pc.d_ek : pc.d_eb);
             le.e = e;
         }
+        return true;
     }
 
     // Pair order of the RI sums without a bound range: by molecule, then the longest primitive
@@ -1051,8 +1098,16 @@ struct lbx_context : Context
         return so;
     }
 
-    // orders and (one-lane forms) the lane side's E of an RI sum launch
-    void setSumSides(KArgs &a, const PairClass &lane, const PairClass &unif, bool bounded, int kind, bool f32)
+    // whether the lane side's E of a one-lane RI sum launch is there
+    bool sumLaneReady(const PairClass &lane, bool bounded, bool f32)
+    {
+        const std::vector<int> &order = bounded ? lane.order : sumOrder(lane).order;
+        return interleave(sum_e[{&lane, bounded}], lane, false, order, nullptr, bounded ? lane.d_order : sumOrder(lane).d_order,
+                          nullptr, f32);
+    }
+
+    // orders and (one-lane forms, sumLaneReady) the lane side's E of an RI sum launch
+    void setSumSides(KArgs &a, const PairClass &lane, const PairClass &unif, bool bounded, int kind)
     {
         if (!bounded)
         {
@@ -1061,8 +1116,7 @@ struct lbx_context : Context
         }
         if (kind != KIND_LANE)
             return;
-        LaneE &le = sum_e[{&lane, bounded}];
-        interleave(le, lane, false, bounded ? lane.order : sumOrder(lane).order, nullptr, a.bra.order, nullptr, f32);
+        const LaneE &le = sum_e[{&lane, bounded}];
         a.le = le.e;
         a.le32 = le.e32;
         a.lbase = le.base;
@@ -1117,19 +1171,47 @@ struct lbx_context : Context
         return k_cols.emplace(idx, k).first->second;
     }
 
-    // The J/K kernel of class pair (i >= j) with the given variant, its arguments over the
-    // quartets with lo <= Q_ab Q_cd < hi (staged tables: flushStaged() before the launch) and its
-    // task table.
+    // The lane side of a one-lane J/K kernel
+    struct JKLane
+    {
+        const LanePerm *lp = nullptr;
+        const LaneE *le = nullptr;
+        bool kLds = false;   // K rows of the uniform pair in LDS
+    };
+
+    // false when there is no room for its interleaved E
+    bool jkLane(int i, int j, const KernelSlot &s, bool f32, JKLane &l)
+    {
+        const PairClass &lside = s.swap ? cls[j] : cls[i], &uside = s.swap ? cls[i] : cls[j];
+        // K rows of the uniform pair in LDS: up to 64 KiB, and at least three lane blocks to share
+        // them (a workgroup's four waves take four blocks of a group); else K by atomics alone, which
+        // bound the classes of low angular momentum (16 updates per (ps|ps) quartet at 23 G/s:
+        // (H2O)10 def2-TZVP (ps|ps) 2.3 ms, with the rows in LDS 1.1)
+        l.kLds = lside.n_pairs > 128 && (nSph(uside.la) + nSph(uside.lb)) * kColumns(lside) * 8 <= 65536;
+        l.lp = &lanePerm(s.swap ? j : i, l.kLds);
+        LaneE &le = lane_e[{l.lp, s.swap}];
+        l.le = &le;
+        return interleave(le, lside, s.swap, lside.order, &l.lp->perm, lside.d_order, l.lp->d_perm, f32);
+    }
+
+    // The J/K kernel of class pair (i >= j) with the given variant (the one-wave form in its place
+    // when a one-lane form's copy of E has no room), its arguments over the quartets with
+    // lo <= Q_ab Q_cd < hi (staged tables: flushStaged() before the launch) and its task table.
     struct JKLaunch
     {
         Launcher fn;
         KArgs a;
         const TaskTable *t;
+        int var;
     };
     JKLaunch prepareJK(int i, int j, int var, const double *D, double *J, double *K,
                        double thresh, double thresh_hi = kNoUpper)
     {
         const PairClass &bra = cls[i], &ket = cls[j];
+        JKLane lane;
+        if (slotFor(MODE_JK, bra, ket, var).kind == KIND_LANE &&
+            !jkLane(i, j, slotFor(MODE_JK, bra, ket, var), isF32Variant(var), lane))
+            var = isF32Variant(var) ? VAR_MFMA32 : VAR_MFMA;
         const KernelSlot &s = slotFor(MODE_JK, bra, ket, var);
         // the one-wave-per-quartet kernel walks consecutive tasks of one pair of the side whose
         // E matrices are larger, so those stay in cache across the tasks
@@ -1161,16 +1243,10 @@ struct lbx_context : Context
             while (gshift < 6 && groupBytes * (2 << gshift) <= double(1 << 20))
                 gshift++;
         }
-        // K rows of the uniform pair in LDS: up to 64 KiB, and at least three lane blocks to share
-        // them (a workgroup's four waves take four blocks of a group); else K by atomics alone, which
-        // bound the classes of low angular momentum (16 updates per (ps|ps) quartet at 23 G/s:
-        // (H2O)10 def2-TZVP (ps|ps) 2.3 ms, with the rows in LDS 1.1)
-        const PairClass &uside = s.swap ? bra : ket;
-        const bool kLds = blockMajor && nlane > 128 && (nSph(uside.la) + nSph(uside.lb)) * kColumns(lside) * 8 <= 65536;
-        if (kLds)
+        const LanePerm *lp = lane.lp;
+        if (blockMajor && lane.kLds)
             gshift = std::max(gshift, 2);
-        const LanePerm *lp = blockMajor && nlane > 0 ? &lanePerm(s.swap ? j : i, kLds) : nullptr;
-        if (blockMajor && it->second.nblk == 0 && nlane > 0)
+        if (blockMajor && it->second.nblk == 0)
             buildBlockMajor(*this, it->second, nlane, 1, gshift, lp->perm, lp->bqlo, lp->bqhi);
         const TaskTable &t = it->second;
         KArgs a = baseArgs(*this, bra, ket, t, i == j);
@@ -1189,8 +1265,10 @@ struct lbx_context : Context
             a.bprefix = t.d_bprefix;
             a.bq0 = t.d_bq0;
             a.ntasks = t.btasks;
-            setLaneE(a, lside, s.swap, *lp, isF32Variant(var));
-            if (kLds)
+            a.le = lane.le->e;
+            a.le32 = lane.le->e32;
+            a.lbase = lane.le->base;
+            if (lane.kLds)
             {
                 const KCols &k = kCols(s.swap ? j : i);
                 a.kcol_a = k.d_a;
@@ -1259,16 +1337,17 @@ struct lbx_context : Context
             a.ntasks = ts.ntasks;
             sampled = ts.quartets;
         }
-        return {s.fn, a, &t};
+        return {s.fn, a, &t, var};
     }
 
-    // Queues it on the context stream.
-    void launchJK(int i, int j, int var, const double *D, double *J, double *K, double thresh)
+    // Queues it on the context stream; returns the variant that runs.
+    int launchJK(int i, int j, int var, const double *D, double *J, double *K, double thresh)
     {
         const JKLaunch l = prepareJK(i, j, var, D, J, K, thresh);
         flushStaged();
         l.fn(l.a, stream);
         LBX_HIP(hipGetLastError());
+        return l.var;
     }
 
     // when > 0, launchJK runs only a sample of ~sample_quartets quartets (autotuner timing) and
@@ -1347,13 +1426,13 @@ struct lbx_context : Context
             for (int v : {static_cast<int>(VAR_VALU_BRA), static_cast<int>(VAR_MFMA)})
             {
                 const KernelSlot &k = kernelSlot(MODE_SUM, lane.la, lane.lb, unif.la, unif.lb, v);
-                if (!k.fn)
+                if (!k.fn || (k.kind == KIND_LANE && !sumLaneReady(lane, false, false)))
                     continue;
                 TaskTable t = buildTasksMol(*this, lane, unif, same, k.width, 0.0, kNoUpper, false);
                 KArgs a = baseArgs(*this, lane, unif, t, same);
                 a.kind = kind;
                 a.out = scratch.p;
-                setSumSides(a, lane, unif, false, k.kind, false);
+                setSumSides(a, lane, unif, false, k.kind);
                 flushStaged();
                 k.fn(a, stream);   // loads the code
                 LBX_HIP(hipEventRecord(e0, stream));
@@ -1394,6 +1473,7 @@ struct lbx_context : Context
         }
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
+        freeExtras();   // the forms that lost keep nothing
         dropRiGraph();
         ri_prepared.clear();
         ri_counts.clear();
@@ -1414,12 +1494,16 @@ struct lbx_context : Context
                 const KernelSlot &ks = slotFor(MODE_SUM, lane, unif, var);
                 const KernelSlot &k32 = kernelSlot(MODE_SUM, lane.la, lane.lb, unif.la, unif.lb, VAR_VALU_BRA32);
                 const bool tiers = split > 0.0 && k32.fn;
-                auto one = [&](const KernelSlot &k, double lo, double hi, bool fp32)
+                auto one = [&](const KernelSlot &form, double lo, double hi, bool fp32)
                 {
+                    // without room for the copy of E, the one-wave form (FP64)
+                    const bool room = form.kind != KIND_LANE || sumLaneReady(lane, split > 0.0, fp32);
+                    const KernelSlot &k = room ? form : slotFor(MODE_SUM, lane, unif, VAR_MFMA);
+                    fp32 = fp32 && room;
                     TaskTable t = buildTasksMol(*this, lane, unif, same, k.width, lo, hi);
                     KArgs a = baseArgs(*this, lane, unif, t, same);
                     a.kind = kind;
-                    setSumSides(a, lane, unif, split > 0.0, k.kind, fp32);
+                    setSumSides(a, lane, unif, split > 0.0, k.kind);
                     launches.push_back({k.fn, a, variantTime(MODE_SUM, lane, unif, k, fp32, t.quartets, double(t.ntasks))});
                     n[kind == 3 ? 0 : 1] += t.quartets;
                     n[2] += t.flops;
@@ -1553,6 +1637,7 @@ struct lbx_context : Context
         hipStream_t saved = stream;
         JKGraph g;
         g.stats = st;
+        capturing = true;
         try
         {
             stream = cs;
@@ -1571,11 +1656,13 @@ struct lbx_context : Context
                 throw;
             }
             LBX_HIP(hipStreamEndCapture(cs, &g.graph));
+            capturing = false;
             stream = saved;
             LBX_HIP(hipGraphInstantiate(&g.exec, g.graph, nullptr, nullptr, 0));
         }
         catch (...)
         {
+            capturing = false;
             stream = saved;
             if (g.graph)
                 (void)hipGraphDestroy(g.graph);
@@ -1626,6 +1713,24 @@ struct lbx_context : Context
 
 namespace
 {
+    // A call on a context: one that runs out of device memory frees what the context holds to save
+    // time only, and is made again without it.
+    template <class F>
+    int guardedIn(lbx_context *ctx, F &&f)
+    {
+        const int rc = guarded(f);
+        if (rc != LBX_ERR_NOMEM || !ctx)
+            return rc;
+        bool freed = false;
+        (void)guarded([&] {
+            std::lock_guard<std::mutex> lk(ctx->mu);
+            (void)hipGetLastError();   // not the next launch's error
+            freed = ctx->freeExtras();
+            ctx->no_extras = ctx->no_extras || freed;
+        });
+        return freed ? guarded(f) : rc;
+    }
+
     // Shells, pair classes, E matrices and per-pair molecule ids of a new context.
     void setupContext(lbx_context &ctx, const lbx_basis &main_basis, const lbx_basis *aux_basis)
     {
@@ -1800,8 +1905,18 @@ extern "C"
                            if (!ctx || bytes < 0)
                                throw Error(LBX_ERR_INVALID, "lbx_set_memory_limit: null context or negative limit");
                            std::lock_guard<std::mutex> lk(ctx->mu);
-                           std::lock_guard<std::mutex> la(ctx->alloc_mu);
-                           ctx->limit = static_cast<size_t>(bytes);
+                           bool over = false;
+                           {
+                               std::lock_guard<std::mutex> la(ctx->alloc_mu);
+                               ctx->limit = static_cast<size_t>(bytes);
+                               over = bytes > 0 && ctx->held > ctx->limit;
+                           }
+                           ctx->no_extras = false;
+                           if (over)
+                               ctx->freeExtras();
+                           // sums prepared without the copies would stay so
+                           ctx->dropRiGraph();
+                           ctx->ri_prepared.clear();
                        });
     }
 
@@ -1831,7 +1946,7 @@ extern "C"
 
     int lbx_eri4(lbx_context *ctx, double *out)
     {
-        return guarded([&]
+        return guardedIn(ctx, [&]
                        {
                            if (!ctx || !out)
                                throw Error(LBX_ERR_INVALID, "lbx_eri4: null argument");
@@ -1854,7 +1969,7 @@ extern "C"
 
     int lbx_eri4_diag(lbx_context *ctx, double *out)
     {
-        return guarded([&]
+        return guardedIn(ctx, [&]
                        {
                            if (!ctx || !out)
                                throw Error(LBX_ERR_INVALID, "lbx_eri4_diag: null argument");
@@ -1884,7 +1999,7 @@ extern "C"
 
     int lbx_eri3(lbx_context *ctx, double *out)
     {
-        return guarded([&]
+        return guardedIn(ctx, [&]
                        {
                            if (!ctx || !out)
                                throw Error(LBX_ERR_INVALID, "lbx_eri3: null argument");
@@ -1909,7 +2024,7 @@ extern "C"
 
     int lbx_eri2(lbx_context *ctx, double *out)
     {
-        return guarded([&]
+        return guardedIn(ctx, [&]
                        {
                            if (!ctx || !out)
                                throw Error(LBX_ERR_INVALID, "lbx_eri2: null argument");
@@ -1933,7 +2048,7 @@ extern "C"
 
     int lbx_eri2_diag(lbx_context *ctx, double *out)
     {
-        return guarded([&]
+        return guardedIn(ctx, [&]
                        {
                            if (!ctx || !out)
                                throw Error(LBX_ERR_INVALID, "lbx_eri2_diag: null argument");
@@ -2245,7 +2360,7 @@ extern "C"
         int blocksEntry(lbx_context *ctx, int kind, int op, long nq, const int *shells, double *out,
                         const char *who, bool no_alloc = false)
         {
-            return guarded([&]
+            return guardedIn(ctx, [&]
                            {
                                if (!ctx || nq < 0 || (nq > 0 && (!shells || !out)))
                                    throw Error(LBX_ERR_INVALID, std::string(who) + ": null argument or negative count");
@@ -2315,7 +2430,7 @@ extern "C"
 
     int lbx_eri4d1(lbx_context *ctx, double *out)
     {
-        return guarded([&]
+        return guardedIn(ctx, [&]
                        {
                            if (!ctx || !out)
                                throw Error(LBX_ERR_INVALID, "lbx_eri4d1: null argument");
@@ -2327,7 +2442,7 @@ extern "C"
 
     int lbx_eri3d1(lbx_context *ctx, double *out)
     {
-        return guarded([&]
+        return guardedIn(ctx, [&]
                        {
                            if (!ctx || !out)
                                throw Error(LBX_ERR_INVALID, "lbx_eri3d1: null argument");
@@ -2341,7 +2456,7 @@ extern "C"
 
     int lbx_eri2d1(lbx_context *ctx, double *out)
     {
-        return guarded([&]
+        return guardedIn(ctx, [&]
                        {
                            if (!ctx || !out)
                                throw Error(LBX_ERR_INVALID, "lbx_eri2d1: null argument");
@@ -2367,13 +2482,13 @@ extern "C"
         // energy of noise, ten times that of forms which add 64 quartets at once.  Small systems,
         // whose sums are short, and parts of more than 4 GiB go without.
         const int ncls = static_cast<int>(c.cls.size());
-        const int nparts = n < 400 ? 1 : static_cast<int>(std::clamp<long long>((4LL << 30) / (8 * n * n), 1, ncls));
+        int nparts = n < 400 ? 1 : static_cast<int>(std::clamp<long long>((4LL << 30) / (8 * n * n), 1, ncls));
+        if (nparts > 1 && !j_parts)
+            j_parts = takeExtra<double>((nparts - 1) * n * n);
+        if (!j_parts)
+            nparts = 1;
         if (nparts > 1)
-        {
-            if (!j_parts)
-                j_parts = c.alloc<double>((nparts - 1) * n * n);
             fill(j_parts, (nparts - 1) * n * n, 0.0, c.stream);
-        }
         lbx_jk_stats st{};
         std::vector<QueuedLaunch> queue;
         auto launch = [&](int i, int j, int tier, int var, double lo, double hi)
@@ -2382,6 +2497,7 @@ extern "C"
             const int part = (i + j) % nparts;
             const JKLaunch l = prepareJK(i, j, var, D, part ? j_parts + (part - 1) * n * n : J, K, lo, hi);
             const TaskTable &t = *l.t;
+            var = l.var;
             st.quartets += t.quartets;
             st.flops += t.flops;
             if (isF32Variant(var))
@@ -2444,7 +2560,7 @@ extern "C"
     int lbx_jk(lbx_context *ctx, const double *D, double *J, double *K, double schwarz_thresh,
                int precision, double mixed_thresh, lbx_jk_stats *stats)
     {
-        return guarded([&]
+        return guardedIn(ctx, [&]
                        {
                            if (!ctx || !D || !J || !K)
                                throw Error(LBX_ERR_INVALID, "lbx_jk: null argument");
@@ -2495,7 +2611,7 @@ extern "C"
     int lbx_ri_sums(lbx_context *ctx, double *out, int precision, double mixed_thresh,
                     lbx_ri_stats *stats)
     {
-        return guarded([&]
+        return guardedIn(ctx, [&]
                        {
                            if (!ctx || !out)
                                throw Error(LBX_ERR_INVALID, "lbx_ri_sums: null argument");
@@ -2603,7 +2719,7 @@ extern "C"
     int lbx_jk_grad(lbx_context *ctx, const double *D, double *grad, double schwarz_thresh,
                     int precision, double mixed_thresh, lbx_jk_stats *stats)
     {
-        return guarded([&]
+        return guardedIn(ctx, [&]
                        {
                            if (!ctx || !D || !grad)
                                throw Error(LBX_ERR_INVALID, "lbx_jk_grad: null argument");
@@ -2675,7 +2791,7 @@ extern "C"
 
     int lbx_tune(lbx_context *ctx, const double *D, double schwarz_thresh)
     {
-        return guarded([&]
+        return guardedIn(ctx, [&]
                        {
                            if (!ctx)
                                throw Error(LBX_ERR_INVALID, "lbx_tune: null argument");
@@ -2719,8 +2835,9 @@ extern "C"
                                            // first launch builds the task table and loads the code;
                                            // the timed one runs a sample of leading quartets
                                            ctx->sample_quartets = kTuneSample;
-                                           ctx->launchJK(static_cast<int>(i), static_cast<int>(j), v, D, J.p, K.p,
-                                                         schwarz_thresh);
+                                           if (ctx->launchJK(static_cast<int>(i), static_cast<int>(j), v, D, J.p, K.p,
+                                                             schwarz_thresh) != v)
+                                               continue;   // no room for its copy of E
                                            LBX_HIP(hipEventRecord(e0, c.stream));
                                            ctx->launchJK(static_cast<int>(i), static_cast<int>(j), v, D, J.p, K.p,
                                                          schwarz_thresh);
@@ -2756,8 +2873,10 @@ extern "C"
                                (void)hipEventDestroy(e1);
                                throw;
                            }
+                           ctx->sample_quartets = 0;
                            (void)hipEventDestroy(e0);
                            (void)hipEventDestroy(e1);
+                           ctx->freeExtras();   // the forms that lost keep nothing
                        });
     }
 
@@ -2810,7 +2929,7 @@ extern "C"
 
     int lbx_ri_jk(lbx_context *ctx, const double *D, double *J, double *K)
     {
-        return guarded([&]
+        return guardedIn(ctx, [&]
                        {
                            if (!ctx || !D || !J)
                                throw Error(LBX_ERR_INVALID, "lbx_ri_jk: null argument");
@@ -2831,7 +2950,7 @@ extern "C"
 
     int lbx_one_electron(lbx_context *ctx, double *S, double *T, int ncharges, const double *charges, double *V)
     {
-        return guarded([&]
+        return guardedIn(ctx, [&]
                        {
                            if (!ctx || (!S && !T && !V))
                                throw Error(LBX_ERR_INVALID, "lbx_one_electron: null context or no output");
@@ -2879,7 +2998,7 @@ extern "C"
     int lbx_one_electron_grad(lbx_context *ctx, const double *D, const double *W, int ncharges,
                               const double *charges, double *grad, double *charge_grad)
     {
-        return guarded([&]
+        return guardedIn(ctx, [&]
                        {
                            if (!ctx || !D || !grad)
                                throw Error(LBX_ERR_INVALID, "lbx_one_electron_grad: null argument");

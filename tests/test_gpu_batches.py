@@ -223,7 +223,8 @@ def until_it_fits(ctx, call, lbx):
 @pytest.mark.parametrize("what", ["jk", "grad", "one_electron_grad", "ri_jk", "sums"])
 def test_calls_after_running_out_of_memory(lbx, what):
     """A call that ran out of memory leaves a context on which a later one gives the results of a fresh
-    context.  Tolerances: the order of atomic additions (1e-12), FP32 tiers the same kernels."""
+    context.  Tolerances: the order of atomic additions (1e-12), FP32 tiers the same kernels (the mixed
+    sums under the limit run FP64 ones: test_sums_without_room_for_copies)."""
     import torch
     mixed = dict(precision=lbx.LBX_MIXED, mixed_thresh=1e-2)
     m = B.synthetic_molecule(78, 2, 3.0, B.RECIPE_MAIN, B.RECIPE_AUX)
@@ -238,9 +239,82 @@ def test_calls_after_running_out_of_memory(lbx, what):
     got, refused, _ = until_it_fits(ctx, lambda: calls[what](ctx), lbx)
     assert refused > 10
     ctx.set_memory_limit(0)
-    for out in (got, calls[what](ctx)):
+    for out in [calls[what](ctx)] + ([got] if what != "sums" else []):
         for a, b in zip(out, ref):
             close(a.cpu().numpy(), b.cpu().numpy(), rel=0.0, floor=1e-12)
+
+
+CLASS_PAIRS = [(la, lb, lc, ld) for la in range(4) for lb in range(la + 1) for lc in range(4) for ld in range(lc + 1)
+               if la * (la + 1) // 2 + lb >= lc * (lc + 1) // 2 + ld]
+
+
+@pytest.mark.parametrize("variant", [0, 3])
+@pytest.mark.parametrize("graphs", [False, True])
+def test_jk_without_room_for_copies(lbx, variant, graphs):
+    """A J/K build under the least memory limit that it goes through with: without the one-lane kernels'
+    copies of E and the parts of J (420 functions) it runs the one-wave forms with one J, at no more
+    memory than a context that is told to.  FP64: the order of the sums, 1e-12 of the largest element;
+    FP32 tier 1e-5 (the other parity tests')."""
+    import torch
+    m = B.synthetic_molecule(79, 14, 9.0, B.RECIPE_MAIN)
+    D = torch.tensor(B.density_from_orbitals(3, m.shells.nbf, 20, 0.1), device="cuda")
+    mixed = dict(precision=lbx.LBX_MIXED, mixed_thresh=1e30) if variant == 3 else {}
+    J, K = torch.empty_like(D), torch.empty_like(D)
+    run = lambda c: c.jk(D, schwarz=1e-10, J=J, K=K, **mixed)[:2]
+    wave = lbx.Context(m)
+    for c in CLASS_PAIRS:
+        assert wave.set_variant(c, 5 if variant == 3 else 2)
+    ref = [x.clone() for x in run(wave)]
+    wave = lbx.Context(m)
+    for c in CLASS_PAIRS:
+        wave.set_variant(c, 5 if variant == 3 else 2)
+    _, _, least = until_it_fits(wave, lambda: run(wave), lbx)
+    ctx = lbx.Context(m)
+    assert sum(ctx.set_variant(c, variant) for c in CLASS_PAIRS) > 30
+    ctx.set_graphs(graphs)
+    _, _, limit = until_it_fits(ctx, lambda: run(ctx), lbx)
+    assert limit <= least * 1.25 + (2 << 20)   # the lane orders
+    for unbounded in (False, False, False, True, True):
+        if unbounded:
+            ctx.set_memory_limit(0)
+            ctx.set_graphs(False)
+        for got, want in zip(run(ctx), ref):
+            close(got.cpu().numpy(), want.cpu().numpy(), rel=0.0, floor=1e-5 if variant == 3 else 1e-12)
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+def test_sums_without_room_for_copies(lbx, mixed):
+    """RI sums under the least memory limit against the unbounded ones: without the copies of E the
+    triplets that had an FP32 one-lane form run in FP64.  1e-12 (FP64), 1e-6 of the largest sum."""
+    mols = [B.synthetic_molecule(80 + k, 3, 4.5, B.RECIPE_MAIN, B.RECIPE_AUX) for k in range(3)]
+    kw = dict(precision=lbx.LBX_MIXED, mixed_thresh=1e-2) if mixed else {}
+    ref, sr = lbx.Context.batch(mols).ri_sums(**kw)
+    ctx = lbx.Context.batch(mols)
+    (got, st), refused, _ = until_it_fits(ctx, lambda: ctx.ri_sums(**kw), lbx)
+    assert refused > 0 and st["triplets"] == sr["triplets"]
+    assert st["triplets_fp32"] < sr["triplets_fp32"] or not mixed
+    close(got.cpu().numpy(), ref.cpu().numpy(), rel=0.0, floor=1e-6 if mixed else 1e-12)
+
+
+def test_copies_freed_before_a_call_fails(lbx):
+    """A call that cannot have its memory (the fitted tensor of 1000 functions and 60000 auxiliary ones,
+    480 GB) frees the parts of J (14 of 8 MB) before it fails, and J and K are the same without them."""
+    import torch
+    rng = np.random.default_rng(5)
+    nat = 1000
+    coords = np.stack([1.5 * np.arange(nat), rng.uniform(0, 1, nat), rng.uniform(0, 1, nat)], 1)
+    main = B.Shells.from_lists([[(0, [0.8], [1.0])] for _ in range(nat)])
+    aux = B.Shells.from_lists([[(0, [float(e)], [1.0]) for e in rng.uniform(0.5, 4.0, 60)] for _ in range(nat)])
+    ctx = lbx.Context(B.Molecule(coords, main, aux))
+    D = torch.tensor(B.density_from_orbitals(3, nat, 20, 0.1), device="cuda")
+    J, K, _ = ctx.jk(D)
+    free = torch.cuda.mem_get_info()[0]
+    with pytest.raises(lbx.LbxError, match="lbx error -3"):
+        ctx.ri_jk(D, exchange=False)
+    assert torch.cuda.mem_get_info()[0] - free >= 100 << 20
+    J2, K2, _ = ctx.jk(D)
+    close(J2.cpu().numpy(), J.cpu().numpy(), rel=0.0, floor=1e-12)
+    close(K2.cpu().numpy(), K.cpu().numpy(), rel=0.0, floor=1e-12)
 
 
 @pytest.mark.parametrize("ns", [14, 15, 16, 19, 23])
