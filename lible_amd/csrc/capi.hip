@@ -487,6 +487,14 @@ namespace lbx
             return s.kind == KIND_WAVE ? cost::waveForm(b, k, f32, quartets) : cost::blockForm(b, k, f32, quartets);
         }
 
+        // Whether the kernel of a variant is a form of its own: a one-lane number whose form is not built
+        // runs the one-wave form, which has a number already.
+        bool ownForm(int v, const KernelSlot &s)
+        {
+            const bool laneVariant = v != VAR_MFMA && v != VAR_MFMA32 && v != VAR_BLOCK && v != VAR_BLOCK32;
+            return s.fn && laneVariant == (s.kind == KIND_LANE);
+        }
+
         // The form with the smallest estimate among the FP64 (or FP32) ones, and that estimate; -1
         // when the class pair has none.  wavesBra, wavesKet: tasks of the one-lane forms with the
         // bra (ket) pairs on the lanes.
@@ -498,9 +506,8 @@ namespace lbx
             for (int v = 0; v < N_VARIANTS; v++)
             {
                 const KernelSlot &s = kernelSlot(mode, bra.la, bra.lb, ket.la, ket.lb, v);
-                const bool laneVariant = v != VAR_MFMA && v != VAR_MFMA32 && v != VAR_BLOCK && v != VAR_BLOCK32;
-                if (!s.fn || isF32Variant(v) != f32 || laneVariant != (s.kind == KIND_LANE))
-                    continue;   // (the one-wave form under a one-lane number is the same kernel)
+                if (!ownForm(v, s) || isF32Variant(v) != f32)
+                    continue;
                 const double t = variantTime(mode, bra, ket, s, f32, quartets, s.swap ? wavesKet : wavesBra);
                 if (best < 0 || t < tBest)
                 {
@@ -2828,7 +2835,7 @@ extern "C"
                                        double best_ms = 0, best32_ms = 0;
                                        for (int v = 0; v < N_VARIANTS; v++)
                                        {
-                                           if (!kernelSlot(MODE_JK, bra.la, bra.lb, ket.la, ket.lb, v).fn)
+                                           if (!ownForm(v, kernelSlot(MODE_JK, bra.la, bra.lb, ket.la, ket.lb, v)))
                                                continue;
                                            if (isF32Variant(v))
                                                ensureF32(c);

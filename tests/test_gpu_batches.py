@@ -206,6 +206,39 @@ def test_ri_jk_repeats(lbx, nmain, naux):
         assert torch.equal(Jo, ctx.ri_jk(D, exchange=False)[0])
 
 
+# class pairs whose one-lane number (0, 1; FP32 3, 4) runs the one-wave form: at most three column passes,
+# or seven of at least three columns, and 5500 FMAs are built as one-lane forms
+STAND_IN = {
+    0: "2111 2121 2211 2220 3021 3022 3030 3111 3120", 1: "2211 3021 3130 3211 3220 3310",
+    3: "2222 3022 3122 3131 3211 3221 3222 3230 3231 3311 3320",
+    4: "2220 3120 3122 3130 3210 3211 3220 3221 3222 3230 3231 3310 3311 3320 3321 3330"}
+STAND_IN = {v: [tuple(map(int, c)) for c in cs.split()] for v, cs in STAND_IN.items()}
+
+
+def profiled(ctx, lbx, D, fp32):
+    """The kernel of each class pair of one J/K build: the FP64 ones, or with every quartet in FP32."""
+    ctx.profile(True)
+    ctx.jk(D, schwarz=0.0, **(dict(precision=lbx.LBX_MIXED, mixed_thresh=1e30) if fp32 else {}))
+    out = {p["class"]: p["kernel"] for p in ctx.profile_read() if p["quartets"] > 0}
+    ctx.profile(False)
+    return out
+
+
+def test_tune_times_each_form_once(lbx):
+    """The tuner's choice is a form that the class pair has, never a one-lane number that stands for the
+    one-wave form."""
+    import torch
+    m = B.synthetic_molecule(81, 3, 4.5, B.RECIPE_MAIN)
+    D = torch.tensor(B.density_from_orbitals(3, m.shells.nbf, 6, 0.2), device="cuda")
+    for fp32, variants in ((False, (0, 1)), (True, (3, 4))):
+        ctx = lbx.Context(m)
+        ctx.tune(D)
+        kernels = profiled(ctx, lbx, D, fp32)
+        assert len(kernels) == 55
+        for v in variants:
+            assert not [c for c in STAND_IN[v] if kernels[c] == lbx.VARIANTS[v]]
+
+
 def until_it_fits(ctx, call, lbx):
     """call() under a memory limit raised in steps of a tenth until it goes through -> its result and
     the number of calls that ran out of memory."""
