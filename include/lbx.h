@@ -245,8 +245,8 @@ int lbx_set_variant(lbx_context *ctx, int la, int lb, int lc, int ld, int varian
  * lbx_profile_read returns the accumulated totals since the last enable. */
 typedef struct lbx_class_profile {
     int la, lb, lc, ld;
-    int kernel;            /* variant: 0 bra on lanes, 1 ket on lanes, 2 MFMA, 6 block;
-                              3 / 4 / 5 / 7 their FP32 forms */
+    int kernel;            /* the form that ran last: 0 bra on lanes, 1 ket on lanes, 2 MFMA,
+                              6 block; 3 / 4 / 5 / 7 their FP32 forms */
     int calls;
     double ms;             /* summed kernel time */
     double quartets;       /* summed quartets */

@@ -1202,7 +1202,7 @@ struct lbx_context : Context
     }
 
     // The J/K kernel of class pair (i >= j) with the given variant (the one-wave form in its place
-    // when a one-lane form's copy of E has no room), its arguments over the quartets with
+    // when the one-lane form is not built or its copy of E has no room), its arguments over the quartets with
     // lo <= Q_ab Q_cd < hi (staged tables: flushStaged() before the launch) and its task table.
     struct JKLaunch
     {
@@ -1215,9 +1215,10 @@ struct lbx_context : Context
                        double thresh, double thresh_hi = kNoUpper)
     {
         const PairClass &bra = cls[i], &ket = cls[j];
+        // the number of the form that runs, which the profile reports
         JKLane lane;
-        if (slotFor(MODE_JK, bra, ket, var).kind == KIND_LANE &&
-            !jkLane(i, j, slotFor(MODE_JK, bra, ket, var), isF32Variant(var), lane))
+        const KernelSlot &asked = slotFor(MODE_JK, bra, ket, var);
+        if (!ownForm(var, asked) || (asked.kind == KIND_LANE && !jkLane(i, j, asked, isF32Variant(var), lane)))
             var = isF32Variant(var) ? VAR_MFMA32 : VAR_MFMA;
         const KernelSlot &s = slotFor(MODE_JK, bra, ket, var);
         // the one-wave-per-quartet kernel walks consecutive tasks of one pair of the side whose

@@ -206,6 +206,9 @@ def test_ri_jk_repeats(lbx, nmain, naux):
         assert torch.equal(Jo, ctx.ri_jk(D, exchange=False)[0])
 
 
+CLASS_PAIRS = [(la, lb, lc, ld) for la in range(4) for lb in range(la + 1) for lc in range(4) for ld in range(lc + 1)
+               if la * (la + 1) // 2 + lb >= lc * (lc + 1) // 2 + ld]
+
 # class pairs whose one-lane number (0, 1; FP32 3, 4) runs the one-wave form: at most three column passes,
 # or seven of at least three columns, and 5500 FMAs are built as one-lane forms
 STAND_IN = {
@@ -222,6 +225,22 @@ def profiled(ctx, lbx, D, fp32):
     out = {p["class"]: p["kernel"] for p in ctx.profile_read() if p["quartets"] > 0}
     ctx.profile(False)
     return out
+
+
+@pytest.mark.parametrize("variant", range(8))
+def test_profile_names_the_form_that_ran(lbx, variant):
+    """With a variant fixed wherever it is accepted, the profile reports that form, or the one-wave form
+    where the number stands for it."""
+    import torch
+    m = B.synthetic_molecule(81, 3, 4.5, B.RECIPE_MAIN)
+    D = torch.tensor(B.density_from_orbitals(3, m.shells.nbf, 6, 0.2), device="cuda")
+    ctx = lbx.Context(m)
+    used = [c for c in CLASS_PAIRS if ctx.set_variant(c, variant)]
+    assert len(used) == {0: 31, 1: 30, 3: 48, 4: 42}.get(variant, 55)
+    kernels = profiled(ctx, lbx, D, variant in (3, 4, 5, 7))
+    for c in used:
+        wave = c in STAND_IN.get(variant, [])
+        assert kernels[c] == lbx.VARIANTS[(5 if variant > 2 else 2) if wave else variant], c
 
 
 def test_tune_times_each_form_once(lbx):
@@ -275,10 +294,6 @@ def test_calls_after_running_out_of_memory(lbx, what):
     for out in [calls[what](ctx)] + ([got] if what != "sums" else []):
         for a, b in zip(out, ref):
             close(a.cpu().numpy(), b.cpu().numpy(), rel=0.0, floor=1e-12)
-
-
-CLASS_PAIRS = [(la, lb, lc, ld) for la in range(4) for lb in range(la + 1) for lc in range(4) for ld in range(lc + 1)
-               if la * (la + 1) // 2 + lb >= lc * (lc + 1) // 2 + ld]
 
 
 @pytest.mark.parametrize("variant", [0, 3])
