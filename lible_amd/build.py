@@ -80,19 +80,29 @@ def _big_stack():
         resource.setrlimit(resource.RLIMIT_STACK, (hard, hard))
 
 
+def _command(src: str, obj: str, defines: list[str]) -> list[str]:
+    return [hipcc(), "-x", "hip", "-c", src, "-o", obj, "-MMD", "-MF", obj + ".d"] + FLAGS + defines
+
+
 def _compile(src: str, obj: str, defines: list[str]) -> tuple[str, float]:
     t = time.time()
-    cmd = [hipcc(), "-x", "hip", "-c", src, "-o", obj, "-MMD", "-MF", obj + ".d"] + FLAGS + defines
+    cmd = _command(src, obj, defines)
     r = subprocess.run(cmd, capture_output=True, text=True, preexec_fn=_big_stack)
     if r.returncode != 0:
         raise RuntimeError(f"compile failed: {' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
+    with open(obj + ".cmd", "w") as f:
+        f.write("\n".join(cmd))
     return obj, time.time() - t
 
 
-def _stale(src: str, obj: str) -> bool:
-    """True unless obj is newer than src and every project header its last compilation read."""
-    if not os.path.exists(obj) or not os.path.exists(obj + ".d"):
+def _stale(src: str, obj: str, defines: list[str]) -> bool:
+    """True unless obj was compiled by this command line (compiler, flags, unit and part numbers) and
+    is newer than src and every project header its last compilation read."""
+    if not all(os.path.exists(p) for p in (obj, obj + ".d", obj + ".cmd")):
         return True
+    with open(obj + ".cmd") as f:
+        if f.read() != "\n".join(_command(src, obj, defines)):
+            return True
     with open(obj + ".d") as f:
         words = f.read().replace("\\\n", " ").split()
     deps = [src] + [w for w in words if not w.endswith(":") and (w.startswith(ROOT) or w.startswith(CSRC))]
@@ -101,7 +111,7 @@ def _stale(src: str, obj: str) -> bool:
 
 def build(jobs: int | None = None, verbose: bool = True, incremental: bool = False) -> str:
     """Compiles every unit and links the library (incremental: only units older than their
-    sources or any header)."""
+    sources or any header, or compiled by another command line)."""
     os.makedirs(BUILD, exist_ok=True)
     jobs = jobs or max(1, min(os.cpu_count() or 4, 8))
     work = [
@@ -130,7 +140,7 @@ def build(jobs: int | None = None, verbose: bool = True, incremental: bool = Fal
     # heaviest units (highest bra class) first
     work.sort(key=lambda w: -(int(w[2][0].split("=")[1]) % 12) if w[2] else 1)
     t0 = time.time()
-    todo = [w for w in work if not incremental or _stale(w[0], w[1])]
+    todo = [w for w in work if not incremental or _stale(*w)]
     with cf.ThreadPoolExecutor(jobs) as ex:
         futs = [ex.submit(_compile, *w) for w in todo]
         for f in cf.as_completed(futs):
@@ -166,7 +176,8 @@ def main(argv=None):
     ap = argparse.ArgumentParser()
     ap.add_argument("-j", type=int, default=None)
     ap.add_argument("--incremental", action="store_true",
-                    help="recompile only units older than their sources or any header")
+                    help="recompile only units older than their sources or any header, or compiled "
+                         "by another command line")
     a = ap.parse_args(argv)
     build(a.j, incremental=a.incremental)
 
