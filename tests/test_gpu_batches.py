@@ -5,8 +5,6 @@ the 64 x 64 tiles of the density-fitting products, blocks in every order of thei
 Tolerances: FP64 sums of at most a few thousand terms in another order, 1e-12 relative with a floor
 of 1e-13 of the largest element (the other parity tests'); the gradient 1e-10 relative as in
 test_jk_grad."""
-import itertools
-
 import numpy as np
 import pytest
 
@@ -45,6 +43,34 @@ def uneven_molecule(seed, contractions):
     return B.Molecule(coords, B.Shells.from_lists(per_atom))
 
 
+CLASS_PAIRS = [(la, lb, lc, ld) for la in range(4) for lb in range(la + 1) for lc in range(4) for ld in range(lc + 1)
+               if la * (la + 1) // 2 + lb >= lc * (lc + 1) // 2 + ld]
+
+# class pairs whose one-lane number (0, 1; FP32 3, 4) runs the one-wave form: at most three column passes,
+# or seven of at least three columns, and 5500 FMAs are built as one-lane forms
+STAND_IN = {
+    0: "2111 2121 2211 2220 3021 3022 3030 3111 3120", 1: "2211 3021 3130 3211 3220 3310",
+    3: "2222 3022 3122 3131 3211 3221 3222 3230 3231 3311 3320",
+    4: "2220 3120 3122 3130 3210 3211 3220 3221 3222 3230 3231 3310 3311 3320 3321 3330"}
+STAND_IN = {v: [tuple(map(int, c)) for c in cs.split()] for v, cs in STAND_IN.items()}
+
+
+def profiled(ctx, lbx, D, fp32):
+    """The kernel of each class pair of one J/K build: the FP64 ones, or with every quartet in FP32."""
+    ctx.profile(True)
+    ctx.jk(D, schwarz=0.0, **(dict(precision=lbx.LBX_MIXED, mixed_thresh=1e30) if fp32 else {}))
+    out = {p["class"]: p["kernel"] for p in ctx.profile_read() if p["quartets"] > 0}
+    ctx.profile(False)
+    return out
+
+
+def fix_variant(ctx, lbx, variant):
+    """Fixes a variant wherever it is accepted; returns the class pairs that run it themselves."""
+    used = [c for c in CLASS_PAIRS if ctx.set_variant(c, variant)]
+    assert len(used) == {0: 31, 1: 30, 3: 48, 4: 42}.get(variant, 55)
+    return [c for c in used if c not in STAND_IN.get(variant, [])]
+
+
 # (l, K) lists: K_ab up to 121 (s, s), 81 (p, p) and 25 (f, d), beyond every batch (64 primitive
 # quartets at low L, 3 at (ff|ff)), next to single primitives
 UNEVEN = [[(0, 11), (0, 1), (1, 2)], [(1, 9), (0, 2), (2, 1)], [(2, 5), (1, 1), (3, 1), (0, 1)],
@@ -60,12 +86,29 @@ def test_jk_uneven_contractions(lbx, oracle, contractions, variant):
     Jr, Kr, _ = oracle.Structure(m).jk(D, thresh=0.0)
     ctx = lbx.Context(m)
     if variant is not None:
-        for la, lc in itertools.product(range(4), repeat=2):
-            for lb, ld in itertools.product(range(la + 1), range(lc + 1)):
-                ctx.set_variant((la, lb, lc, ld), variant)
+        assert fix_variant(ctx, lbx, variant) == CLASS_PAIRS
+        kernels = profiled(ctx, lbx, torch.tensor(D, device="cuda"), False)
+        assert kernels and set(kernels.values()) == {lbx.VARIANTS[variant]}
     J, K, _ = ctx.jk(torch.tensor(D, device="cuda"), schwarz=0.0)
     close(J.cpu().numpy(), Jr)
     close(K.cpu().numpy(), Kr)
+
+
+def test_jk_graph_replays_with_parts_of_J(lbx):
+    """Replays of a build whose J is made in parts (420 functions) after the density's contents changed,
+    against eager builds: the order of atomic additions, 1e-12 of the largest element."""
+    import torch
+    m = B.synthetic_molecule(79, 14, 9.0, B.RECIPE_MAIN)
+    ctx, eager = lbx.Context(m), lbx.Context(m)
+    ctx.set_graphs(True)
+    D = torch.empty((ctx.nbf, ctx.nbf), dtype=torch.float64, device="cuda")
+    J, K = torch.empty_like(D), torch.empty_like(D)
+    for seed in range(4):
+        D.copy_(torch.tensor(B.density_from_orbitals(seed, ctx.nbf, 20, 0.1)))
+        ctx.jk(D, schwarz=1e-10, J=J, K=K)
+        Je, Ke, _ = eager.jk(D, schwarz=1e-10)
+        close(J.cpu().numpy(), Je.cpu().numpy(), rel=0.0, floor=1e-12)
+        close(K.cpu().numpy(), Ke.cpu().numpy(), rel=0.0, floor=1e-12)
 
 
 @pytest.mark.parametrize("contractions", UNEVEN)
@@ -206,27 +249,6 @@ def test_ri_jk_repeats(lbx, nmain, naux):
         assert torch.equal(Jo, ctx.ri_jk(D, exchange=False)[0])
 
 
-CLASS_PAIRS = [(la, lb, lc, ld) for la in range(4) for lb in range(la + 1) for lc in range(4) for ld in range(lc + 1)
-               if la * (la + 1) // 2 + lb >= lc * (lc + 1) // 2 + ld]
-
-# class pairs whose one-lane number (0, 1; FP32 3, 4) runs the one-wave form: at most three column passes,
-# or seven of at least three columns, and 5500 FMAs are built as one-lane forms
-STAND_IN = {
-    0: "2111 2121 2211 2220 3021 3022 3030 3111 3120", 1: "2211 3021 3130 3211 3220 3310",
-    3: "2222 3022 3122 3131 3211 3221 3222 3230 3231 3311 3320",
-    4: "2220 3120 3122 3130 3210 3211 3220 3221 3222 3230 3231 3310 3311 3320 3321 3330"}
-STAND_IN = {v: [tuple(map(int, c)) for c in cs.split()] for v, cs in STAND_IN.items()}
-
-
-def profiled(ctx, lbx, D, fp32):
-    """The kernel of each class pair of one J/K build: the FP64 ones, or with every quartet in FP32."""
-    ctx.profile(True)
-    ctx.jk(D, schwarz=0.0, **(dict(precision=lbx.LBX_MIXED, mixed_thresh=1e30) if fp32 else {}))
-    out = {p["class"]: p["kernel"] for p in ctx.profile_read() if p["quartets"] > 0}
-    ctx.profile(False)
-    return out
-
-
 @pytest.mark.parametrize("variant", range(8))
 def test_profile_names_the_form_that_ran(lbx, variant):
     """With a variant fixed wherever it is accepted, the profile reports that form, or the one-wave form
@@ -235,12 +257,10 @@ def test_profile_names_the_form_that_ran(lbx, variant):
     m = B.synthetic_molecule(81, 3, 4.5, B.RECIPE_MAIN)
     D = torch.tensor(B.density_from_orbitals(3, m.shells.nbf, 6, 0.2), device="cuda")
     ctx = lbx.Context(m)
-    used = [c for c in CLASS_PAIRS if ctx.set_variant(c, variant)]
-    assert len(used) == {0: 31, 1: 30, 3: 48, 4: 42}.get(variant, 55)
+    own = fix_variant(ctx, lbx, variant)
     kernels = profiled(ctx, lbx, D, variant in (3, 4, 5, 7))
-    for c in used:
-        wave = c in STAND_IN.get(variant, [])
-        assert kernels[c] == lbx.VARIANTS[(5 if variant > 2 else 2) if wave else variant], c
+    assert all(kernels[c] == lbx.VARIANTS[variant] for c in own)
+    assert all(kernels[c] == lbx.VARIANTS[5 if variant > 2 else 2] for c in STAND_IN.get(variant, []))
 
 
 def test_tune_times_each_form_once(lbx):
@@ -310,15 +330,13 @@ def test_jk_without_room_for_copies(lbx, variant, graphs):
     J, K = torch.empty_like(D), torch.empty_like(D)
     run = lambda c: c.jk(D, schwarz=1e-10, J=J, K=K, **mixed)[:2]
     wave = lbx.Context(m)
-    for c in CLASS_PAIRS:
-        assert wave.set_variant(c, 5 if variant == 3 else 2)
+    fix_variant(wave, lbx, 5 if variant == 3 else 2)
     ref = [x.clone() for x in run(wave)]
     wave = lbx.Context(m)
-    for c in CLASS_PAIRS:
-        wave.set_variant(c, 5 if variant == 3 else 2)
+    fix_variant(wave, lbx, 5 if variant == 3 else 2)
     _, _, least = until_it_fits(wave, lambda: run(wave), lbx)
     ctx = lbx.Context(m)
-    assert sum(ctx.set_variant(c, variant) for c in CLASS_PAIRS) > 30
+    fix_variant(ctx, lbx, variant)
     ctx.set_graphs(graphs)
     _, _, limit = until_it_fits(ctx, lambda: run(ctx), lbx)
     assert limit <= least * 1.25 + (2 << 20)   # the lane orders
@@ -381,9 +399,11 @@ def test_jk_one_lane_pair_counts(lbx, oracle, ns, variant):
     D = B.density_from_orbitals(9, m.shells.nbf, 3, 0.3)
     Jr, Kr, _ = oracle.Structure(m).jk(D, thresh=1e-10)
     ctx = lbx.Context(m)
-    for la, lc in itertools.product(range(4), repeat=2):
-        for lb, ld in itertools.product(range(la + 1), range(lc + 1)):
-            ctx.set_variant((la, lb, lc, ld), variant)
+    own = fix_variant(ctx, lbx, variant)
+    kernels = profiled(ctx, lbx, torch.tensor(D, device="cuda"), variant >= 3)
+    # (ss) pairs on the lanes, more and fewer than 128 of them, against every uniform side
+    assert ((1, 0, 0, 0) if variant in (1, 4) else (0, 0, 0, 0)) in own
+    assert all(kernels[c] == lbx.VARIANTS[variant] for c in own)
     mixed = dict(precision=lbx.LBX_MIXED, mixed_thresh=1e9) if variant >= 3 else {}
     for _ in range(2):
         J, K, _ = ctx.jk(torch.tensor(D, device="cuda"), schwarz=1e-10, **mixed)

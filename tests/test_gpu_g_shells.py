@@ -187,6 +187,23 @@ def test_g_derivatives_blocks_and_limits(lbx, oracle):
         lbx.Context(mh)
 
 
+@pytest.mark.parametrize("ls", [(4, 0, 2, 0), (2, 0, 4, 0), (0, 4, 0, 3), (4, 0, 0, 4), (4, 0, 1, 1), (4, 0, 0), (0, 4, 3),
+                                (4, 0, 5), (4, 1, 2)])
+def test_g_block_routes(lbx, oracle, ls):
+    """Plain blocks with a main g shell, by the compiled one-wave kernel ((gs|ls), also of the ket first)
+    and by the run-time-L one, in the caller's shell order."""
+    m = B.synthetic_molecule(407, 2, 3.0, RECIPE_G1, RECIPE_AUX_H)
+    s = oracle.Structure(m)
+    ref = s.eri4() if len(ls) == 4 else s.eri3()
+    offs = [np.concatenate([[0], np.cumsum(2 * sh.l + 1)]) for sh in (m.shells, m.aux)]
+    rng = np.random.default_rng(9)
+    side = lambda k: 1 if len(ls) == 3 and k == 2 else 0
+    shells = np.stack([rng.choice(np.flatnonzero((m.shells, m.aux)[side(k)].l == l), 11) for k, l in enumerate(ls)], 1)
+    got = lbx.Context(m).blocks(shells.astype(np.int32)).cpu().numpy()[:, 0]
+    want = np.stack([ref[tuple(slice(offs[side(k)][x], offs[side(k)][x + 1]) for k, x in enumerate(q))] for q in shells])
+    close(got, want, floor=1e-13 * np.abs(ref).max() / np.abs(want).max())
+
+
 def _oracle_rhf(s, S, H, e_nuc, nocc):
     """Plain RHF with DIIS over the oracle's one-electron integrals and J/K."""
     sv, U = np.linalg.eigh(S)
