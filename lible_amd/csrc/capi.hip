@@ -2256,7 +2256,8 @@ extern "C"
             };
             // The integrals themselves: the compiled one-wave kernel of the class pair, whose bra is
             // the side with the higher class (or higher l of two auxiliary shells); the run-time-L
-            // kernel for derivatives and for main-basis g shells, which it does not cover.
+            // kernel for derivatives and for the class pairs with a main g shell that it does not cover
+            // (it covers (gs|ls): the instances of auxiliary g shells).
             const bool flip = kind == 2 ? bra->la < ket->la
                                         : kernelSlot(MODE_BLOCK, bra->la, bra->lb, ket->la, ket->lb, VAR_MFMA).fn == nullptr;
             const KernelSlot *wave = nullptr;

@@ -12,6 +12,19 @@
 namespace lbx
 {
     typedef double v4d __attribute__((ext_vector_type(4)));
+    typedef float v4f __attribute__((ext_vector_type(4)));
+
+    // 16x16x4 MFMA in FP64 or FP32.  Both take A[j][g] and B[g][j] from lane (g, j) = (lane / 16,
+    // lane % 16); accumulator element r of that lane holds D[4 r + g][j] for FP64 and
+    // D[4 g + r][j] for FP32.
+    __device__ __forceinline__ v4d mfma16(double a, double b, v4d c)
+    {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+    }
+    __device__ __forceinline__ v4f mfma16(float a, float b, v4f c)
+    {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
 
     constexpr double kTwoPi52 = 34.98683665524972;   // 2 pi^{5/2}
 
@@ -50,69 +63,6 @@ namespace lbx
             s = fma(s, m, row[2] * 0.5);
             s = fma(s, m, row[1]);
             s = fma(s, m, row[0]);
-            F[L] = s;
-            const double ex = exp(-x);
-            const double x2 = 2.0 * x;
-#pragma unroll
-            for (int k = L - 1; k >= 0; k--)
-                F[k] = fma(x2, F[k + 1], ex) * (1.0 / (2 * k + 1));
-        }
-    }
-
-    // The same evaluation split in two so that the table row can be fetched one iteration ahead
-    // of its use (the row load is a random gather whose latency otherwise stalls the wave):
-    // boysFetch loads the 7 tabulated values (any x: the row index is clamped to the table),
-    // boysEval finishes with exactly the operations of boysF.
-    struct BoysRow
-    {
-        double x;
-        double r[7];
-    };
-
-    template <int L>
-    __device__ __forceinline__ void boysFetch(double x, const double *__restrict__ tab, BoysRow &b)
-    {
-        b.x = x;
-        int iv = static_cast<int>(x * 100.0);
-        iv = iv < kBoysRows - 1 ? iv : kBoysRows - 1;
-        iv = iv > 0 ? iv : 0;
-        const double *row = tab + iv * kBoysCols + L;
-#pragma unroll
-        for (int j = 0; j < 7; j++)
-            b.r[j] = row[j];
-    }
-
-    template <int L>
-    __device__ __forceinline__ void boysEval(const BoysRow &b, double *F)
-    {
-        const double x = b.x;
-        if (x == 0.0)
-        {
-            F[0] = 1.0;
-#pragma unroll
-            for (int k = 1; k <= L; k++)
-                F[k] = 1.0 / (2 * k + 1);
-        }
-        else if (x > kBoysLargeX)
-        {
-            const double rx = 1.0 / x;
-            F[0] = 0.5 * sqrt(M_PI * rx);
-#pragma unroll
-            for (int k = 1; k <= L; k++)
-                F[k] = F[k - 1] * (k - 0.5) * rx;
-        }
-        else
-        {
-            const int iv = static_cast<int>(x * 100.0);
-            const double dx = x - iv * kBoysStep;
-            const double m = -dx;
-            double s = b.r[6] * (1.0 / 720.0);
-            s = fma(s, m, b.r[5] * (1.0 / 120.0));
-            s = fma(s, m, b.r[4] * (1.0 / 24.0));
-            s = fma(s, m, b.r[3] * (1.0 / 6.0));
-            s = fma(s, m, b.r[2] * 0.5);
-            s = fma(s, m, b.r[1]);
-            s = fma(s, m, b.r[0]);
             F[L] = s;
             const double ex = exp(-x);
             const double x2 = 2.0 * x;

@@ -20,13 +20,6 @@
 
 namespace lbx
 {
-    // 16x16x4 FP64 MFMA, A[j][g] and B[g][j] from lane (g, j) = (lane / 16, lane % 16); accumulator
-    // element r of that lane holds D[4 r + g][j].
-    __device__ __forceinline__ v4d gmfma(double a, double b, v4d c)
-    {
-        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-    }
-
     template <int LA, int LB, int LC, int LD, typename T>
     struct GWPlan
     {
@@ -194,7 +187,7 @@ namespace lbx
                                 {
                                     const bool in = 16 * tp + j < HP && ab0 + g4 < SP;
                                     const double a = in ? (eb + 16 * tp * SP + ab0)[ebOff] : T(0);
-                                    y[tp] = gmfma(a, wB[kk], y[tp]);
+                                    y[tp] = mfma16(a, wB[kk], y[tp]);
                                 }
                             }
                             waveFence();
@@ -241,7 +234,7 @@ namespace lbx
                                     const double b = in ? (ek + 4 * kt * SQ)[ekOff] : T(0);
 #pragma unroll
                                     for (int tp = 0; tp < TP1; tp++)
-                                        s[tp] = gmfma(R[sTab[tabS + 16 * tp * TW + 4 * kt]], b, s[tp]);
+                                        s[tp] = mfma16(double(R[sTab[tabS + 16 * tp * TW + 4 * kt]]), b, s[tp]);
                                 }
                                 // keep the phases apart: left alone the scheduler fetches all their operands
                                 // first, and the registers for that cost more than the latency
@@ -255,7 +248,7 @@ namespace lbx
                                 {
 #pragma unroll
                                     for (int tq = 0; tq < TQ; tq++)
-                                        qa[tq] = gmfma(R[sTab[tabQ + 4 * kt * TW + 16 * tq]], y[kt >> 2][kt & 3], qa[tq]);
+                                        qa[tq] = mfma16(double(R[sTab[tabQ + 4 * kt * TW + 16 * tq]]), y[kt >> 2][kt & 3], qa[tq]);
                                 }
                                 // V
 #pragma unroll
@@ -317,7 +310,7 @@ namespace lbx
                                         const int h = 4 * kt;
                                         const bool in = h + g4 < HP && ab < SP;
                                         const double a = in ? (e1b + (x * HP + h) * SP + 16 * ts)[e1bOff] : T(0);
-                                        gx = gmfma(a, s[kt >> 2][kt & 3], gx);
+                                        gx = mfma16(a, s[kt >> 2][kt & 3], gx);
                                     }
 #pragma unroll
                                     for (int r = 0; r < 4; r++)

@@ -97,15 +97,6 @@ namespace lbx
         int kcols;
     };
 
-    constexpr LBX_HD int rFlops(int L)
-    {
-        int r = 0;
-        for (int n = 0; n < L; n++)
-            for (int m = 1; m <= L - n; m++)
-                r += (m + 1) * (m + 2) / 2;
-        return 2 * r;
-    }
-
     template <int LA, int LB, int LC, int LD>
     struct Cls
     {

@@ -18,20 +18,6 @@
 
 namespace lbx
 {
-    typedef float v4f __attribute__((ext_vector_type(4)));
-
-    // 16x16x4 MFMA in FP64 or FP32.  Both take A[j][g] and B[g][j] from lane (g, j) = (lane / 16,
-    // lane % 16); accumulator element r of that lane holds D[4 r + g][j] for FP64 and
-    // D[4 g + r][j] for FP32.
-    __device__ __forceinline__ v4d mfma16(double a, double b, v4d c)
-    {
-        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-    }
-    __device__ __forceinline__ v4f mfma16(float a, float b, v4f c)
-    {
-        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-    }
-
     template <int N>
     using ic = std::integral_constant<int, N>;
 

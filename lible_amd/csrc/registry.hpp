@@ -46,6 +46,7 @@ namespace lbx
         int kind = KIND_LANE;
     };
 
-    // mode 0 J/K, 1 dense, 2 diagonal, 3 per-molecule sums; la, lc <= 5, lb, ld <= 3
+    // mode 0 J/K, 1 dense, 2 diagonal, 3 per-molecule sums, 4 listed blocks (Mode); la, lc <= 5,
+    // lb, ld <= 4
     KernelSlot &kernelSlot(int mode, int la, int lb, int lc, int ld, int variant);
 }
