@@ -74,19 +74,6 @@ namespace lbx
                 h[blockIdx.x] = s;
         }
 
-        // h_P = tr(T_P) where T_P = W_P D is there already
-        __global__ __launch_bounds__(256) void fitTraceKernel(const double *__restrict__ T, double *__restrict__ h,
-                                                              long long n)
-        {
-            const double *t = T + blockIdx.x * n * n;
-            double s = 0.0;
-            for (long long i = threadIdx.x; i < n; i += 256)
-                s += t[i * (n + 1)];
-            s = blockSum256(s);
-            if (threadIdx.x == 0)
-                h[blockIdx.x] = s;
-        }
-
         // out = sum over the P of group blockIdx.y of W_P h_P; each group has an n2-sized output of its own
         __global__ __launch_bounds__(256) void fitCoulombKernel(const double *__restrict__ W, const double *__restrict__ h,
                                                                 double *__restrict__ out, long long n2, int naux, int group)
@@ -102,43 +89,60 @@ namespace lbx
             out[blockIdx.y * n2 + i] = s;
         }
 
-        // out[i] = sum of the groups' outputs, in order
+        // out[i] = sum of the groups' outputs, in order (64 elements a workgroup, its waves a quarter of
+        // the groups each)
         __global__ __launch_bounds__(256) void sumGroupsKernel(const double *__restrict__ in, double *__restrict__ out,
                                                                long long n2, int groups)
         {
-            const long long i = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
-            if (i >= n2)
-                return;
+            __shared__ double quarter[4][64];
+            const int j = threadIdx.x & 63, w = threadIdx.x >> 6;
+            const long long i = min(blockIdx.x * 64LL + j, n2 - 1);
             double s = 0.0;
 #pragma unroll 8
-            for (int g = 0; g < groups; g++)
+            for (int g = groups * w / 4; g < groups * (w + 1) / 4; g++)
                 s += in[g * n2 + i];
-            out[i] = s;
+            quarter[w][j] = s;
+            __syncthreads();
+            if (w == 0)
+                out[i] = (quarter[0][j] + quarter[1][j]) + (quarter[2][j] + quarter[3][j]);
         }
 
-        // Whether D is symmetric to rounding, per block: flags[blockIdx.x] = 1 where it is not.  K is then
-        // not symmetric either, and its upper triangle is made too.
-        __global__ __launch_bounds__(256) void asymmetryKernel(const double *__restrict__ D, int n, int *flags)
+        // Two things that a K needs, in one launch.  Workgroups below naux: h_P = tr(T_P) where
+        // T_P = W_P D is there already.  The kFlagBlocks others: whether D is symmetric to rounding,
+        // flags[b] = 1 where it is not; K is then not symmetric either, and its upper triangle is made too.
+        constexpr int kFlagBlocks = 256;
+        __global__ __launch_bounds__(256) void traceSymmetryKernel(const double *__restrict__ T, const double *__restrict__ D,
+                                                                   double *__restrict__ h, int *flags, int n, int naux)
         {
             const long long tot = static_cast<long long>(n) * n;
+            if (static_cast<int>(blockIdx.x) < naux)
+            {
+                const double *t = T + blockIdx.x * tot;
+                double s = 0.0;
+                for (int i = threadIdx.x; i < n; i += 256)
+                    s += t[i * (n + 1LL)];
+                s = blockSum256(s);
+                if (threadIdx.x == 0)
+                    h[blockIdx.x] = s;
+                return;
+            }
+            const int b = static_cast<int>(blockIdx.x) - naux;
             bool differ = false;
-            for (long long e = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x; e < tot;
-                 e += static_cast<long long>(gridDim.x) * 256)
+            for (long long e = b * 256LL + threadIdx.x; e < tot; e += kFlagBlocks * 256LL)
             {
                 const int i = static_cast<int>(e / n), j = static_cast<int>(e % n);
                 if (j < i)
                 {
-                    const double a = D[e], b = D[static_cast<long long>(j) * n + i];
-                    differ |= fabs(a - b) > 1e-14 * fmax(fabs(a), fabs(b));
+                    const double x = D[e], y = D[static_cast<long long>(j) * n + i];
+                    differ |= fabs(x - y) > 1e-14 * fmax(fabs(x), fabs(y));
                 }
             }
             const int any = __syncthreads_or(differ);
             if (threadIdx.x == 0)
-                flags[blockIdx.x] = any;
+                flags[b] = any;
         }
 
-        // the flags of asymmetryKernel's kFlagBlocks workgroups (all 256 threads call)
-        constexpr int kFlagBlocks = 256;
+        // the flags of traceSymmetryKernel (all 256 threads call)
         __device__ __forceinline__ bool asymmetric(const int *flags) { return __syncthreads_or(flags[threadIdx.x]); }
 
         // tile number -> tile: the tiles with row >= column first, then the others
@@ -444,7 +448,6 @@ namespace lbx
         auto blocks1d = [](long long m) { return dim3(static_cast<int>(std::min<long long>((m + 255) / 256, 65536))); };
         if (K)
         {
-            hipLaunchKernelGGL(asymmetryKernel, dim3(kFlagBlocks), dim3(256), 0, stream, D, ni, c.ri_flags);
             // T_P = D^T W_P as panelGemm reads its operands; blockIdx.y holds at most 65535 auxiliary
             // functions
             const int nt = (ni + 63) / 64;
@@ -454,7 +457,9 @@ namespace lbx
                 hipLaunchKernelGGL((panelGemm<false>), dim3(nt * nt, np), dim3(256), 0, stream, D, c.ri_w + p0 * n2,
                                    c.ri_t + p0 * n2, ni, n, n, 1, nullptr);
             }
-            // K = sum_P T_P W_P^T
+            hipLaunchKernelGGL(traceSymmetryKernel, dim3(static_cast<int>(naux) + kFlagBlocks), dim3(256), 0, stream,
+                               c.ri_t, D, c.ri_h, c.ri_flags, ni, static_cast<int>(naux));
+            // K = sum_P T_P^T W_P
             const long long kTotal = n * naux;
             const long long chunk = ((kTotal + splits - 1) / splits + 15) / 16 * 16;
             hipLaunchKernelGGL((panelGemm<true>), dim3(static_cast<unsigned>(splits * nt * nt)), dim3(256), 0, stream,
@@ -465,17 +470,15 @@ namespace lbx
                                    static_cast<int>(splits), c.ri_flags);
             else
                 hipLaunchKernelGGL(mirrorKernel, blocks1d(n2), dim3(256), 0, stream, K, ni, c.ri_flags);
-            hipLaunchKernelGGL(fitTraceKernel, dim3(static_cast<int>(naux)), dim3(256), 0, stream, c.ri_t, c.ri_h, n);
         }
         else
             hipLaunchKernelGGL(fitDotKernel, dim3(static_cast<int>(naux)), dim3(256), 0, stream, c.ri_w, D, c.ri_h, n2);
-        {
-            const int bx = static_cast<int>((n2 + 255) / 256), groups = static_cast<int>((naux + jGroup - 1) / jGroup);
-            hipLaunchKernelGGL(fitCoulombKernel, dim3(bx, groups), dim3(256), 0, stream, c.ri_w, c.ri_h,
-                               groups > 1 ? c.ri_part : J, n2, static_cast<int>(naux), static_cast<int>(jGroup));
-            if (groups > 1)
-                hipLaunchKernelGGL(sumGroupsKernel, dim3(bx), dim3(256), 0, stream, c.ri_part, J, n2, groups);
-        }
+        const int bx = static_cast<int>((n2 + 255) / 256), groups = static_cast<int>((naux + jGroup - 1) / jGroup);
+        hipLaunchKernelGGL(fitCoulombKernel, dim3(bx, groups), dim3(256), 0, stream, c.ri_w, c.ri_h,
+                           groups > 1 ? c.ri_part : J, n2, static_cast<int>(naux), static_cast<int>(jGroup));
+        if (groups > 1)
+            hipLaunchKernelGGL(sumGroupsKernel, dim3(static_cast<int>((n2 + 63) / 64)), dim3(256), 0, stream, c.ri_part, J,
+                               n2, groups);
         LBX_HIP(hipGetLastError());
         LBX_HIP(hipStreamSynchronize(stream));
     }
