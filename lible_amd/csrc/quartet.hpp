@@ -130,9 +130,10 @@ namespace lbx
         static constexpr int NC1f = ncFor32(SQ, HQ, SP);
         // Whether the one-lane form is built: at most three column passes (each its own instance) or
         // up to seven of at least three columns, and at most 5500 FMAs in the unrolled transforms.
-        // Past that its waves run 2-28 times slower than the one-wave form (spilled registers,
+        // Past that most run 2-28 times slower than the one-wave form (spilled registers,
         // code beyond the instruction cache: (ff|ps) FP32 28x, (fd|ps) FP32 27x, (dp|dp) FP64 1.2 ms
-        // for one wave), which then serves the class pair under this variant too.
+        // for one wave), which then serves the class pair under this variant too.  Not all: (fp|ds) at 40
+        // atoms took 95 ms with the bra on the lanes and takes 102 in the one-wave form.
         static constexpr bool laneBuilt(int nc, int sl, int hl, int su, int hu)
         {
             if (nc < 1)

@@ -7,8 +7,10 @@
 // once), and a constant for the launch.  The coefficients (milliseconds per 10^6 of a count, on
 // the MI355X) are a non-negative fit of the logarithm of 2900 timed launches: every form of every class
 // pair to (ff|ff) on water clusters of 1 to 10 molecules in def2-SVP, -TZVP and -QZVP and on 2 to
-// 19 atoms of the synthetic s to f shells, 0.03 to 200 ms each, typically within 45%.  J/K time
-// summed over the class pairs, ms, by this rule / by the fastest form of each:
+// 19 atoms of the synthetic s to f shells, 0.03 to 200 ms each; the typical residual is a factor of
+// 1.45, and single class pairs are further off: (pp|pp) of (H2O)10 def2-TZVP stays on the one-wave form
+// at 3.8 ms where the one-lane form takes 1.0, RI sums of two molecules take 3.5 ms (tuned 1.2).  J/K
+// time summed over the class pairs, ms, by this rule / by the fastest form of each:
 //   H2O SVP 0.77 / 0.74, (H2O)8 SVP 5.5 / 4.9, (H2O)10 TZVP 40 / 35, 7 atoms s-f 9.8 / 8.3,
 //   19 atoms s-f 155 / 154;
 //   FP32 forms: 0.67 / 0.64, 5.2 / 4.9, 30 / 28, 8.6 / 7.4, 89 / 88
